@@ -58,7 +58,7 @@ int fail(int status, const char* fmt, ...)
     if (_e != hipSuccess) return fail(NSM_ERR_HIP, "kernel launch: %s", hipGetErrorString(_e));    \
   } while (0)
 
-constexpr int kElemChunk = 32;   // elements per FP64 element workgroup
+constexpr int kElemChunk = nsm::kFp64ChunkElems;  // elements per FP64 element chunk
 constexpr int kNodeChunk = 256;  // nodes per node workgroup (the model's node tiles)
 constexpr int kMaxBlocksPerMesh = 8;
 

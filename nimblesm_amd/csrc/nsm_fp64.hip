@@ -4,7 +4,7 @@
 //
 // Compiled with -ffp-contract=off: every FP64 expression keeps NimbleSM's
 // evaluation order so results match the reference's FP64 run bit for bit.
-// Work mapping: one 64-wide wavefront holds 8 elements, lane
+// Work mapping: one 64-wide wavefront (a workgroup) holds 8 elements, lane
 // k of an element serves as node k (gather, force output) and as Gauss point
 // k (F, stress); LDS carries the per-element node data and per-point
 // inverse Jacobians between the two roles.
@@ -20,21 +20,22 @@ namespace {
 // order of src/nimble_element.cc:55-171 (Gauss constant written as in :58).
 // ---------------------------------------------------------------------------
 struct HexTables {
-  double N[64];    // [ipt][node]
-  double dN[192];  // [ipt][node][dir]
+  double N[64];       // [ipt][node]
+  double dN[8][12];   // magnitudes of the shape derivatives, see ShapeRow
 };
+
+constexpr double kNodeSign[8][3] = {{-1, -1, -1}, {1, -1, -1}, {1, 1, -1}, {-1, 1, -1},
+                                    {-1, -1, 1},  {1, -1, 1},  {1, 1, 1},  {-1, 1, 1}};
 
 constexpr HexTables make_hex_tables()
 {
   HexTables    t{};
-  const double val     = 0.577350269189626;
-  const int    sg[8][3] = {{-1, -1, -1}, {1, -1, -1}, {1, 1, -1}, {-1, 1, -1},
-                           {-1, -1, 1},  {1, -1, 1},  {1, 1, 1},  {-1, 1, 1}};
-  const double c       = 1.0 / 8.0;
+  const double val = 0.577350269189626;
+  const double c   = 1.0 / 8.0;
   for (int q = 0; q < 8; q++) {
-    const double r = sg[q][0] > 0 ? val : -val;
-    const double s = sg[q][1] > 0 ? val : -val;
-    const double u = sg[q][2] > 0 ? val : -val;
+    const double r = kNodeSign[q][0] > 0 ? val : -val;
+    const double s = kNodeSign[q][1] > 0 ? val : -val;
+    const double u = kNodeSign[q][2] > 0 ? val : -val;
     t.N[8 * q + 0] = c * (1.0 - r) * (1.0 - s) * (1.0 - u);
     t.N[8 * q + 1] = c * (1.0 + r) * (1.0 - s) * (1.0 - u);
     t.N[8 * q + 2] = c * (1.0 + r) * (1.0 + s) * (1.0 - u);
@@ -43,38 +44,64 @@ constexpr HexTables make_hex_tables()
     t.N[8 * q + 5] = c * (1.0 + r) * (1.0 - s) * (1.0 + u);
     t.N[8 * q + 6] = c * (1.0 + r) * (1.0 + s) * (1.0 + u);
     t.N[8 * q + 7] = c * (1.0 - r) * (1.0 + s) * (1.0 + u);
-    double* d = &t.dN[24 * q];
-    d[0]  = -c * (1.0 - s) * (1.0 - u);
-    d[1]  = -c * (1.0 - r) * (1.0 - u);
-    d[2]  = -c * (1.0 - r) * (1.0 - s);
-    d[3]  = c * (1.0 - s) * (1.0 - u);
-    d[4]  = -c * (1.0 + r) * (1.0 - u);
-    d[5]  = -c * (1.0 + r) * (1.0 - s);
-    d[6]  = c * (1.0 + s) * (1.0 - u);
-    d[7]  = c * (1.0 + r) * (1.0 - u);
-    d[8]  = -c * (1.0 + r) * (1.0 + s);
-    d[9]  = -c * (1.0 + s) * (1.0 - u);
-    d[10] = c * (1.0 - r) * (1.0 - u);
-    d[11] = -c * (1.0 - r) * (1.0 + s);
-    d[12] = -c * (1.0 - s) * (1.0 + u);
-    d[13] = -c * (1.0 - r) * (1.0 + u);
-    d[14] = c * (1.0 - r) * (1.0 - s);
-    d[15] = c * (1.0 - s) * (1.0 + u);
-    d[16] = -c * (1.0 + r) * (1.0 + u);
-    d[17] = c * (1.0 + r) * (1.0 - s);
-    d[18] = c * (1.0 + s) * (1.0 + u);
-    d[19] = c * (1.0 + r) * (1.0 + u);
-    d[20] = c * (1.0 + r) * (1.0 + s);
-    d[21] = -c * (1.0 + s) * (1.0 + u);
-    d[22] = c * (1.0 - r) * (1.0 + u);
-    d[23] = c * (1.0 - r) * (1.0 + s);
+    for (int b = 0; b < 4; b++) {
+      t.dN[q][b]     = c * (b & 1 ? 1.0 + s : 1.0 - s) * (b & 2 ? 1.0 + u : 1.0 - u);
+      t.dN[q][4 + b] = c * (b & 1 ? 1.0 + r : 1.0 - r) * (b & 2 ? 1.0 + u : 1.0 - u);
+      t.dN[q][8 + b] = c * (b & 1 ? 1.0 + r : 1.0 - r) * (b & 2 ? 1.0 + s : 1.0 - s);
+    }
   }
   return t;
 }
 
 __constant__ HexTables c_hex = make_hex_tables();
 
-constexpr int kEPW     = 32;        // elements per 256-thread workgroup
+// Shape derivatives between point q and node j (signs s_q, s_j):
+//   dN_j/dxi_d (q) = s_j[d] m, m the product of 1/8 and, over the two other
+//   directions e in ascending order, 1 + s_j[e] s_q[e] val.
+// m depends on the signs only through their products, so one row of 12
+// magnitudes per point, 4 per direction d by the other side's signs in the
+// directions e, serves a lane in both its roles: as point q it takes the
+// entry of node j's signs and j's sign (a constant once the loop over j is
+// unrolled), as node n the entry of point q's signs and its own sign.  The
+// reference's 24 derivatives per point hold the same 12 numbers and their
+// negatives; -(1/8) (..) (..) is the negated product exactly, so products
+// with them differ in sign only.  Half the table loads and registers: with
+// the eigenvector selects of nsm_fp64_math.h and workgroups of one wavefront
+// (kEPW) the element launch went from 1.356 to 1.228 ms (128^3 model), 768 to
+// 707 us (128 x 24^3 ensemble, 78 registers where 96 spilled) and 10.5 to
+// 9.1 us (16^3 model).  What bounds it is VALU issue (90% of the SIMD cycles).
+struct ShapeRow {
+  double m[12];
+};
+__device__ __forceinline__ ShapeRow shape_row(int q)
+{
+  ShapeRow r;
+#pragma unroll
+  for (int i = 0; i < 12; i++) r.m[i] = c_hex.dN[q][i];
+  return r;
+}
+// magnitude in direction d towards the point or node with sign index j
+__device__ __forceinline__ constexpr int shape_entry(int d, int j)
+{
+  const int e0 = d == 0 ? 1 : 0, e1 = d == 2 ? 1 : 2;
+  return 4 * d + (kNodeSign[j][e0] > 0 ? 1 : 0) + (kNodeSign[j][e1] > 0 ? 2 : 0);
+}
+// derivatives of node j at the row's point
+__device__ __forceinline__ void node_derivatives(const ShapeRow& row, int j, double s[3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const double m = row.m[shape_entry(d, j)];
+    s[d]           = kNodeSign[j][d] > 0 ? m : -m;
+  }
+}
+
+// One wavefront per workgroup: the barriers between the node and point roles
+// then cost nothing and no wave waits for another's divisions.  At five waves
+// per SIMD either way, element launch with 8 / 16 / 32 elements per workgroup:
+// 128^3 model 1.228 / 1.247 / 1.240 ms, 128 x 24^3 ensemble 0.707 / 0.718 /
+// 0.719 ms, 16^3 model 9.1 / 9.1 / 10.4 us.
+constexpr int kEPW     = kFp64Elems;  // elements per workgroup
 constexpr int kThreads = 8 * kEPW;  // 8 lanes per element
 
 using namespace fp64;
@@ -83,13 +110,15 @@ using namespace fp64;
 // dN_j/dxi (src/nimble_element.h:442-482, which forms both in one loop; each
 // entry is its own chain of products and sums, so forming them apart gives
 // the same bits).  xs/us are [8][3]: b alone, then both.
-__device__ __forceinline__ void reference_jacobian(int q, const double (*xs)[3], double b[9])
+__device__ __forceinline__ void reference_jacobian(const ShapeRow& row, const double (*xs)[3], double b[9])
 {
   for (int i = 0; i < 9; i++) b[i] = 0.0;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const double rc1 = xs[j][0], rc2 = xs[j][1], rc3 = xs[j][2];
-    const double s1 = c_hex.dN[24 * q + 3 * j], s2 = c_hex.dN[24 * q + 3 * j + 1], s3 = c_hex.dN[24 * q + 3 * j + 2];
+    double       s[3];
+    node_derivatives(row, j, s);
+    const double s1 = s[0], s2 = s[1], s3 = s[2];
     b[0] += rc1 * s1;
     b[1] += rc1 * s2;
     b[2] += rc1 * s3;
@@ -103,8 +132,8 @@ __device__ __forceinline__ void reference_jacobian(int q, const double (*xs)[3],
 }
 
 // both in one pass over the nodes
-__device__ __forceinline__ void jacobians(int q, const double (*xs)[3], const double (*us)[3], double a[9],
-                                          double b[9])
+__device__ __forceinline__ void jacobians(const ShapeRow& row, const double (*xs)[3], const double (*us)[3],
+                                          double a[9], double b[9])
 {
   for (int i = 0; i < 9; i++) a[i] = b[i] = 0.0;
 #pragma unroll
@@ -113,7 +142,9 @@ __device__ __forceinline__ void jacobians(int q, const double (*xs)[3], const do
     const double cc1 = rc1 + us[j][0];
     const double cc2 = rc2 + us[j][1];
     const double cc3 = rc3 + us[j][2];
-    const double s1 = c_hex.dN[24 * q + 3 * j], s2 = c_hex.dN[24 * q + 3 * j + 1], s3 = c_hex.dN[24 * q + 3 * j + 2];
+    double       s[3];
+    node_derivatives(row, j, s);
+    const double s1 = s[0], s2 = s[1], s3 = s[2];
     a[0] += cc1 * s1;
     a[1] += cc1 * s2;
     a[2] += cc1 * s3;
@@ -138,13 +169,15 @@ __device__ __forceinline__ void jacobians(int q, const double (*xs)[3], const do
 // The same two Jacobians from the current coordinates x = X + u formed once
 // per node (xc), as the element kernels stage them: each node's sum is the
 // one the functions above form in every lane, so the bits are the same.
-__device__ __forceinline__ void current_jacobian_x(int q, const double (*xc)[3], double a[9])
+__device__ __forceinline__ void current_jacobian_x(const ShapeRow& row, const double (*xc)[3], double a[9])
 {
   for (int i = 0; i < 9; i++) a[i] = 0.0;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const double cc1 = xc[j][0], cc2 = xc[j][1], cc3 = xc[j][2];
-    const double s1 = c_hex.dN[24 * q + 3 * j], s2 = c_hex.dN[24 * q + 3 * j + 1], s3 = c_hex.dN[24 * q + 3 * j + 2];
+    double       s[3];
+    node_derivatives(row, j, s);
+    const double s1 = s[0], s2 = s[1], s3 = s[2];
     a[0] += cc1 * s1;
     a[1] += cc1 * s2;
     a[2] += cc1 * s3;
@@ -154,18 +187,22 @@ __device__ __forceinline__ void current_jacobian_x(int q, const double (*xc)[3],
     a[6] += cc3 * s1;
     a[7] += cc3 * s2;
     a[8] += cc3 * s3;
+    // four nodes' coordinates in registers at a time
+    if (j == 3) __builtin_amdgcn_sched_barrier(0);
   }
 }
 
-__device__ __forceinline__ void jacobians_x(int q, const double (*xs)[3], const double (*xc)[3], double a[9],
-                                            double b[9])
+__device__ __forceinline__ void jacobians_x(const ShapeRow& row, const double (*xs)[3], const double (*xc)[3],
+                                            double a[9], double b[9])
 {
   for (int i = 0; i < 9; i++) a[i] = b[i] = 0.0;
 #pragma unroll
   for (int j = 0; j < 8; j++) {
     const double rc1 = xs[j][0], rc2 = xs[j][1], rc3 = xs[j][2];
     const double cc1 = xc[j][0], cc2 = xc[j][1], cc3 = xc[j][2];
-    const double s1 = c_hex.dN[24 * q + 3 * j], s2 = c_hex.dN[24 * q + 3 * j + 1], s3 = c_hex.dN[24 * q + 3 * j + 2];
+    double       s[3];
+    node_derivatives(row, j, s);
+    const double s1 = s[0], s2 = s[1], s3 = s[2];
     a[0] += cc1 * s1;
     a[1] += cc1 * s2;
     a[2] += cc1 * s3;
@@ -211,10 +248,18 @@ __device__ __forceinline__ void def_grad(const double a[9], const double bi[9], 
 // (src/nimble_element.h:586-617).
 __device__ __forceinline__ void node_force(int n, const double (*ai)[10], const double (*sg)[6], double f[3])
 {
+  ShapeRow row = shape_row(n);
+#pragma unroll
+  for (int i = 0; i < 12; i++) {
+    // node n's sign in the entry's direction (signs of x: + at 1, 2, 5, 6;
+    // of y: + at 2, 3, 6, 7; of z: + at 4 .. 7)
+    const bool minus = i < 4 ? !((n + 1) & 2) : i < 8 ? !(n & 2) : !(n & 4);
+    row.m[i]         = mult_sign(row.m[i], minus ? -1.0 : 1.0);
+  }
   f[0] = f[1] = f[2] = 0.0;
 #pragma unroll
   for (int q = 0; q < 8; q++) {
-    const double d0 = c_hex.dN[24 * q + 3 * n], d1 = c_hex.dN[24 * q + 3 * n + 1], d2 = c_hex.dN[24 * q + 3 * n + 2];
+    const double d0 = row.m[shape_entry(0, q)], d1 = row.m[shape_entry(1, q)], d2 = row.m[shape_entry(2, q)];
     const double* A  = ai[q];
     const double* s  = sg[q];
     const double  x1 = d0 * A[0] + d1 * A[3] + d2 * A[6];
@@ -294,10 +339,10 @@ __device__ __forceinline__ void element_fp64(Lds& lds, int64_t e, bool valid, do
   if (valid) {
     double a[9];
     if (kRefTable || kMode == kElementForcesFromStress) {
-      current_jacobian_x(k, lds.nodes.xc[el], a);
+      current_jacobian_x(shape_row(k), lds.nodes.xc[el], a);
     } else {
       double b[9];
-      jacobians_x(k, lds.nodes.x[el], lds.nodes.xc[el], a, b);
+      jacobians_x(shape_row(k), lds.nodes.x[el], lds.nodes.xc[el], a, b);
       detb = invert3x3<false>(b, bi);
     }
     if (kMode != kElementForcesFromStress) {
@@ -364,8 +409,21 @@ __global__ __launch_bounds__(kThreads, kMode == kElementFull && kRefTable ? 5 : 
                                  status);
 }
 
-// Ensemble: workgroup g takes chunk chunks[g] (at most kEPW elements of one
-// block of one sample); the sample's slots are [3][8][E_mesh] at slot_base,
+constexpr int kParts = kFp64ChunkElems / kEPW;
+static_assert(kFp64ChunkElems % kEPW == 0, "whole parts");
+__device__ __forceinline__ EnsRange ens_chunk_part(const EnsRange* __restrict__ chunks, unsigned g)
+{
+  EnsRange  ch    = ens_load(chunks, (int64_t)(g / kParts));
+  const int first = (int)(g % kParts) * kEPW;
+  ch.first += first;
+  ch.count = min(ch.count - first, kEPW);
+  return ch;
+}
+
+// Ensemble: workgroup g takes part g % kParts (kEPW elements) of chunk
+// chunks[g / kParts] (at most kFp64ChunkElems elements of one block of one
+// sample; a table of single wavefronts' ranges would be four times as long to
+// build and upload); the sample's slots are [3][8][E_mesh] at slot_base,
 // its mesh's reference Jacobians [E_mesh][8][10] at 80 elem_base.
 __global__ __launch_bounds__(kThreads, 5) void k_ens_element_fp64(EnsNodes en, const EnsRange* __restrict__ chunks,
                                                                const int* __restrict__ conn,
@@ -375,7 +433,8 @@ __global__ __launch_bounds__(kThreads, 5) void k_ens_element_fp64(EnsNodes en, c
                                                                double* __restrict__ slots, int* __restrict__ status)
 {
   __shared__ Lds  lds;
-  const EnsRange  ch = ens_load(chunks, (int64_t)xcd_tile(blockIdx.x, gridDim.x));
+  const EnsRange  ch = ens_chunk_part(chunks, xcd_tile(blockIdx.x, gridDim.x));
+  if (ch.count <= 0) return;  // uniform across the workgroup
   const EnsSample sm = ens_load(en.samples, (int64_t)ch.s);
   const EnsMesh   ms = ens_load(en.meshes, (int64_t)sm.mesh);
   const int       el = threadIdx.x >> 3;
@@ -406,7 +465,7 @@ __global__ __launch_bounds__(kThreads) void k_reference_jacobians(int64_t E, con
   __syncthreads();
   if (e < E) {
     double b[9], bi[9];
-    reference_jacobian(k, xs[el], b);
+    reference_jacobian(shape_row(k), xs[el], b);
     const double det = invert3x3(b, bi);
 #pragma unroll
     for (int i = 0; i < 9; i++) out[(e * 8 + k) * 10 + i] = bi[i];
@@ -432,7 +491,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_defgrad(int64_t E, const doub
   __syncthreads();
   if (e < E) {
     double a[9], b[9], bi[9], Fq[9];
-    jacobians(k, xs[el], us[el], a, b);
+    jacobians(shape_row(k), xs[el], us[el], a, b);
     if (invert3x3<false>(b, bi) <= 0.0) atomicOr(status, 1);
     def_grad(a, bi, Fq);
     for (int i = 0; i < 9; i++) F[(e * 8 + k) * 9 + i] = Fq[i];
@@ -456,7 +515,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_forces(int64_t E, const doubl
   double ainv[10];
   if (e < E) {
     double a[9], b[9];
-    jacobians_x(k, lds.nodes.x[el], lds.nodes.xc[el], a, b);
+    jacobians_x(shape_row(k), lds.nodes.x[el], lds.nodes.xc[el], a, b);
     ainv[9] = invert3x3(a, ainv);
     if (ainv[9] <= 0.0) atomicOr(status, 1);
   }
@@ -531,7 +590,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_lumped_mass(int64_t E, double
   __syncthreads();
   if (e < E) {
     double a[9], b[9], bi[9];
-    jacobians(k, xs[el], zs[el], a, b);
+    jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
     if (det[el][k] <= 0.0) atomicOr(status, 1);
   }
@@ -600,7 +659,7 @@ __global__ __launch_bounds__(kThreads) void k_element_mass(int64_t e_begin, int6
   __syncthreads();
   if (e < e_end) {
     double a[9], b[9], bi[9];
-    jacobians(k, xs[el], zs[el], a, b);
+    jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
     if (det[el][k] <= 0.0) atomicOr(status, 1);
   }
@@ -617,7 +676,7 @@ __global__ __launch_bounds__(kThreads) void k_ens_element_mass(EnsNodes en, cons
                                                                int* __restrict__ status)
 {
   __shared__ double xs[kEPW][8][3], zs[kEPW][8][3], det[kEPW][8];
-  const EnsRange    ch = ens_load(chunks, (int64_t)blockIdx.x);
+  const EnsRange    ch = ens_chunk_part(chunks, blockIdx.x);
   const EnsSample   sm = ens_load(en.samples, (int64_t)ch.s);
   const EnsMesh     ms = ens_load(en.meshes, (int64_t)sm.mesh);
   const int         el = threadIdx.x >> 3, k = threadIdx.x & 7;
@@ -634,7 +693,7 @@ __global__ __launch_bounds__(kThreads) void k_ens_element_mass(EnsNodes en, cons
   __syncthreads();
   if (ok) {
     double a[9], b[9], bi[9];
-    jacobians(k, xs[el], zs[el], a, b);
+    jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
     if (det[el][k] <= 0.0) atomicOr(status, 1);
   }
@@ -719,7 +778,7 @@ void launch_ens_element_fp64(const EnsNodes& en, const EnsRange* chunks, int num
                              hipStream_t s)
 {
   if (num_chunks <= 0) return;
-  hipLaunchKernelGGL(k_ens_element_fp64, dim3((unsigned)num_chunks), dim3(kThreads), 0, s, en, chunks, conn, rjac, K,
+  hipLaunchKernelGGL(k_ens_element_fp64, dim3((unsigned)num_chunks * kParts), dim3(kThreads), 0, s, en, chunks, conn, rjac, K,
                      G, slots, status);
 }
 
@@ -727,7 +786,7 @@ void launch_ens_element_mass(const EnsNodes& en, const EnsRange* chunks, int num
                              const double* rho, double* elem_mass, int* status, hipStream_t s)
 {
   if (num_chunks <= 0) return;
-  hipLaunchKernelGGL(k_ens_element_mass, dim3((unsigned)num_chunks), dim3(kThreads), 0, s, en, chunks, conn, rho,
+  hipLaunchKernelGGL(k_ens_element_mass, dim3((unsigned)num_chunks * kParts), dim3(kThreads), 0, s, en, chunks, conn, rho,
                      elem_mass, status);
 }
 

@@ -162,8 +162,13 @@ __device__ __forceinline__ double cbrt_ref(double x)
   return ldexp(x > 0.0 ? ym : -ym, xe / 3);
 }
 
-// x times the sign of y (src/nimble_utils.h:131-136)
-__device__ __forceinline__ double mult_sign(double x, double y) { return x * (double)(1 - 2 * (y < 0.0)); }
+// x times the sign of y (src/nimble_utils.h:131-136): x (1 - 2 (y < 0)), the
+// product with -1 or 1 as a flip of the sign bit
+__device__ __forceinline__ double mult_sign(double x, double y)
+{
+  const uint64_t flip = y < 0.0 ? 0x8000000000000000ull : 0ull;
+  return __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, x) ^ flip);
+}
 
 // 6/5 minimax rational approximation of cos(acos(x)/3) on [0,1]
 // (coefficients as published in src/nimble_utils.h:650-665).
@@ -228,11 +233,13 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
   const bool k2l   = !(k0l || k1l);
 
   double kr[3], ra[3], rb[3];
-  for (int i = 0; i < 3; i++) kr[i] = (k0l ? r0[i] : 0.0) + (k1l ? r1[i] : 0.0) + (k2l ? r2[i] : 0.0);
+  // exactly one of k0l, k1l, k2l holds: the reference's sum of the chosen row
+  // and two zeros is the chosen row plus 0.0
+  for (int i = 0; i < 3; i++) kr[i] = (k0l ? r0[i] : k1l ? r1[i] : r2[i]) + 0.0;
   for (int i = 0; i < 3; i++) ra[i] = k0l ? r1[i] : r0[i];
   for (int i = 0; i < 3; i++) rb[i] = k2l ? r1[i] : r2[i];
 
-  const double ki_ki = 1.0 / ((k0l ? k0 : 0.0) + (k1l ? k1 : 0.0) + (k2l ? k2 : 0.0));
+  const double ki_ki = 1.0 / (k0l ? k0 : k1l ? k1 : k2);  // k0, k1, k2: sums of squares, never -0.0
 
   const double ki_dpr1 = ki_ki * (kr[0] * ra[0] + kr[1] * ra[1] + kr[2] * ra[2]);
   const double ki_dpr2 = ki_ki * (kr[0] * rb[0] + kr[1] * rb[1] + kr[2] * rb[2]);
@@ -279,7 +286,8 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
 
   for (int i = 0; i < 3; i++) e0[i] = fac1 * ar[i] - fac2 * kr[i];
   const bool both_zero = (rm2xx2 == 0.0) && (rm2xy_rm2xy == 0.0);
-  for (int i = 0; i < 3; i++) e0[i] = both_zero ? ar[i] : e0[i];
+  if (__builtin_expect(__ballot(both_zero) != 0, 0))  // uniform across the wave
+    for (int i = 0; i < 3; i++) e0[i] = both_zero ? ar[i] : e0[i];
 
   e1[0] = e2[1] * e0[2] - e2[2] * e0[1];
   e1[1] = e2[2] * e0[0] - e2[0] * e0[2];
@@ -291,18 +299,23 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
 
   const double c2tol = (c1 * c1) * (-1.0e-30);
   const bool   neg   = c2 < c2tol;  // otherwise: triple eigenvalue
-  ev[0] = neg ? eval0 : c1;
-  ev[1] = neg ? eval1 : c1;
-  ev[2] = neg ? eval2 : c1;
-  e0[0] = neg ? e0[0] : 1.0;
-  e0[1] = neg ? e0[1] : 0.0;
-  e0[2] = neg ? e0[2] : 0.0;
-  e1[0] = neg ? e1[0] : 0.0;
-  e1[1] = neg ? e1[1] : 1.0;
-  e1[2] = neg ? e1[2] : 0.0;
-  e2[0] = neg ? e2[0] : 0.0;
-  e2[1] = neg ? e2[1] : 0.0;
-  e2[2] = neg ? e2[2] : 1.0;
+  ev[0] = eval0;
+  ev[1] = eval1;
+  ev[2] = eval2;
+  if (__builtin_expect(__ballot(!neg) != 0, 0)) {  // uniform across the wave
+    ev[0] = neg ? eval0 : c1;
+    ev[1] = neg ? eval1 : c1;
+    ev[2] = neg ? eval2 : c1;
+    e0[0] = neg ? e0[0] : 1.0;
+    e0[1] = neg ? e0[1] : 0.0;
+    e0[2] = neg ? e0[2] : 0.0;
+    e1[0] = neg ? e1[0] : 0.0;
+    e1[1] = neg ? e1[1] : 1.0;
+    e1[2] = neg ? e1[2] : 0.0;
+    e2[0] = neg ? e2[0] : 0.0;
+    e2[1] = neg ? e2[1] : 0.0;
+    e2[2] = neg ? e2[2] : 1.0;
+  }
 }
 
 // Left stretch V of F = V R from the eigen-decomposition of F^{-T} F^{-1}

@@ -136,6 +136,9 @@ __host__ __device__ __forceinline__ int64_t fp64_slot(int64_t e, int j) { return
 __host__ __device__ __forceinline__ int64_t round_up8(int64_t n) { return (n + 7) & ~(int64_t)7; }
 
 // ---- element kernels over the elements of a block table ----
+// elements per workgroup of the FP64 element kernels (one wavefront), and per
+// entry of an ensemble's chunk table
+constexpr int kFp64Elems = 8, kFp64ChunkElems = 32;
 // FP64 element kernel modes: F, stress and forces; F only; forces from the
 // stress already in sip
 constexpr int kElementFull = 0, kElementDefGrad = 1, kElementForcesFromStress = 2;
