@@ -474,62 +474,137 @@ __global__ __launch_bounds__(kThreads) void k_reference_jacobians(int64_t E, con
 }
 
 // ---------------------------------------------------------------------------
-// Seams on gathered arrays
+// Seams on gathered arrays.  A wave's share of a row-major [E][..] array
+// is one contiguous range, but a lane's row of it (3, 6 or 9 doubles) is not
+// a whole number of cache lines, and a wave that loads or stores its lanes'
+// rows value by value touches every line of the range once per value.  So the
+// ranges move between memory and LDS in address order (8 bytes per lane, 512
+// contiguous bytes per wave and instruction; doubles need no more alignment
+// than the caller's arrays have) and the lanes take their rows from LDS.
+// What bounds them then is memory: 500,009 elements, deformation gradients
+// 186 -> 92 us (960 bytes per element, 5.2 TB/s), forces 166 -> 115 us (960
+// bytes, 4.2 TB/s).  The stress seam is bound by VALU issue (98% of the SIMD
+// cycles at 864 instructions per point, 128 us for 4.0M points) and keeps its
+// direct loads: through LDS it took 130-139 us.
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kThreads) void k_seam_defgrad(int64_t E, const double* __restrict__ Xg,
+// Values threadIdx.x + i kThreads, i < kPer, of the n >= 1 at g, every load in
+// flight at once (a thread past the end takes the last value).
+template <int kPer>
+__device__ __forceinline__ void load_range(const double* __restrict__ g, int n, double (&r)[kPer])
+{
+#pragma unroll
+  for (int i = 0; i < kPer; i++) r[i] = g[min((int)threadIdx.x + i * kThreads, n - 1)];
+}
+template <int kPer>
+__device__ __forceinline__ void put_range(const double (&r)[kPer], double* s)
+{
+#pragma unroll
+  for (int i = 0; i < kPer; i++) s[threadIdx.x + i * kThreads] = r[i];
+}
+// the n values at s in LDS to g
+template <int kPer>
+__device__ __forceinline__ void store_range(const double* s, int n, double* __restrict__ g)
+{
+  double r[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; i++) r[i] = s[threadIdx.x + i * kThreads];
+#pragma unroll
+  for (int i = 0; i < kPer; i++)
+    if ((int)threadIdx.x + i * kThreads < n) g[threadIdx.x + i * kThreads] = r[i];
+}
+
+// A seam's status word is host memory the device writes only when an element
+// is inverted; it is read after the stream has been waited for.
+__device__ __forceinline__ void raise(int* status)
+{
+  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kThreads, 4) void k_seam_defgrad(int64_t E, const double* __restrict__ Xg,
                                                            const double* __restrict__ ug, double* __restrict__ F,
                                                            int* __restrict__ status)
 {
-  __shared__ double xs[kEPW][8][3], us[kEPW][8][3];
+  __shared__ __attribute__((aligned(16))) union {
+    struct {
+      double x[kEPW][8][3], xc[kEPW][8][3];  // X and X + u
+    } in;
+    double F[kThreads * 9];
+  } lds;
   const int     el = threadIdx.x >> 3, k = threadIdx.x & 7;
-  const int64_t e  = (int64_t)blockIdx.x * kEPW + el;
-  if (e < E)
-    for (int c = 0; c < 3; c++) {
-      xs[el][k][c] = Xg[(e * 8 + k) * 3 + c];
-      us[el][k][c] = ug[(e * 8 + k) * 3 + c];
-    }
+  const int64_t e0 = (int64_t)blockIdx.x * kEPW;
+  const int     ne = (int)(E - e0 < kEPW ? E - e0 : kEPW);
+  double        xr[3], ur[3];
+  load_range(Xg + 24 * e0, 24 * ne, xr);
+  load_range(ug + 24 * e0, 24 * ne, ur);
+  put_range(xr, &lds.in.x[0][0][0]);
+#pragma unroll
+  for (int i = 0; i < 3; i++) xr[i] = xr[i] + ur[i];
+  put_range(xr, &lds.in.xc[0][0][0]);
   __syncthreads();
-  if (e < E) {
-    double a[9], b[9], bi[9], Fq[9];
-    jacobians(shape_row(k), xs[el], us[el], a, b);
-    if (invert3x3<false>(b, bi) <= 0.0) atomicOr(status, 1);
+  double Fq[9];
+  if (el < ne) {
+    // one Jacobian after the other: both at once take twice the registers
+    const ShapeRow row = shape_row(k);
+    double         a[9], b[9], bi[9];
+    reference_jacobian(row, lds.in.x[el], b);
+    if (invert3x3(b, bi) <= 0.0) raise(status);
+    __builtin_amdgcn_sched_barrier(0);
+    current_jacobian_x(row, lds.in.xc[el], a);
     def_grad(a, bi, Fq);
-    for (int i = 0; i < 9; i++) F[(e * 8 + k) * 9 + i] = Fq[i];
   }
+  __syncthreads();
+  if (el < ne)
+#pragma unroll
+    for (int i = 0; i < 9; i++) lds.F[9 * threadIdx.x + i] = Fq[i];
+  __syncthreads();
+  store_range<9>(lds.F, 72 * ne, F + 72 * e0);
 }
 
-__global__ __launch_bounds__(kThreads) void k_seam_forces(int64_t E, const double* __restrict__ Xg,
+__global__ __launch_bounds__(kThreads, 5) void k_seam_forces(int64_t E, const double* __restrict__ Xg,
                                                           const double* __restrict__ ug,
                                                           const double* __restrict__ sig, double* __restrict__ f,
                                                           int* __restrict__ status)
 {
-  __shared__ Lds lds;
+  __shared__ __attribute__((aligned(16))) struct {
+    union {
+      double xc[kEPW][8][3];
+      double ai[kEPW][8][10];
+      double f[kThreads * 3];
+    };
+    double sg[kEPW][8][6];
+  } lds;
   const int     el = threadIdx.x >> 3, k = threadIdx.x & 7;
-  const int64_t e  = (int64_t)blockIdx.x * kEPW + el;
-  if (e < E)
-    for (int c = 0; c < 3; c++) {
-      lds.nodes.x[el][k][c]  = Xg[(e * 8 + k) * 3 + c];
-      lds.nodes.xc[el][k][c] = Xg[(e * 8 + k) * 3 + c] + ug[(e * 8 + k) * 3 + c];
-    }
+  const int64_t e0 = (int64_t)blockIdx.x * kEPW;
+  const int     ne = (int)(E - e0 < kEPW ? E - e0 : kEPW);
+  double        xr[3], ur[3], sr[6];
+  load_range(Xg + 24 * e0, 24 * ne, xr);
+  load_range(ug + 24 * e0, 24 * ne, ur);
+  load_range(sig + 48 * e0, 48 * ne, sr);
+#pragma unroll
+  for (int i = 0; i < 3; i++) xr[i] = xr[i] + ur[i];
+  put_range(xr, &lds.xc[0][0][0]);
+  put_range(sr, &lds.sg[0][0][0]);
   __syncthreads();
   double ainv[10];
-  if (e < E) {
-    double a[9], b[9];
-    jacobians_x(shape_row(k), lds.nodes.x[el], lds.nodes.xc[el], a, b);
+  if (el < ne) {
+    double a[9];
+    current_jacobian_x(shape_row(k), lds.xc[el], a);
     ainv[9] = invert3x3(a, ainv);
-    if (ainv[9] <= 0.0) atomicOr(status, 1);
+    if (ainv[9] <= 0.0) raise(status);
   }
   __syncthreads();
-  if (e < E) {
-    for (int i = 0; i < 10; i++) lds.pts.ai[el][k][i] = ainv[i];
-    for (int i = 0; i < 6; i++) lds.pts.sg[el][k][i] = sig[(e * 8 + k) * 6 + i];
-  }
+  if (el < ne)
+#pragma unroll
+    for (int i = 0; i < 10; i++) lds.ai[el][k][i] = ainv[i];
   __syncthreads();
-  if (e < E) {
-    double fn[3];
-    node_force(k, lds.pts.ai[el], lds.pts.sg[el], fn);
-    for (int c = 0; c < 3; c++) f[(e * 8 + k) * 3 + c] = fn[c];
-  }
+  double fn[3];
+  if (el < ne) node_force(k, lds.ai[el], lds.sg[el], fn);
+  __syncthreads();
+  if (el < ne)
+#pragma unroll
+    for (int c = 0; c < 3; c++) lds.f[3 * threadIdx.x + c] = fn[c];
+  __syncthreads();
+  store_range<3>(lds.f, 24 * ne, f + 24 * e0);
 }
 
 __global__ __launch_bounds__(256) void k_seam_stress(int64_t P, double K, double G, const double* __restrict__ F,
@@ -592,7 +667,7 @@ __global__ __launch_bounds__(kThreads) void k_seam_lumped_mass(int64_t E, double
     double a[9], b[9], bi[9];
     jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
-    if (det[el][k] <= 0.0) atomicOr(status, 1);
+    if (det[el][k] <= 0.0) raise(status);
   }
   __syncthreads();
   if (e < E) lumped_row(k, rho, det[el], &m[e * 8 + k]);

@@ -69,23 +69,82 @@ namespace {
     if (_e != hipSuccess) return fail(NSM_ERR_HIP, "kernel launch: %s", hipGetErrorString(_e));    \
   } while (0)
 
-// Small device scratch shared by the stateless seam entry points: one status
-// word per device, allocated on first use and kept for the process.
-std::mutex       g_seam_mutex;
-std::map<int, int*> g_seam_status;
-
-int seam_status_buffer(int** out)
-{
-  int dev = 0;
-  NSM_HIP(hipGetDevice(&dev));
-  std::lock_guard<std::mutex> lk(g_seam_mutex);
-  auto                        it = g_seam_status.find(dev);
-  if (it == g_seam_status.end()) {
-    int* p = nullptr;
-    NSM_HIP(hipMalloc(&p, sizeof(int)));
-    it = g_seam_status.emplace(dev, p).first;
+// Status words of the stateless seam entry points: pinned host memory every
+// device can write, one word per call in flight (a cache line each), taken
+// from a free list for the length of the call, so calls on different threads
+// and streams do not share one.  A word holds 0 unless a kernel of its call
+// met an inverted element.  The call waits for its stream and reads the word
+// where it lies: clearing a device word before the kernel and copying it to
+// the host after it cost a call two more stream operations.
+// A call on 343 elements: 20 -> 13 us.
+class SeamStatus {
+ public:
+  // the call's word, 0 on entry
+  static int take(int** out)
+  {
+    std::lock_guard<std::mutex> lk(mutex());
+    if (!free_list()) {
+      constexpr size_t kPage = 4096;
+      char*            p     = nullptr;
+      NSM_HIP(hipHostMalloc((void**)&p, kPage, hipHostMallocPortable));
+      std::memset(p, 0, kPage);
+      for (size_t i = 0; i < kPage; i += sizeof(Line)) {
+        Line* l     = (Line*)(p + i);
+        l->next     = free_list();
+        free_list() = l;
+      }
+    }
+    Line* l     = free_list();
+    free_list() = l->next;
+    *out        = &l->word;
+    return NSM_OK;
   }
-  *out = it->second;
+  static void give_back(int* w)
+  {
+    Line* l                  = (Line*)w;
+    *(volatile int*)&l->word = 0;
+    std::lock_guard<std::mutex> lk(mutex());
+    l->next     = free_list();
+    free_list() = l;
+  }
+
+ private:
+  struct alignas(64) Line {
+    int   word;
+    Line* next;
+  };
+  // never destroyed: calls may still run while the process ends
+  static std::mutex& mutex()
+  {
+    static std::mutex* m = new std::mutex;
+    return *m;
+  }
+  static Line*& free_list()
+  {
+    static Line* head = nullptr;
+    return head;
+  }
+};
+
+// `launch` with a status word on `stream`, and its outcome once the stream
+// has done it
+template <typename Launch>
+int run_seam(int64_t n, void* stream, Launch&& launch)
+{
+  if (n < 0) return fail(NSM_ERR_ARG, "negative size");
+  if (n == 0) return NSM_OK;
+  int* status = nullptr;
+  int  st     = SeamStatus::take(&status);
+  if (st) return st;
+  launch(status, (hipStream_t)stream);
+  hipError_t e = hipGetLastError();
+  const hipError_t done = hipStreamSynchronize((hipStream_t)stream);
+  if (e == hipSuccess) e = done;
+  const int h = *(volatile int*)status;
+  // a word whose kernel may still be running is not used again
+  if (done == hipSuccess) SeamStatus::give_back(status);
+  if (e != hipSuccess) return fail(NSM_ERR_HIP, "element seam: %s", hipGetErrorString(e));
+  if (h) return fail(NSM_ERR_NEG_JACOBIAN, "non-positive Jacobian determinant (Invert3x3)");
   return NSM_OK;
 }
 
@@ -853,51 +912,30 @@ const char* nsm_last_error(void) { return g_last_error.c_str(); }
 const char* nsm_version(void) { return "nimblesm_amd 0.1 gfx950"; }
 
 // ------------------------------------------------------------------- seams
-#define NSM_SEAM_PROLOGUE(n)                                                          \
-  if ((n) < 0) return fail(NSM_ERR_ARG, "negative size");                             \
-  if ((n) == 0) return NSM_OK;                                                        \
-  int* status = nullptr;                                                              \
-  {                                                                                   \
-    int _st = seam_status_buffer(&status);                                            \
-    if (_st) return _st;                                                              \
-  }                                                                                   \
-  hipStream_t s = (hipStream_t)stream;                                                \
-  NSM_HIP(hipMemsetAsync(status, 0, sizeof(int), s));
-
-static int seam_epilogue(int* status, hipStream_t s)
-{
-  NSM_LAUNCHED();
-  int h = 0;
-  NSM_HIP(hipMemcpyAsync(&h, status, sizeof(int), hipMemcpyDeviceToHost, s));
-  NSM_HIP(hipStreamSynchronize(s));
-  if (h) return fail(NSM_ERR_NEG_JACOBIAN, "non-positive Jacobian determinant (Invert3x3)");
-  return NSM_OK;
-}
-
 int nsm_hex_compute_deformation_gradients(int64_t num_elem, const double* X_gathered, const double* u_gathered,
                                           double* F, void* stream)
 {
   if (num_elem > 0 && (!X_gathered || !u_gathered || !F)) return fail(NSM_ERR_ARG, "null pointer");
-  NSM_SEAM_PROLOGUE(num_elem);
-  nsm::launch_seam_defgrad(num_elem, X_gathered, u_gathered, F, status, s);
-  return seam_epilogue(status, s);
+  return run_seam(num_elem, stream, [&](int* status, hipStream_t s) {
+    nsm::launch_seam_defgrad(num_elem, X_gathered, u_gathered, F, status, s);
+  });
 }
 
 int nsm_hex_compute_nodal_forces(int64_t num_elem, const double* X_gathered, const double* u_gathered,
                                  const double* sigma, double* f, void* stream)
 {
   if (num_elem > 0 && (!X_gathered || !u_gathered || !sigma || !f)) return fail(NSM_ERR_ARG, "null pointer");
-  NSM_SEAM_PROLOGUE(num_elem);
-  nsm::launch_seam_forces(num_elem, X_gathered, u_gathered, sigma, f, status, s);
-  return seam_epilogue(status, s);
+  return run_seam(num_elem, stream, [&](int* status, hipStream_t s) {
+    nsm::launch_seam_forces(num_elem, X_gathered, u_gathered, sigma, f, status, s);
+  });
 }
 
 int nsm_hex_compute_lumped_mass(int64_t num_elem, double density, const double* X_gathered, double* m, void* stream)
 {
   if (num_elem > 0 && (!X_gathered || !m)) return fail(NSM_ERR_ARG, "null pointer");
-  NSM_SEAM_PROLOGUE(num_elem);
-  nsm::launch_seam_lumped_mass(num_elem, density, X_gathered, m, status, s);
-  return seam_epilogue(status, s);
+  return run_seam(num_elem, stream, [&](int* status, hipStream_t s) {
+    nsm::launch_seam_lumped_mass(num_elem, density, X_gathered, m, status, s);
+  });
 }
 
 int nsm_hex_compute_characteristic_length(int64_t num_elem, const double* x_gathered, double* out, void* stream)

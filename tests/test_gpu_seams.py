@@ -212,3 +212,35 @@ def test_quotients_at_extreme_exponents_bit_exact(hip_device, elems, scale):
     N.HexElement.ComputeNodalForces(_dev(Xs, hip_device), _dev(us, hip_device), _dev(so, hip_device), f)
     torch.cuda.synchronize()
     assert np.array_equal(f.cpu().numpy().view(np.uint64), O.nodal_forces(Xs, us, so).view(np.uint64))
+
+
+@pytest.mark.parametrize("E", [1, 7, 8, 9, 65])
+def test_seams_at_the_edges_of_a_wavefront(hip_device, elems, E):
+    """Element counts around a workgroup's 8 elements: every output is the
+    oracle's bit for bit and nothing past the last element is written; an
+    inverted last element is reported, and only by its own call."""
+    import torch
+
+    X, u = elems[0][:E].copy(), elems[1][:E]
+    guard = 80
+    new = lambda n: torch.full((n + guard,), 7.0, dtype=torch.float64, device=hip_device)  # noqa: E731
+    F, s, f = new(72 * E), new(48 * E), new(24 * E)
+    Xd, ud = _dev(X, hip_device), _dev(u, hip_device)
+    mat = N.NeohookeanMaterial(7800.0, 1.6e11, 0.8e11)
+    N.HexElement.ComputeDeformationGradients(Xd, ud, F)
+    mat.GetStress(F[:72 * E], s)
+    N.HexElement.ComputeNodalForces(Xd, ud, s, f)
+    torch.cuda.synchronize()
+    Fo = O.deformation_gradients(X, u)
+    so = O.stress(1.6e11, 0.8e11, Fo)
+    for got, want in ((F, Fo), (s, so), (f, O.nodal_forces(X, u, so))):
+        got = got.cpu().numpy()
+        assert np.array_equal(got[:-guard], want.ravel())
+        assert np.all(got[-guard:] == 7.0)
+    X[-1, 4:, 2] -= 5.0  # top face below the bottom face
+    for call in (lambda x: N.HexElement.ComputeDeformationGradients(x, ud, F),
+                 lambda x: N.HexElement.ComputeNodalForces(x, ud, s, f)):
+        with pytest.raises(N.NimbleError) as ei:
+            call(_dev(X, hip_device))
+        assert ei.value.status == 3
+        call(Xd)
