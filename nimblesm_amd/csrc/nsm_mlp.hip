@@ -28,6 +28,7 @@ namespace {
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef float  f32x4 __attribute__((ext_vector_type(4)));
 
 int fail(int status, const char* fmt, ...)
@@ -326,15 +327,15 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ y, const 
   if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
 }
 
-// loss of pass p = sum of its kMseBlocks partials (ascending) / n, for
-// passes 0 .. gridDim.x - 1 (partial[p kMseBlocks + b])
-__global__ __launch_bounds__(64) void k_mse_total(const double* __restrict__ partial, int64_t n,
+// loss of pass p = sum of its `count` partials (ascending) / n, for passes
+// 0 .. gridDim.x - 1 (partial[p count + b])
+__global__ __launch_bounds__(64) void k_mse_total(const double* __restrict__ partial, int count, int64_t n,
                                                   double* __restrict__ loss_out)
 {
   if (threadIdx.x != 0) return;
-  const double* p = partial + (int64_t)blockIdx.x * kMseBlocks;
+  const double* p = partial + (int64_t)blockIdx.x * count;
   double        s = 0.0;
-  for (int b = 0; b < kMseBlocks; b++) s += p[b];
+  for (int b = 0; b < count; b++) s += p[b];
   loss_out[blockIdx.x] = s / (double)n;
 }
 
@@ -346,21 +347,390 @@ __global__ __launch_bounds__(256) void k_bias_grad(const float* __restrict__ G, 
 }
 
 // Adam on the FP32 master parameters; BF16 copies for the forward pass.
-__global__ __launch_bounds__(256) void k_adam(float* __restrict__ p, const float* __restrict__ g,
-                                              float* __restrict__ m1, float* __restrict__ m2,
-                                              bf16* __restrict__ p_bf, int64_t n, float lr, float b1, float b2,
-                                              float c1, float c2, float eps)
+struct Adam {
+  float *p, *m1, *m2;
+  bf16*  p_bf;
+  float  lr, b1, b2, c1, c2, eps;
+};
+
+struct AdamState {
+  float p, m1, m2;
+};
+__device__ __forceinline__ AdamState adam_load(const Adam& o, int64_t i) { return {o.p[i], o.m1[i], o.m2[i]}; }
+
+// parameter i in state t with gradient gi; its new BF16 value.  The fused
+// multiply-adds are written out, so every kernel rounds alike.
+__device__ __forceinline__ bf16 adam_update(const Adam& o, int64_t i, const AdamState& t, float gi)
+{
+  const float a  = __builtin_fmaf(1.0f - o.b1, gi, o.b1 * t.m1);
+  const float v  = __builtin_fmaf(gi, (1.0f - o.b2) * gi, o.b2 * t.m2);
+  o.m1[i]        = a;
+  o.m2[i]        = v;
+  const float pi = t.p - o.lr * (a / o.c1) / (sqrtf(v / o.c2) + o.eps);
+  o.p[i]         = pi;
+  return o.p_bf[i] = (bf16)pi;
+}
+
+__global__ __launch_bounds__(256) void k_adam(Adam o, const float* __restrict__ g, int64_t n)
 {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float a  = b1 * m1[i] + (1.0f - b1) * gi;
-  const float v  = b2 * m2[i] + (1.0f - b2) * gi * gi;
-  m1[i]          = a;
-  m2[i]          = v;
-  const float pi = p[i] - lr * (a / c1) / (sqrtf(v / c2) + eps);
-  p[i]           = pi;
-  p_bf[i]        = (bf16)pi;
+  if (i < n) adam_update(o, i, adam_load(o, i), g[i]);
+}
+
+// ---------------------------------------------------------------------------
+// Small networks (at most kRowLayers layers, no width above kRowWidth): a
+// training pass in two launches instead of ten, a forward pass in one.
+//
+// Layer by layer such a pass is a chain of launches that each wait for a
+// few loads: at batch 512 the products of the 4-256-256-256-64 network are
+// 0.46 GFLOP, under a microsecond of the matrix cores, and took 69 us.  But
+// the rows of a batch are independent until the weight gradients: a
+// workgroup takes 16 rows through every layer forward, the loss and the
+// input gradients back (k_rows), activations in LDS, one wave per 16 columns
+// of a layer's output and the next layer's weights on their way to registers
+// while a layer computes.  It leaves H_l and D_l transposed, so that the
+// weight-gradient products read both operands along the batch, 16 bytes per
+// lane, straight into MFMA operands; k_weights forms every weight and bias
+// gradient in one launch and applies Adam to each where it is formed.
+// Products use the MFMA steps, K ranges and summation orders of the
+// layer-by-layer kernels: gradients and outputs are the same bits (the loss
+// adds its FP64 squares by rows).
+//
+// Weights are kept twice, in BF16 and padded to multiples of 32 with zeros:
+// wf [np][kp] with k along the input (forward), wt [kp][np] with k along the
+// output (input gradients), each in MFMA operand order (operand_index).  Padded columns of a layer's output are 0 (zero weights
+// and bias, gelu(0) = 0).  Rows past the batch, up to Bp (a multiple of 32),
+// are stored as 0 in H and D.
+//
+// Training iteration of the 4-256-256-256-64 network, layer by layer and
+// here: batch 64 54 -> 19 us, 512 66 -> 23 us, 1024 100 -> 29 us, 2048 185 ->
+// 37 us, 4096 243 -> 56 us, 16384 693 -> 205 us.  At 512: k_rows 15 us, of
+// which about 4 are weight loads (one CU reads the 0.6 MB of both copies from
+// L2) and 3 the stores of H, D and G, the rest the chain of seven dependent
+// products; k_weights 8 us, one round of loads per 16 K steps and Adam.
+// ---------------------------------------------------------------------------
+constexpr int kRowWidth = 256, kRowLayers = 4, kRowThreads = 1024, kRowSteps = kRowWidth / kKStep;
+
+// Place of element (r, k) of an operand of `steps` k steps stored in MFMA
+// operand order: 16 rows x 32 k are one contiguous block of 1 KB, lane
+// r % 16 + 16 (k % 32 / 8) holding 16 bytes of it.  A wave's operand load is
+// then 1 KB in lane order; from rows at a stride it took four times as long
+// (consecutive lanes in different cache lines), and a pass of k_rows 27 us.
+__device__ __forceinline__ int64_t operand_index(int64_t r, int64_t k, int64_t steps)
+{
+  return ((r >> 4) * steps + (k >> 5)) * 512 + ((r & 15) + 16 * ((k & 31) >> 3)) * 8 + (k & 7);
+}
+
+struct RowLayer {
+  int          din, dout, kp, np;  // widths, and rounded up to 32
+  int64_t      w_off, b_off;       // in the flat parameter array
+  bf16 *       wf, *wt;
+  const float* bias;
+  bf16 *       ht, *dt;  // H of the layer's input [kp][Bp], D of its output [np][Bp], in operand order
+  float*       gt;       // G of its output [Bp][np]
+};
+
+struct RowArgs {
+  int64_t      B, Bp;
+  const float* x;        // [B][d_0]
+  const float* target;   // [B][d_L] (training)
+  float*       y;        // [B][d_L] (forward only)
+  double*      partial;  // squared error per workgroup (training)
+  float        scale;    // 2 / (B d_L)
+  RowLayer     l[kRowLayers];
+};
+
+// One wave's columns of a layer's weights: lane c + 16 q holds column c,
+// k = 32 s + 8 q .. + 7 in v[s].
+struct RowWeights {
+  bf16x8 v[kRowSteps];
+};
+
+// Every load is executed whatever the layer's size (past its columns or its
+// last k step the indices are clamped): with no branch around them the waits
+// for one layer's weights leave the next layer's in flight.
+__device__ __forceinline__ void load_weights(const bf16* w, int ld, int cols, int wave, int lane, RowWeights& f)
+{
+  const bf16x8* p = reinterpret_cast<const bf16x8*>(w + (int64_t)min(wave, cols / 16 - 1) * 16 * ld) + lane;
+#pragma unroll
+  for (int s = 0; s < kRowSteps; s++) f.v[s] = p[64 * min(s, ld / kKStep - 1)];
+}
+
+// Rows of a workgroup in the matrix-core tiles: tile t's accumulator lane
+// c + 16 q holds column c of tile rows 4 q .. 4 q + 3, of which the first
+// kPer are rows 4 kPer t + kPer q + r of the workgroup (the others repeat the
+// last of them and are not used).
+template <int kPer, int kRT, int kLd>
+__device__ __forceinline__ void row_product(const bf16 (*act)[kLd], const RowWeights& f, int kp, int lane,
+                                            f32x4 (&acc)[kRT])
+{
+  const int m = lane & 15, row = (m >> 2) * kPer + min(m & 3, kPer - 1);
+#pragma unroll
+  for (int t = 0; t < kRT; t++) {
+    const bf16* p = &act[4 * kPer * t + row][8 * (lane >> 4)];
+    bf16x8      v[kRowSteps];
+#pragma unroll
+    for (int s = 0; s < kRowSteps; s++) v[s] = *reinterpret_cast<const bf16x8*>(p + min(s * kKStep, kp - kKStep));
+    acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (kp == kRowWidth) {  // uniform
+#pragma unroll
+      for (int s = 0; s < kRowSteps; s++)
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[s], f.v[s], acc[t], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int s = 0; s < kRowSteps - 1; s++)
+        if (s * kKStep < kp) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[s], f.v[s], acc[t], 0, 0, 0);
+    }
+  }
+}
+
+// kL layers, 4 kPer kRT rows per workgroup
+template <int kL, int kPer, int kRT, bool kTrain>
+__global__ __launch_bounds__(kRowThreads) void k_rows(RowArgs a)
+{
+  constexpr int kRows = 4 * kPer * kRT, kLd = kRowWidth + kPad;
+  typedef float  fvec __attribute__((ext_vector_type(kPer)));
+  typedef __bf16 bvec __attribute__((ext_vector_type(kPer)));
+  __shared__ __attribute__((aligned(16))) bf16 act[2][kRows][kLd];
+  __shared__ double                            red[kRowThreads / 64];
+  const int     tid = (int)threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int     col = wave * 16 + (lane & 15), row0 = kPer * (lane >> 4);
+  const int64_t b0  = (int64_t)blockIdx.x * kRows;
+
+  RowWeights w;
+  load_weights(a.l[0].wf, a.l[0].kp, a.l[0].np, wave, lane, w);
+  {
+    const int din = a.l[0].din, kp = a.l[0].kp;
+    for (int i = tid; i < kRows * kp; i += kRowThreads) {
+      const int  r = i & (kRows - 1), k = i / kRows;
+      const bool ok = b0 + r < a.B && k < din;
+      const bf16 v  = ok ? (bf16)a.x[(b0 + r) * din + k] : (bf16)0.0f;
+      act[0][r][k]  = v;
+      if (kTrain) a.l[0].ht[operand_index(k, b0 + r, a.Bp / kKStep)] = v;
+    }
+  }
+  float gp[kL][kRT][kPer];  // gelu'(z) of the hidden layers (training)
+  float bias[kL], tgt[kRT][kPer];
+#pragma unroll
+  for (int l = 0; l < kL; l++) bias[l] = a.l[l].bias[min(col, a.l[l].dout - 1)];
+  if (kTrain)
+#pragma unroll
+    for (int t = 0; t < kRT; t++)
+#pragma unroll
+      for (int r = 0; r < kPer; r++)
+        tgt[t][r] = a.target[min(b0 + 4 * kPer * t + row0 + r, a.B - 1) * a.l[kL - 1].dout +
+                             min(col, a.l[kL - 1].dout - 1)];
+  __syncthreads();
+
+#pragma unroll
+  for (int l = 0; l < kL; l++) {
+    const RowLayer& y  = a.l[l];
+    const RowLayer& up = a.l[l + 1 < kL ? l + 1 : l];
+    RowWeights next;
+    if (l + 1 < kL)
+      load_weights(up.wf, up.kp, up.np, wave, lane, next);
+    else if (kTrain && kL > 1)
+      load_weights(y.wt, y.np, y.kp, wave, lane, next);
+    double sq = 0.0;
+    if (wave * 16 < y.np) {
+      f32x4 acc[kRT];
+      row_product<kPer, kRT, kLd>(act[l & 1], w, y.kp, lane, acc);
+#pragma unroll
+      for (int t = 0; t < kRT; t++) {
+        const int     rl = 4 * kPer * t + row0;  // first of the lane's kPer rows
+        const int64_t at = operand_index(col, b0 + rl, a.Bp / kKStep);
+        bvec          hv;
+        fvec          gv;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) {
+          const bool  ok = b0 + rl + r < a.B;
+          const float z  = acc[t][r] + (col < y.dout ? bias[l] : 0.0f);
+          if (l + 1 < kL) {
+            if (kTrain) gp[l][t][r] = gelu_grad(z);
+            const bf16 h                  = (bf16)gelu(z);
+            act[(l + 1) & 1][rl + r][col] = h;
+            hv[r]                         = ok ? h : (bf16)0.0f;
+          } else if (!kTrain) {
+            if (ok && col < y.dout) a.y[(b0 + rl + r) * y.dout + col] = z;
+          } else {
+            const float e = ok && col < y.dout ? z - tgt[t][r] : 0.0f;
+            sq += (double)e * (double)e;
+            gv[r]                         = a.scale * e;
+            hv[r]                         = (bf16)gv[r];
+            act[(l + 1) & 1][rl + r][col] = hv[r];
+          }
+        }
+        if (kTrain && l + 1 < kL) {
+          *reinterpret_cast<bvec*>(up.ht + at) = hv;
+        } else if (kTrain) {
+#pragma unroll
+          for (int r = 0; r < kPer; r++) y.gt[(b0 + rl + r) * y.np + col] = gv[r];
+          *reinterpret_cast<bvec*>(y.dt + at) = hv;
+        }
+      }
+    }
+    if (kTrain && l == kL - 1) {
+#pragma unroll
+      for (int m = 32; m > 0; m >>= 1) sq += __shfl_down(sq, m, 64);
+      if (lane == 0) red[wave] = sq;
+    }
+    if (kTrain || l + 1 < kL) __syncthreads();
+    w = next;
+  }
+  if (!kTrain) return;
+  if (tid == 0) {
+    double s = 0.0;
+    for (int i = 0; i < kRowThreads / 64; i++) s += red[i];
+    a.partial[blockIdx.x] = s;
+  }
+
+  // G of layer l - 1's output = (D_l W_l) gelu'(z), its D in act
+#pragma unroll
+  for (int l = kL - 1; l > 0; l--) {
+    const RowLayer& y    = a.l[l];
+    const RowLayer& dst  = a.l[l > 0 ? l - 1 : 0];
+    const int       from = (kL - 1 - l + (kL & 1)) & 1;  // act[kL & 1] holds D of the last layer
+    RowWeights      next;
+    if (l > 1) load_weights(dst.wt, dst.np, dst.kp, wave, lane, next);
+    if (wave * 16 < y.kp) {
+      f32x4 acc[kRT];
+      row_product<kPer, kRT, kLd>(act[from], w, y.np, lane, acc);
+#pragma unroll
+      for (int t = 0; t < kRT; t++) {
+        const int     rl = 4 * kPer * t + row0;
+        const int64_t at = operand_index(col, b0 + rl, a.Bp / kKStep);
+        bvec          dv;
+        fvec          gv;
+#pragma unroll
+        for (int r = 0; r < kPer; r++) {
+          gv[r] = b0 + rl + r < a.B ? acc[t][r] * gp[l > 0 ? l - 1 : 0][t][r] : 0.0f;
+          dv[r] = (bf16)gv[r];
+          act[from ^ 1][rl + r][col] = dv[r];
+        }
+#pragma unroll
+        for (int r = 0; r < kPer; r++) dst.gt[(b0 + rl + r) * dst.np + col] = gv[r];
+        *reinterpret_cast<bvec*>(dst.dt + at) = dv;
+      }
+    }
+    if (l > 1) __syncthreads();
+    w = next;
+  }
+}
+
+// Weight and bias gradients of every layer from H and D: workgroups
+// [0, tiles[0]) take 32 x 32 tiles of the first layer's weights (four waves
+// of 16 x 16), the next tiles[1] the second's, ..., then four bias columns
+// each.  The K range (batch) is cut and summed as mlp_gemm's split-K does.
+// kUpdate: Adam on each parameter where its gradient is formed, else the
+// gradients go to g.
+struct WeightArgs {
+  int      layers;
+  int      tiles[kRowLayers], tiles_x[kRowLayers];
+  int64_t  B, Bp;
+  int      splits, k_chunk;
+  float*   g;
+  Adam     adam;
+  RowLayer l[kRowLayers];
+};
+
+template <bool kUpdate>
+__global__ __launch_bounds__(256) void k_weights(WeightArgs a)
+{
+  const int lane = (int)threadIdx.x & 63, wave = (int)threadIdx.x >> 6;
+  int       w    = (int)blockIdx.x;
+#pragma unroll
+  for (int l = 0; l < kRowLayers; l++) {
+    if (l >= a.layers) break;
+    const RowLayer& y = a.l[l];
+    if (w >= a.tiles[l]) {
+      w -= a.tiles[l];
+      continue;
+    }
+    const int m0 = (w / a.tiles_x[l]) * 32 + (wave >> 1) * 16, n0 = (w % a.tiles_x[l]) * 32 + (wave & 1) * 16;
+    if (m0 >= y.dout || n0 >= y.din) return;  // uniform across the wave
+    const bf16x8* pd = reinterpret_cast<const bf16x8*>(y.dt + m0 * a.Bp) + lane;
+    const bf16x8* ph = reinterpret_cast<const bf16x8*>(y.ht + n0 * a.Bp) + lane;
+    // this lane's four parameters, loaded beside the operands
+    const int     k = n0 + (lane & 15), n4 = m0 + 4 * (lane >> 4);
+    const int64_t i0 = y.w_off + (int64_t)n4 * y.din + k;
+    AdamState     old[4];
+    if (kUpdate)
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        if (k < y.din && n4 + r < y.dout) old[r] = adam_load(a.adam, i0 + (int64_t)r * y.din);
+    f32x4 sum{0.f, 0.f, 0.f, 0.f};
+    for (int z = 0; z < a.splits; z++) {
+      const int kb = z * a.k_chunk, ke = (int)min(a.Bp, (int64_t)kb + a.k_chunk);
+      f32x4     acc{0.f, 0.f, 0.f, 0.f};
+      constexpr int kFlight = 16;  // steps whose loads are in flight together
+      for (int k0 = kb; k0 < ke; k0 += kFlight * kKStep) {
+        bf16x8 d[kFlight], h[kFlight];
+#pragma unroll
+        for (int s = 0; s < kFlight; s++) {
+          const int k = min(k0 + s * kKStep, ke - kKStep);
+          d[s]        = pd[2 * k];
+          h[s]        = ph[2 * k];
+        }
+#pragma unroll
+        for (int s = 0; s < kFlight; s++)
+          if (k0 + s * kKStep < ke) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d[s], h[s], acc, 0, 0, 0);
+      }
+      if (a.splits == 1)
+        sum = acc;
+      else
+#pragma unroll
+        for (int r = 0; r < 4; r++) sum[r] += acc[r];
+    }
+    if (k >= y.din) return;
+    bf16x4 v;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const int64_t i = i0 + (int64_t)r * y.din;
+      v[r]            = (bf16)0.0f;
+      if (n4 + r >= y.dout) continue;
+      if (kUpdate) {
+        v[r]                               = adam_update(a.adam, i, old[r], sum[r]);
+        y.wf[operand_index(n4 + r, k, y.kp / kKStep)] = v[r];
+      } else {
+        a.g[i] = sum[r];
+      }
+    }
+    if (kUpdate) *reinterpret_cast<bf16x4*>(y.wt + operand_index(k, n4, y.np / kKStep)) = v;
+    return;
+  }
+  // bias columns, as bias_grad_columns sums them
+  int n = 4 * w + wave;
+#pragma unroll
+  for (int l = 0; l < kRowLayers; l++) {
+    if (l >= a.layers) break;
+    const RowLayer& y = a.l[l];
+    if (n >= y.dout) {
+      n -= y.dout;
+      continue;
+    }
+    float s = 0.0f;
+    for (int64_t b = lane; b < a.B; b += 64) s += y.gt[b * y.np + n];
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) s += __shfl_down(s, m, 64);
+    if (lane == 0) {
+      if (kUpdate)
+        adam_update(a.adam, y.b_off + n, adam_load(a.adam, y.b_off + n), s);
+      else
+        a.g[y.b_off + n] = s;
+    }
+    return;
+  }
+}
+
+// BF16 weights W [dout][din] into the padded copies
+__global__ __launch_bounds__(256) void k_pack(const bf16* __restrict__ W, RowLayer y)
+{
+  const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (i >= y.din * y.dout) return;
+  const int  n = i / y.din, k = i % y.din;
+  const bf16 v = W[i];
+  y.wf[operand_index(n, k, y.kp / kKStep)] = v;
+  y.wt[operand_index(k, n, y.np / kKStep)] = v;
 }
 
 inline unsigned blocks_of(int64_t n, int per) { return (unsigned)((n + per - 1) / per); }
@@ -393,9 +763,22 @@ struct nsm_mlp {
   float*               t32 = nullptr;  // targets [cap][d_L]
   double*              loss = nullptr; // [loss_cap]
   int64_t              loss_cap = 0;
-  double*              loss_part = nullptr;  // [min(loss_cap, kLossChunk)][kMseBlocks]
+  double*              loss_part = nullptr;  // [min(passes, kLossChunk)][partials per pass]
+  int64_t              loss_part_cap = 0;
   float*               split = nullptr;      // split-K partial products
   int64_t              split_cap = 0;
+
+  // small networks (k_rows, k_weights): padded BF16 weights, transposed
+  // activations and gradients of a batch of row_cap rows
+  bool                  rows = false;
+  std::vector<RowLayer> row;
+  bf16*                 row_weights = nullptr;
+  bool                  row_stale   = false;  // pb is newer than the padded copies
+  char*                 row_batch   = nullptr;
+  int64_t               row_cap     = 0;
+  float*                y32         = nullptr;  // output [y_cap][d_L] of k_rows' forward pass
+  int64_t               y_cap       = 0;
+  int64_t               x_cap = 0, t_cap = 0;   // rows of x32, t32
 
   int L() const { return (int)width.size() - 1; }
   int max_width() const { return *std::max_element(width.begin(), width.end()); }
@@ -453,16 +836,26 @@ void free_batch(nsm_mlp* net)
   for (auto* q : net->h) (void)hipFree(q);
   net->z.clear();
   net->h.clear();
-  for (void* q : {(void*)net->gf, (void*)net->gb, (void*)net->gf2, (void*)net->gb2, (void*)net->x32,
-                  (void*)net->t32})
+  for (void* q : {(void*)net->gf, (void*)net->gb, (void*)net->gf2, (void*)net->gb2})
     if (q) (void)hipFree(q);
   net->gf = nullptr;
   net->gb = nullptr;
   net->gf2 = nullptr;
   net->gb2 = nullptr;
-  net->x32 = nullptr;
-  net->t32 = nullptr;
   net->cap = 0;
+}
+
+// `*buf` of at least rows * width values
+template <typename T>
+int ensure_rows(T** buf, int64_t* cap, int64_t rows, int64_t width)
+{
+  if (rows <= *cap) return NSM_OK;
+  if (*buf) MLP_HIP(hipFree(*buf));
+  *buf = nullptr;
+  *cap = 0;
+  MLP_HIP(hipMalloc((void**)buf, (size_t)(rows * width) * sizeof(T)));
+  *cap = rows;
+  return NSM_OK;
 }
 
 int ensure_batch(nsm_mlp* net, int64_t B)
@@ -481,8 +874,6 @@ int ensure_batch(nsm_mlp* net, int64_t B)
   MLP_HIP(hipMalloc((void**)&net->gb, (size_t)(B * mw) * sizeof(bf16)));
   MLP_HIP(hipMalloc((void**)&net->gf2, (size_t)(B * mw) * sizeof(float)));
   MLP_HIP(hipMalloc((void**)&net->gb2, (size_t)(B * mw) * sizeof(bf16)));
-  MLP_HIP(hipMalloc((void**)&net->x32, (size_t)(B * net->width[0]) * sizeof(float)));
-  MLP_HIP(hipMalloc((void**)&net->t32, (size_t)(B * net->width[(size_t)L]) * sizeof(float)));
   net->cap = B;
   return NSM_OK;
 }
@@ -603,6 +994,162 @@ int backward(nsm_mlp* net, int64_t B, double* partial)
   return NSM_OK;
 }
 
+// ---- small networks: k_rows and k_weights
+// Training batches up to kRowBatch rows, the largest measured (205 us per
+// iteration against 693); longer ones, and other networks, run layer by layer.
+constexpr int64_t kRowBatch = 16384;
+
+bool fits_rows(const std::vector<int>& width)
+{
+  return (int)width.size() - 1 <= kRowLayers && *std::max_element(width.begin(), width.end()) <= kRowWidth;
+}
+
+// padded weights (zeroed once: the padding is never written)
+int create_rows(nsm_mlp* net)
+{
+  int64_t total = 0;
+  net->row.resize((size_t)net->L());
+  for (int l = 0; l < net->L(); l++) {
+    RowLayer& y = net->row[(size_t)l];
+    y           = RowLayer{};
+    y.din       = net->width[(size_t)l];
+    y.dout      = net->width[(size_t)l + 1];
+    y.kp        = (y.din + 31) / 32 * 32;
+    y.np        = (y.dout + 31) / 32 * 32;
+    y.w_off     = net->w_off[(size_t)l];
+    y.b_off     = net->b_off[(size_t)l];
+    y.bias      = net->p + y.b_off;
+    total += 2 * (int64_t)y.kp * y.np;
+  }
+  MLP_HIP(hipMalloc((void**)&net->row_weights, (size_t)total * sizeof(bf16)));
+  MLP_HIP(hipMemsetAsync(net->row_weights, 0, (size_t)total * sizeof(bf16), net->stream));
+  bf16* q = net->row_weights;
+  for (RowLayer& y : net->row) {
+    y.wf = q;
+    y.wt = q + (int64_t)y.kp * y.np;
+    q += 2 * (int64_t)y.kp * y.np;
+  }
+  net->rows      = true;
+  net->row_stale = true;
+  return NSM_OK;
+}
+
+int pack_rows(nsm_mlp* net)
+{
+  if (!net->row_stale) return NSM_OK;
+  for (const RowLayer& y : net->row) {
+    hipLaunchKernelGGL(k_pack, dim3(blocks_of((int64_t)y.din * y.dout, 256)), dim3(256), 0, net->stream,
+                       net->pb + y.w_off, y);
+    MLP_LAUNCHED();
+  }
+  net->row_stale = false;
+  return NSM_OK;
+}
+
+template <int kPer, int kRT, bool kTrain>
+int launch_rows(nsm_mlp* net, const RowArgs& a, int64_t rows)
+{
+  const dim3 g(blocks_of(rows, 4 * kPer * kRT)), b(kRowThreads);
+  switch (net->L()) {
+    case 1: hipLaunchKernelGGL((k_rows<1, kPer, kRT, kTrain>), g, b, 0, net->stream, a); break;
+    case 2: hipLaunchKernelGGL((k_rows<2, kPer, kRT, kTrain>), g, b, 0, net->stream, a); break;
+    case 3: hipLaunchKernelGGL((k_rows<3, kPer, kRT, kTrain>), g, b, 0, net->stream, a); break;
+    default: hipLaunchKernelGGL((k_rows<4, kPer, kRT, kTrain>), g, b, 0, net->stream, a);
+  }
+  MLP_LAUNCHED();
+  return NSM_OK;
+}
+
+// forward pass of the B rows in x32 into y32
+int forward_rows(nsm_mlp* net, int64_t B)
+{
+  int st = pack_rows(net);
+  if (st || (st = ensure_rows(&net->y32, &net->y_cap, B, net->width.back()))) return st;
+  RowArgs a{};
+  a.B = a.Bp = B;
+  a.x = net->x32;
+  a.y = net->y32;
+  std::copy(net->row.begin(), net->row.end(), a.l);
+  // 4, 16 or 32 rows per workgroup: few while that spreads the call over more
+  // CUs, many to share the weight loads once every CU has a workgroup
+  if (B <= 1024) return launch_rows<1, 1, false>(net, a, B);
+  return B <= 4096 ? launch_rows<4, 1, false>(net, a, B) : launch_rows<4, 2, false>(net, a, B);
+}
+
+// Rows per workgroup of a training pass: 4 while that leaves at most one
+// workgroup per CU of 256 (a workgroup's time is its chain of products and
+// hardly depends on its rows), then 8, then 16.
+int train_group(int64_t B) { return B <= 1024 ? 4 : B <= 2048 ? 8 : 16; }
+
+int64_t row_partials(int64_t B) { return (B + 31) / 32 * 32 / train_group(B); }
+
+// One pass over the B rows in x32, t32: squared-error partials
+// (row_partials(B) of them) and gradients, which go to net->g, or through
+// Adam when `adam` is given.
+int train_rows(nsm_mlp* net, int64_t B, double* partial, const Adam* adam)
+{
+  int st = pack_rows(net);
+  if (st) return st;
+  const int64_t Bp = (B + 31) / 32 * 32;
+  if (Bp > net->row_cap) {
+    int64_t per_row = 0;  // bytes
+    for (const RowLayer& y : net->row) per_row += 2 * y.kp + 6 * y.np;
+    if (net->row_batch) MLP_HIP(hipFree(net->row_batch));
+    net->row_batch = nullptr;
+    net->row_cap   = 0;
+    MLP_HIP(hipMalloc((void**)&net->row_batch, (size_t)(per_row * Bp)));
+    net->row_cap = Bp;
+  }
+  char* q = net->row_batch;  // every array a multiple of 64 bytes
+  for (RowLayer& y : net->row) {
+    y.ht = (bf16*)q, q += 2 * y.kp * Bp;
+    y.dt = (bf16*)q, q += 2 * y.np * Bp;
+    y.gt = (float*)q, q += 4 * y.np * Bp;
+  }
+  RowArgs a{};
+  a.B       = B;
+  a.Bp      = Bp;
+  a.x       = net->x32;
+  a.target  = net->t32;
+  a.partial = partial;
+  a.scale   = 2.0f / (float)(B * net->width.back());
+  std::copy(net->row.begin(), net->row.end(), a.l);
+  switch (train_group(B)) {
+    case 4: st = launch_rows<1, 1, true>(net, a, Bp); break;
+    case 8: st = launch_rows<2, 1, true>(net, a, Bp); break;
+    default: st = launch_rows<4, 1, true>(net, a, Bp);
+  }
+  if (st) return st;
+
+  WeightArgs w{};
+  w.layers = net->L();
+  w.B      = B;
+  w.Bp     = Bp;
+  GemmArgs split{};
+  split.K   = (int)B;
+  w.splits  = prepare(split, B <= kSplitAbove ? 1 : (int)std::min<int64_t>(kMaxSplits, (B + kSplitAbove - 1) / kSplitAbove));
+  w.k_chunk = split.k_chunk;
+  w.g       = net->g;
+  unsigned grid = 0;
+  int      cols = 0;
+  for (int l = 0; l < net->L(); l++) {
+    w.l[l]       = net->row[(size_t)l];
+    w.tiles_x[l] = w.l[l].kp / 32;
+    w.tiles[l]   = w.tiles_x[l] * (w.l[l].np / 32);
+    grid += (unsigned)w.tiles[l];
+    cols += w.l[l].dout;
+  }
+  grid += blocks_of(cols, 4);
+  if (adam) {
+    w.adam = *adam;
+    hipLaunchKernelGGL(k_weights<true>, dim3(grid), dim3(256), 0, net->stream, w);
+  } else {
+    hipLaunchKernelGGL(k_weights<false>, dim3(grid), dim3(256), 0, net->stream, w);
+  }
+  MLP_LAUNCHED();
+  return NSM_OK;
+}
+
 uint64_t splitmix(uint64_t& s)
 {
   uint64_t z = (s += 0x9E3779B97F4A7C15ULL);
@@ -618,6 +1165,7 @@ int upload_params(nsm_mlp* net, const float* host)
   hipLaunchKernelGGL(k_to_bf16, dim3(blocks_of(net->num_params, 256)), dim3(256), 0, net->stream, net->p, net->pb,
                      net->num_params);
   MLP_LAUNCHED();
+  net->row_stale = true;
   MLP_HIP(hipMemsetAsync(net->m1, 0, (size_t)net->num_params * sizeof(float), net->stream));
   MLP_HIP(hipMemsetAsync(net->m2, 0, (size_t)net->num_params * sizeof(float), net->stream));
   net->adam_t = 0;
@@ -627,8 +1175,8 @@ int upload_params(nsm_mlp* net, const float* host)
 
 int load_rows(nsm_mlp* net, int64_t B, const float* x, const float* t)
 {
-  int st = ensure_batch(net, B);
-  if (st) return st;
+  int st = ensure_rows(&net->x32, &net->x_cap, B, net->width[0]);
+  if (st || (t && (st = ensure_rows(&net->t32, &net->t_cap, B, net->width.back())))) return st;
   MLP_HIP(hipMemcpyAsync(net->x32, x, (size_t)(B * net->width[0]) * sizeof(float), hipMemcpyHostToDevice,
                          net->stream));
   if (t)
@@ -641,21 +1189,13 @@ int load_rows(nsm_mlp* net, int64_t B, const float* x, const float* t)
 // and turned into losses by one k_mse_total launch per chunk
 constexpr int kLossChunk = 4096;
 
-// losses for `passes` forward/backward passes and partials for
+// losses for `passes` forward/backward passes and `per_pass` partials for
 // min(passes, kLossChunk) of them
-int ensure_loss(nsm_mlp* net, int64_t passes)
+int ensure_loss(nsm_mlp* net, int64_t passes, int64_t per_pass)
 {
-  if (passes <= net->loss_cap) return NSM_OK;
-  if (net->loss) MLP_HIP(hipFree(net->loss));
-  if (net->loss_part) MLP_HIP(hipFree(net->loss_part));
-  net->loss      = nullptr;
-  net->loss_part = nullptr;
-  net->loss_cap  = 0;
-  MLP_HIP(hipMalloc((void**)&net->loss, (size_t)passes * sizeof(double)));
-  MLP_HIP(hipMalloc((void**)&net->loss_part,
-                    (size_t)(std::min<int64_t>(passes, kLossChunk) * kMseBlocks) * sizeof(double)));
-  net->loss_cap = passes;
-  return NSM_OK;
+  int st = ensure_rows(&net->loss, &net->loss_cap, passes, 1);
+  if (st) return st;
+  return ensure_rows(&net->loss_part, &net->loss_part_cap, std::min<int64_t>(passes, kLossChunk) * per_pass, 1);
 }
 
 }  // namespace
@@ -695,6 +1235,10 @@ int nsm_mlp_create(int num_layers, const int* widths, uint64_t seed, nsm_mlp** o
       hipMalloc((void**)&net->m2, n * 4) != hipSuccess ||
       hipMalloc((void**)&net->split, (size_t)net->split_cap * 4) != hipSuccess)
     return cleanup(fail(NSM_ERR_NOMEM, "device allocation of the parameters failed"));
+  if (fits_rows(net->width)) {
+    const int rst = create_rows(net);
+    if (rst) return cleanup(rst);
+  }
   // uniform(-a, a) weights with a = sqrt(6 / (fan_in + fan_out)), zero biases
   std::vector<float> init(n, 0.0f);
   uint64_t           s = seed;
@@ -718,7 +1262,8 @@ int nsm_mlp_destroy(nsm_mlp* net)
   if (net->stream) (void)hipStreamSynchronize(net->stream);
   free_batch(net);
   for (void* q : {(void*)net->p, (void*)net->pb, (void*)net->g, (void*)net->m1, (void*)net->m2, (void*)net->loss,
-                  (void*)net->loss_part, (void*)net->split})
+                  (void*)net->loss_part, (void*)net->split, (void*)net->x32, (void*)net->t32, (void*)net->y32,
+                  (void*)net->row_weights, (void*)net->row_batch})
     if (q) (void)hipFree(q);
   if (net->stream) (void)hipStreamDestroy(net->stream);
   delete net;
@@ -755,8 +1300,9 @@ int nsm_mlp_forward(nsm_mlp* net, int64_t batch, const float* x, float* y)
   if (batch == 0) return NSM_OK;
   MLP_HIP(hipSetDevice(net->device));
   int st = load_rows(net, batch, x, nullptr);
-  if (st || (st = forward(net, batch))) return st;
-  MLP_HIP(hipMemcpyAsync(y, net->z.back(), (size_t)(batch * net->width.back()) * sizeof(float),
+  if (st || (st = net->rows ? forward_rows(net, batch) : ensure_batch(net, batch))) return st;
+  if (!net->rows && (st = forward(net, batch))) return st;
+  MLP_HIP(hipMemcpyAsync(y, net->rows ? net->y32 : net->z.back(), (size_t)(batch * net->width.back()) * sizeof(float),
                          hipMemcpyDeviceToHost, net->stream));
   MLP_HIP(hipStreamSynchronize(net->stream));
   return NSM_OK;
@@ -770,9 +1316,15 @@ int nsm_mlp_loss_gradients(nsm_mlp* net, int64_t batch, const float* x, const fl
   int st = load_rows(net, batch, x, t);
   if (st) return st;
   const int64_t n = batch * net->width.back();
-  if ((st = ensure_loss(net, 1)) || (st = forward(net, batch)) || (st = backward(net, batch, net->loss_part)))
-    return st;
-  hipLaunchKernelGGL(k_mse_total, dim3(1), dim3(64), 0, net->stream, net->loss_part, n, net->loss);
+  const bool    rows     = net->rows && batch <= kRowBatch;
+  const int64_t per_pass = rows ? row_partials(batch) : kMseBlocks;
+  if ((st = ensure_loss(net, 1, per_pass))) return st;
+  if (rows)
+    st = train_rows(net, batch, net->loss_part, nullptr);
+  else if (!(st = ensure_batch(net, batch)) && !(st = forward(net, batch)))
+    st = backward(net, batch, net->loss_part);
+  if (st) return st;
+  hipLaunchKernelGGL(k_mse_total, dim3(1), dim3(64), 0, net->stream, net->loss_part, (int)per_pass, n, net->loss);
   MLP_LAUNCHED();
   MLP_HIP(hipMemcpyAsync(loss, net->loss, sizeof(double), hipMemcpyDeviceToHost, net->stream));
   MLP_HIP(hipMemcpyAsync(grad, net->g, (size_t)net->num_params * sizeof(float), hipMemcpyDeviceToHost,
@@ -790,7 +1342,10 @@ int nsm_mlp_train(nsm_mlp* net, int64_t batch, const float* x, const float* t, i
   MLP_HIP(hipSetDevice(net->device));
   int st = load_rows(net, batch, x, t);
   if (st) return st;
-  if ((st = ensure_loss(net, iterations))) return st;
+  const bool    rows     = net->rows && batch <= kRowBatch;
+  const int64_t per_pass = rows ? row_partials(batch) : kMseBlocks;
+  if ((st = ensure_loss(net, iterations, per_pass))) return st;
+  if (!rows && (st = ensure_batch(net, batch))) return st;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int it = 0; it < iterations; it++) {
     // cosine decay from lr to lr_final
@@ -799,17 +1354,22 @@ int nsm_mlp_train(nsm_mlp* net, int64_t batch, const float* x, const float* t, i
     net->adam_t++;
     const float c1 = (float)(1.0 - std::pow((double)b1, (double)net->adam_t));
     const float c2 = (float)(1.0 - std::pow((double)b2, (double)net->adam_t));
-    if ((st = forward(net, batch, it == 0)) ||
-        (st = backward(net, batch, net->loss_part + (int64_t)(it % kLossChunk) * kMseBlocks)))
-      return st;
-    hipLaunchKernelGGL(k_adam, dim3(blocks_of(net->num_params, 256)), dim3(256), 0, net->stream, net->p, net->g,
-                       net->m1, net->m2, net->pb, net->num_params, lri, b1, b2, c1, c2, eps);
-    MLP_LAUNCHED();
+    const Adam    adam{net->p, net->m1, net->m2, net->pb, lri, b1, b2, c1, c2, eps};
+    double* const partial = net->loss_part + (int64_t)(it % kLossChunk) * per_pass;
+    if (rows) {
+      if ((st = train_rows(net, batch, partial, &adam))) return st;
+    } else {
+      if ((st = forward(net, batch, it == 0)) || (st = backward(net, batch, partial))) return st;
+      hipLaunchKernelGGL(k_adam, dim3(blocks_of(net->num_params, 256)), dim3(256), 0, net->stream, adam, net->g,
+                         net->num_params);
+      MLP_LAUNCHED();
+      net->row_stale = true;
+    }
     // the losses of a full chunk of iterations (or of the last one)
     if ((it + 1) % kLossChunk == 0 || it + 1 == iterations) {
       const int first = it - it % kLossChunk;
       hipLaunchKernelGGL(k_mse_total, dim3((unsigned)(it + 1 - first)), dim3(64), 0, net->stream, net->loss_part,
-                         batch * net->width.back(), net->loss + first);
+                         (int)per_pass, batch * net->width.back(), net->loss + first);
       MLP_LAUNCHED();
     }
   }

@@ -158,3 +158,39 @@ def test_loss_history_across_calls_and_chunks(hip_device):
     assert np.array_equal(a.get_parameters(), b.get_parameters())
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("widths,B", [((5, 33), 1), ((4, 256, 31), 1025), ((3, 32, 256, 7), 2049),
+                                      ((33, 256, 16, 224, 64), 31)])
+def test_small_networks_at_the_edges(hip_device, widths, B):
+    """One to four layers, widths around multiples of 32 and at the widest
+    the row kernels take, batches on both sides of their rows per workgroup:
+    outputs, loss and gradients against the oracle (tolerances as above)."""
+    net = MLP(widths, seed=11)
+    x, t = data(widths, B, 12)
+    p = net.get_parameters().astype(np.float64)
+    y = net.forward(x).astype(np.float64)
+    y16, _ = M.forward(p, widths, x, bf16=True)
+    assert np.linalg.norm(y - y16) / np.linalg.norm(y16) <= (2e-5 if len(widths) == 2 else 2e-3)
+    loss, g = net.loss_gradients(x, t)
+    rl, rg = M.loss_and_grad(p, widths, x, t, bf16=True)
+    assert abs(loss - rl) <= 1e-3 * rl
+    assert np.linalg.norm(g - rg) / np.linalg.norm(rg) <= (2e-5 if len(widths) == 2 else 5e-3)
+    net.close()
+
+
+@pytest.mark.parametrize("B", [96, 16385])  # row kernels; layer by layer
+def test_forward_sees_trained_parameters(hip_device, B):
+    """After training on either path a forward pass uses the new parameters:
+    the same outputs as a network that was given them."""
+    widths = (4, 48, 40)
+    a, b = MLP(widths, seed=1), MLP(widths, seed=2)
+    x, t = data(widths, B, 3)
+    before = a.forward(x[:50])
+    a.train(x, t, 3, 1e-2, 1e-2)
+    b.set_parameters(a.get_parameters())
+    y = a.forward(x[:50])
+    assert not np.array_equal(y, before)
+    assert np.array_equal(y, b.forward(x[:50]))
+    a.close()
+    b.close()
