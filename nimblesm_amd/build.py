@@ -40,6 +40,7 @@ SOURCES = {
     "nsm_model.cpp": ["-ffp-contract=off", "-x", "hip"],
     "nsm_ensemble.cpp": ["-ffp-contract=off", "-x", "hip"],
     "nsm_autotune.cpp": [],
+    "nsm_host_copy.cpp": ["-x", "hip"],
     # surrogate network: BF16 matrix-core GEMMs, FP32 epilogues and Adam
     "nsm_mlp.hip": ["-ffp-contract=fast-honor-pragmas"],
 }

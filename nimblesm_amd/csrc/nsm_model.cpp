@@ -24,6 +24,7 @@
 
 #include "../../include/nimblesm_amd.h"
 #include "nsm_autotune.h"
+#include "nsm_host_copy.h"
 #include "nsm_kernels.h"
 #include "nsm_node_step.h"
 #include "nsm_tiled.h"
@@ -847,9 +848,7 @@ int ip_field_out(nsm_model* md, const void* src, int nc, double* out)
     const int64_t n = std::min(chunk, E - e0);
     nsm::launch_ip_gather(src, L, e0, n, md->d_stage, md->stream);
     NSM_LAUNCHED();
-    NSM_HIP(hipMemcpyAsync(out + e0 * per, md->d_stage, (size_t)(n * per) * sizeof(double), hipMemcpyDeviceToHost,
-                           md->stream));
-    NSM_HIP(hipStreamSynchronize(md->stream));
+    NSM_HIP(nsm::device_to_host(md->device, md->stream, out + e0 * per, md->d_stage, (size_t)(n * per)));
   }
   return NSM_OK;
 }
@@ -866,8 +865,7 @@ int node_field_out(nsm_model* md, const double* src, size_t w, double* out)
     NSM_LAUNCHED();
     src = md->d_stage;
   }
-  NSM_HIP(hipMemcpyAsync(out, src, cnt * sizeof(double), hipMemcpyDeviceToHost, md->stream));
-  NSM_HIP(hipStreamSynchronize(md->stream));
+  NSM_HIP(nsm::device_to_host(md->device, md->stream, out, src, cnt));
   return NSM_OK;
 }
 
@@ -1074,6 +1072,7 @@ int model_create(int64_t num_nodes, const double* reference_coordinates, int num
       return fail(NSM_ERR_ARG, "connectivity entry %lld = %d out of range", (long long)k, conn[k]);
 
   nsm_model* md  = new nsm_model();
+  nsm::host_copy_hold();
   md->precision  = precision;
   md->N          = num_nodes;
   md->E          = E;
@@ -1254,6 +1253,7 @@ int nsm_model_destroy(nsm_model* md)
     (void)hipEventDestroy(p.stop);
   }
   if (md->stream) (void)hipStreamDestroy(md->stream);
+  nsm::host_copy_release();
   delete md;
   return NSM_OK;
 }

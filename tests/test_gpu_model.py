@@ -425,3 +425,33 @@ def test_inverted_element_in_model_reports_error_and_recovers(hip_device, monkey
     m.ComputeInternalForce()
     assert np.abs(m.GetVectorNodeData("internal_force")).max() < 1e-3  # undeformed: f ~ 0
     m.close()
+
+
+@pytest.mark.parametrize("num_nodes", [87381, 87382, 131072, 400001])
+def test_node_fields_of_every_copy_size(hip_device, num_nodes):
+    """Host copies around the 1 MB chunks of a staged copy (2 MB minus 8
+    bytes, just above, whole chunks, a last chunk of a few values), read from
+    two models on two threads at once: every value arrives."""
+    import threading
+
+    X = np.zeros((num_nodes, 3))
+    X[:8] = [[0, 0, 0], [1, 0, 0], [1, 1, 0], [0, 1, 0], [0, 0, 1], [1, 0, 1], [1, 1, 1], [0, 1, 1]]
+    block = N.Block(1, np.arange(8, dtype=np.int32)[None], N.NeohookeanMaterial(7800.0, 1.6e11, 0.8e11))
+    models = [N.ModelData(X, [block]) for _ in range(2)]
+    fields = [np.random.default_rng(k).normal(size=(num_nodes, 3)) for k in range(2)]
+    got = [[], []]
+
+    def read(k):
+        for _ in range(3):
+            got[k].append(models[k].GetVectorNodeData("velocity"))
+
+    for m, v in zip(models, fields):
+        m.SetVectorNodeData("velocity", v)
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for k in range(2):
+        assert len(got[k]) == 3 and all(np.array_equal(g, fields[k]) for g in got[k])
+        models[k].close()
