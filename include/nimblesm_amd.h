@@ -65,7 +65,9 @@ typedef enum nsm_kernel {
   NSM_KERNEL_NODE    = 1, /* CSR gather + central-difference node kernel
                              (tiled: update of nodes shared between tiles)     */
   NSM_KERNEL_REACTION = 2, /* reaction-force sum                                 */
-  NSM_KERNEL_CLOSURE  = 3  /* UQ closure + update of the approximate samples      */
+  NSM_KERNEL_CLOSURE  = 3  /* UQ closure + update of the approximate samples (tiled
+                             models with at most 8 exact samples: with the update
+                             of the nodes shared between tiles)                  */
 } nsm_kernel;
 
 const char* nsm_status_string(int status);

@@ -249,6 +249,13 @@ struct nsm_model {
   double*             uq_state    = nullptr;
   double*             uq_coeff    = nullptr;  // [uq_approx][uq_exact + 1]
   nsm::BcEntry*       uq_bc_table = nullptr;  // bc_table without prescribed displacements
+  // tiled models with at most kUqCachedExact exact samples: all trajectories
+  // in one element and one node launch per step.  Node arrays and moduli of
+  // the nominal trajectory and the exact samples, and the tile partials of
+  // each.
+  nsm::UqTrajectory*  uq_traj     = nullptr;  // [uq_exact + 1]
+  float*              uq_moduli   = nullptr;  // K, then G: [uq_exact + 1][num_blocks] each
+  float*              uq_partials = nullptr;  // [uq_exact + 1][partials][3]
 
   std::vector<BcRecord> bcs;
   std::vector<uint8_t>  reaction_mask;  // host copy of the reaction bit per node
@@ -694,6 +701,55 @@ int launch_trajectory(nsm_model* md, const nsm::StepArgs& sa, int64_t step, int6
   return st ? st : launch_node(md, sa, step, fold_step, pending, sample);
 }
 
+// The tiled step of the nominal trajectory and every exact UQ sample in one
+// element launch (per block group), then every trajectory's shared nodes and
+// the approximate samples in one node launch.
+int launch_uq_tiled(nsm_model* md, const nsm::StepArgs& sa, int64_t step, int64_t fold_step, int64_t* pending)
+{
+  nsm::ReactionArgs     rx;
+  const bool            want_rx = reaction_args(md, step, &rx);
+  const nsm::NodeArrays na      = md->node_arrays();
+  nsm::ReactionFold     fold    = reaction_fold(md, fold_step);
+  nsm::TileArgs         ta      = md->tile_args;
+  const int             T       = md->uq_exact + 1;
+  const int             np      = (int)md->tiles.bnd_ent.size();
+  ta.partials                   = md->uq_partials;
+  size_t           ti;
+  nsm::LaunchTimer timer;
+  int              st = NSM_OK;
+  for (int b0 = 0; b0 < md->num_blocks; b0 += nsm::kMaxLaunchBlocks) {
+    const int nb = std::min(nsm::kMaxLaunchBlocks, md->num_blocks - b0);
+    const int t0 = md->blk_tile_off[(size_t)b0], t1 = md->blk_tile_off[(size_t)(b0 + nb)];
+    if (t1 <= t0) continue;
+    if ((st = time_begin(md, NSM_KERNEL_ELEMENT, &ti, &timer))) return st;
+    const nsm::UqTileWork work{float_table(md, b0, nb, -1),
+                               b0,
+                               md->num_blocks,
+                               t0,
+                               t1 - t0,
+                               T * (t1 - t0),
+                               md->uq_traj,
+                               md->uq_moduli,
+                               md->uq_moduli + (size_t)T * (size_t)md->num_blocks,
+                               np,
+                               md->uq_bc_table,
+                               sa,
+                               fold};
+    nsm::launch_uq_element_tiled(work, ta, md->X, na, (float*)md->Fip, (float*)md->sip, rx, md->status, md->stream,
+                                 timer);
+    NSM_LAUNCHED();
+    if ((st = time_end(md, ti))) return st;
+    fold.n = 0;
+  }
+  if ((st = time_begin(md, md->uq_approx > 0 ? NSM_KERNEL_CLOSURE : NSM_KERNEL_NODE, &ti, &timer))) return st;
+  const nsm::UqClosure uc{md->uq_exact, md->uq_approx, 3 * md->N, md->f, md->uq_state, md->uq_coeff};
+  nsm::launch_uq_nodes(ta, na, md->uq_bc_table, uc, np, sa, rx, md->stream, timer);
+  NSM_LAUNCHED();
+  if ((st = time_end(md, ti))) return st;
+  *pending = want_rx ? step : -1;
+  return NSM_OK;
+}
+
 // Closure forces of the approximate UQ samples from this step's nominal and
 // exact forces, with their node update.
 int launch_closure(nsm_model* md, const nsm::StepArgs& sa)
@@ -707,13 +763,15 @@ int launch_closure(nsm_model* md, const nsm::StepArgs& sa)
   return time_end(md, ti);
 }
 
-// One step of every trajectory: exact UQ samples (their element launches
+// One step of every trajectory (tiled models with few exact samples:
+// launch_uq_tiled): exact UQ samples (their element launches
 // store no F or sigma), the nominal trajectory, then the closure of the
 // approximate samples, which reads this step's nominal and exact forces.
 // Samples are independent of each other and of the nominal trajectory until
 // the closure.
 int launch_step(nsm_model* md, const nsm::StepArgs& sa, int64_t step, int64_t fold_step, int64_t* pending)
 {
+  if (md->uq_traj) return launch_uq_tiled(md, sa, step, fold_step, pending);
   int     st     = NSM_OK;
   int64_t unused = -1;
   for (int k = 0; k < md->uq_exact; k++)
@@ -1246,6 +1304,9 @@ int nsm_model_destroy(nsm_model* md)
   free_dev(md->uq_state);
   free_dev(md->uq_coeff);
   free_dev(md->uq_bc_table);
+  free_dev(md->uq_traj);
+  free_dev(md->uq_moduli);
+  free_dev(md->uq_partials);
   free_dev(md->d_stage);
   for (void* p : md->tile_bufs) (void)hipFree(p);
   for (auto& p : md->event_pool) {
@@ -1696,11 +1757,17 @@ int nsm_model_set_uq_samples(nsm_model* md, int num_exact, const double* bulk_mo
   if (st) return st;
   NSM_HIP(hipStreamSynchronize(md->stream));
   const size_t state_doubles = 12 * (size_t)md->N * (size_t)(num_exact + num_approx);
+  const size_t np            = 3 * md->tiles.bnd_ent.size();  // partial values of one trajectory (tiled models)
+  const size_t old_traj      = md->uq_traj ? (size_t)(md->uq_exact + 1) : 0;
   const size_t old_bytes     = (12 * (size_t)md->N * (size_t)md->uq_samples() +
-                            (size_t)md->uq_approx * (size_t)(md->uq_exact + 1)) * sizeof(double);
+                            (size_t)md->uq_approx * (size_t)(md->uq_exact + 1)) * sizeof(double) +
+                           old_traj * (sizeof(nsm::UqTrajectory) + (2 * (size_t)md->num_blocks + np) * sizeof(float));
   free_dev(md->uq_state);
   free_dev(md->uq_coeff);
   free_dev(md->uq_bc_table);
+  free_dev(md->uq_traj);
+  free_dev(md->uq_moduli);
+  free_dev(md->uq_partials);
   md->device_bytes -= std::min(md->device_bytes, old_bytes);
   md->uq_exact = md->uq_approx = 0;
   md->uq_K.clear();
@@ -1717,6 +1784,36 @@ int nsm_model_set_uq_samples(nsm_model* md, int num_exact, const double* bulk_mo
   md->uq_G.assign(shear_modulus, shear_modulus + nk);
   md->uq_exact  = num_exact;
   md->uq_approx = num_approx;
+  if (md->tiled && num_exact <= nsm::kUqCachedExact && (num_exact + 1) * (int64_t)md->tiles.bnd_ent.size() < INT32_MAX &&
+      (num_exact + 1) * (int64_t)md->tiles.num_tiles < INT32_MAX) {
+    const size_t                   T = (size_t)num_exact + 1, nb = (size_t)md->num_blocks;
+    std::vector<nsm::UqTrajectory> traj(T);
+    std::vector<float>             moduli(2 * T * nb);
+    for (size_t s = 0; s < T; s++) {
+      const nsm::NodeArrays na = md->node_arrays((int)s - 1);
+      traj[s]                  = nsm::UqTrajectory{na.u, na.v, na.a, na.f};
+      for (size_t b = 0; b < nb; b++) {
+        moduli[s * nb + b]       = (float)md->bulk((int)s - 1, (int)b);
+        moduli[(T + s) * nb + b] = (float)md->shear((int)s - 1, (int)b);
+      }
+    }
+    nsm::UqTrajectory* d_traj = nullptr;
+    size_t             bytes  = 0;
+    if (dalloc(&md->uq_moduli, moduli.size(), &bytes) || dalloc(&md->uq_partials, std::max<size_t>(T * np, 1), &bytes) ||
+        dalloc(&d_traj, T, &bytes)) {
+      // no memory for the joint launches: one launch per trajectory
+      free_dev(md->uq_moduli);
+      free_dev(md->uq_partials);
+      (void)hipGetLastError();
+      return NSM_OK;
+    }
+    md->device_bytes += T * (sizeof(nsm::UqTrajectory) + (2 * nb + np) * sizeof(float));
+    md->uq_traj = d_traj;
+    NSM_HIP(hipMemcpyAsync(md->uq_moduli, moduli.data(), moduli.size() * sizeof(float), hipMemcpyHostToDevice,
+                           md->stream));
+    NSM_HIP(hipMemcpyAsync(d_traj, traj.data(), T * sizeof(nsm::UqTrajectory), hipMemcpyHostToDevice, md->stream));
+    NSM_HIP(hipStreamSynchronize(md->stream));
+  }
   return NSM_OK;
 }
 

@@ -69,6 +69,26 @@ struct EnsTileWork {
   EnsFold          fold;
 };
 
+// Off-nominal ensemble: the tiles [t_begin, t_begin + t_count) of the nominal
+// trajectory (s = 0) and of every exact sample (s >= 1) of one model in one
+// launch, work item i being tile t_begin + i % t_count of trajectory
+// i / t_count.  The samples keep no F or sigma and no reaction; block b of
+// trajectory s has moduli K, G[s num_blocks + b].
+struct UqTrajectory {
+  double *u, *v, *a, *f;
+};
+struct UqTileWork {
+  BlockTable<float>   bt;  // block boundaries
+  int                 first_block, num_blocks;
+  int                 t_begin, t_count, count;
+  const UqTrajectory* traj;
+  const float *       K, *G;
+  int                 num_partials;  // of one trajectory
+  const BcEntry*      sample_bc;     // the samples' conditions (the nominal ones are NodeArrays')
+  StepArgs            sa;
+  ReactionFold        fold;
+};
+
 // boundary nodes per workgroup of the boundary kernel (one per thread)
 constexpr int kBoundaryNodesPerGroup = 256;
 unsigned      boundary_grid(int num_bnd);
@@ -95,6 +115,17 @@ void launch_ens_element_tiled(const EnsTileWork& work, const TileArgs& ta, const
 // sample; reaction partial of group g at rx.partials[rx_base + g].
 void launch_ens_boundary_update(const TileArgs& ta, const EnsNodes& en, const EnsRange* groups, int num_groups,
                                 EnsStep es, ReactionArgs rx, int rx_base, hipStream_t s);
+// Every trajectory's tiles of an off-nominal ensemble; then the shared nodes
+// of every trajectory from their partials and, for every node, the closure
+// forces of the approximate samples (as launch_uq_closure) with their update.
+void launch_uq_element_tiled(const UqTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,
+                             float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s,
+                             const LaunchTimer& timer = LaunchTimer{});
+// na: the nominal trajectory; exact samples k at uc.state as in UqClosure
+constexpr int kUqCachedExact = 8;  // most exact samples these launches take
+void launch_uq_nodes(const TileArgs& ta, const NodeArrays& na, const BcEntry* sample_bc, const UqClosure& uc,
+                     int num_partials, const StepArgs& sa, ReactionArgs rx, hipStream_t s,
+                     const LaunchTimer& timer = LaunchTimer{});
 // Element-kernel workgroups one CU holds at once (occupancy).
 int element_tiled_groups_per_cu(int tile_elems);
 // Step of the remaining nodes from their partials (ascending tile order).

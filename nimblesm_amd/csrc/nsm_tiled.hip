@@ -191,8 +191,10 @@ __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const dou
 // ---- the two kinds of element-launch work (nsm_tiled.h) ----
 __device__ __forceinline__ int work_count(const ModelTileWork& w) { return w.t_count; }
 __device__ __forceinline__ int work_count(const EnsTileWork& w) { return w.count; }
+__device__ __forceinline__ int work_count(const UqTileWork& w) { return w.count; }
 __device__ __forceinline__ int work_update_v(const ModelTileWork& w) { return w.sa.update_v; }
 __device__ __forceinline__ int work_update_v(const EnsTileWork& w) { return w.es.update_v; }
+__device__ __forceinline__ int work_update_v(const UqTileWork& w) { return w.sa.update_v; }
 
 __device__ __forceinline__ TileCtx tile_ctx(const ModelTileWork& w, int i)
 {
@@ -206,7 +208,49 @@ __device__ __forceinline__ TileCtx tile_ctx(const EnsTileWork& w, int i)
                  uniform(sm.partial_base), uniform(sm.bc_base), uniform(sm.kg_base)};
 }
 
+__device__ __forceinline__ TileCtx tile_ctx(const UqTileWork& w, int i)
+{
+  int s = 0;
+  for (; i >= w.t_count; i -= w.t_count) s++;  // a few trajectories
+  return TileCtx{w.t_begin + i, s, 0, 0, s * w.num_partials, 0, s * w.num_blocks + w.first_block};
+}
+
+// Node arrays of the item's trajectory
+template <typename Work>
+__device__ __forceinline__ NodeArrays work_arrays(const Work&, const TileCtx&, const NodeArrays& na)
+{
+  return na;
+}
+__device__ __forceinline__ NodeArrays work_arrays(const UqTileWork& w, const TileCtx& c, const NodeArrays& na)
+{
+  const UqTrajectory t = ens_load(w.traj, (int64_t)c.s);
+  NodeArrays         r = na;
+  r.u                  = t.u;
+  r.v                  = t.v;
+  r.a                  = t.a;
+  r.f                  = t.f;
+  return r;
+}
+// its kinematic conditions (not ensembles, whose items carry their own)
+template <typename Work>
+__device__ __forceinline__ const BcEntry* item_bc(const Work&, const TileCtx&, const NodeArrays& na)
+{
+  return na.bc_table;
+}
+__device__ __forceinline__ const BcEntry* item_bc(const UqTileWork& w, const TileCtx& c, const NodeArrays& na)
+{
+  return c.s > 0 ? w.sample_bc : na.bc_table;
+}
+// whether the item stores F and sigma and sums a reaction
+template <typename Work>
+__device__ __forceinline__ bool item_output(const Work&, const TileCtx&)
+{
+  return true;
+}
+__device__ __forceinline__ bool item_output(const UqTileWork&, const TileCtx& c) { return c.s == 0; }
+
 __device__ __forceinline__ const BcEntry* work_bc(const ModelTileWork&) { return nullptr; }
+__device__ __forceinline__ const BcEntry* work_bc(const UqTileWork&) { return nullptr; }
 __device__ __forceinline__ const BcEntry* work_bc(const EnsTileWork& w) { return w.bc; }
 
 // moduli of the tile's block (tiles never straddle blocks)
@@ -223,7 +267,15 @@ __device__ __forceinline__ void tile_moduli(const EnsTileWork& w, const TileCtx&
   G           = tile_table(w.G, b);
 }
 
+__device__ __forceinline__ void tile_moduli(const UqTileWork& w, const TileCtx& c, int e0, float& K, float& G)
+{
+  const int b = c.kg_base + uniform(block_of(w.bt, (int64_t)e0));
+  K           = tile_table(w.K, b);
+  G           = tile_table(w.G, b);
+}
+
 __device__ __forceinline__ StepArgs tile_step(const ModelTileWork& w, const TileCtx&) { return w.sa; }
+__device__ __forceinline__ StepArgs tile_step(const UqTileWork& w, const TileCtx&) { return w.sa; }
 __device__ __forceinline__ StepArgs tile_step(const EnsTileWork& w, const TileCtx& c)
 {
   return ens_step_args(w.es, c.s);
@@ -231,12 +283,13 @@ __device__ __forceinline__ StepArgs tile_step(const EnsTileWork& w, const TileCt
 
 // index of the tile's reaction partial
 __device__ __forceinline__ int tile_rx_slot(const ModelTileWork&, const TileCtx& c, int) { return c.t; }
+__device__ __forceinline__ int tile_rx_slot(const UqTileWork&, const TileCtx& c, int) { return c.t; }
 __device__ __forceinline__ int tile_rx_slot(const EnsTileWork&, const TileCtx&, int i) { return i; }
 
 // A previous step's reaction total(s): workgroup 0 sums the model's
 // partials; in an ensemble every wave of the launch takes samples in turn.
-template <int kThreads>
-__device__ __forceinline__ void fold_previous(const ModelTileWork& w, double* fold_red)
+template <int kThreads, typename Work>
+__device__ __forceinline__ void fold_previous(const Work& w, double* fold_red)
 {
   if (w.fold.n > 0 && blockIdx.x == 0) {  // uniform
     const double total = reaction_total<kThreads>(w.fold.partials, w.fold.tiles, w.fold.n, fold_red);
@@ -280,6 +333,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
 {
   constexpr int  kNodes      = 2 * kThreads;
   constexpr bool kEnsemble   = std::is_same<Work, EnsTileWork>::value;
+  constexpr bool kUq         = std::is_same<Work, UqTileWork>::value;
   // ensembles stage each tile's sample's kinematic-condition entries (one
   // 8-byte word per thread)
   constexpr int  kTileBcWords = kBcWords * kEnsMaxBcCodes;
@@ -315,7 +369,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
   if (tid == 0) bad = 0;
   TileCtx c_first = tile_ctx(work, ib);
   if (!kEnsemble && update_v)
-    for (int b = tid; b < na.num_bc; b += kThreads) sbc[b] = na.bc_table[b];
+    for (int b = tid; b < na.num_bc; b += kThreads) sbc[b] = item_bc(work, c_first, na)[b];
   if (kEnsemble && tid < kTileBcWords)
     reinterpret_cast<uint64_t*>(sbc)[tid] =
         reinterpret_cast<const uint64_t*>(work_bc(work) + c_first.bc_base)[tid];
@@ -325,11 +379,12 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
 #pragma unroll
   for (int k = 0; k < 2; k++) {
     load3(X, ids.gid[k] + c_first.x_delta, xr[k]);
-    load3(na.u, ids.gid[k], ur[k]);
+    load3(work_arrays(work, c_first, na).u, ids.gid[k], ur[k]);
   }
   ElemData  cur = load_elem<kThreads>(ta, c_first.t);
   NodeState ns;
-  stage<kThreads>(ids, c_first.x_delta, xr, ur, na, update_v, sxu, as, tile_table(ta.gather, c_first.t) != 0, ns);
+  stage<kThreads>(ids, c_first.x_delta, xr, ur, work_arrays(work, c_first, na), update_v, sxu, as,
+                  tile_table(ta.gather, c_first.t) != 0, ns);
   // every prologue load complete (vmcnt(0); lgkmcnt and expcnt at their
   // maximum, gfx9 encoding): the loop's waits then depend on its body only
   __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -349,7 +404,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       load3(X, ids_next.gid[k] + cn.x_delta, xr[k]);
-      load3(na.u, ids_next.gid[k], ur[k]);
+      load3(work_arrays(work, cn, na).u, ids_next.gid[k], ur[k]);
     }
     const ElemData el_next   = load_elem<kThreads>(ta, cn.t);
     const SlotIds  ids_after = load_ids<kThreads>(ta, tile_ctx(work, next(next(i))));
@@ -388,8 +443,11 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       // (the step never reads them back) keep node data and partials in cache
       float* const Ft   = kStoreIp ? Fip + (int64_t)e0 * 72 : nullptr;
       float* const St   = kStoreIp ? sip + (int64_t)e0 * 48 : nullptr;
-      const auto   rF   = tile_rsrc(Ft, 72 * 4 * ntl);
-      const auto   rS   = tile_rsrc(St, 48 * 4 * ntl);
+      // an item without element data has blocks of no bytes: its stores are
+      // dropped by the range check
+      const int    nst  = item_output(work, c) ? ntl : 0;
+      const auto   rF   = tile_rsrc(Ft, 72 * 4 * nst);
+      const auto   rS   = tile_rsrc(St, 48 * 4 * nst);
       const int    loff = 8 * lcl;
       auto store = [&](int qm, int qp, const float* Fm, const float* Sm, const float* Fp, const float* Sp) {
         const bool   m_even = qm < qp;  // qm, qp: constants after inlining
@@ -456,8 +514,9 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     }
 
     // ---- interior nodes: complete step; others: this tile's partial
-    const StepArgs sa  = tile_step(work, c);
-    double         rxs = 0.0;
+    const StepArgs   sa  = tile_step(work, c);
+    const NodeArrays nac = work_arrays(work, c, na);
+    double           rxs = 0.0;
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const int ln = tid + k * kThreads;
@@ -482,7 +541,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       if (ids.dst[k] == kInterior) {
         if (rx.coord >= 0 && (ns.flg[k] & kReactionFlag)) rxs += fn[rx.coord];
         double un[3] = {sxu[ln][3], sxu[ln][4], sxu[ln][5]};
-        node_update(na, sbc, ids.gid[k], ns.flg[k], fn, un, ns.v[k], ns.m[k], sa);
+        node_update(nac, sbc, ids.gid[k], ns.flg[k], fn, un, ns.v[k], ns.m[k], sa);
       } else {
         float* const pp = ta.partials + 3 * (int64_t)ids.dst[k];
         pp[0]           = (float)fn[0];
@@ -490,7 +549,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
         pp[2]           = (float)fn[2];
       }
     }
-    if (rx.coord >= 0) {  // uniform across the grid
+    if (rx.coord >= 0 && item_output(work, c)) {  // uniform across the workgroup
       const double s = block_sum<kThreads>(rxs, red);
       if (threadIdx.x == 0) rx.partials[tile_rx_slot(work, c, i)] = s;
     }
@@ -502,7 +561,10 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     cur      = el_next;
     if (i + G < ie) {
       if (kEnsemble && tid < kTileBcWords) reinterpret_cast<uint64_t*>(sbc)[tid] = bc_next;
-      stage<kThreads>(ids, cn.x_delta, xr, ur, na, update_v, sxu, as, tile_table(ta.gather, cn.t) != 0, ns);
+      if (kUq && update_v && (c.s > 0) != (cn.s > 0))  // the next item's conditions (once per launch)
+        for (int b = tid; b < na.num_bc; b += kThreads) sbc[b] = item_bc(work, cn, na)[b];
+      stage<kThreads>(ids, cn.x_delta, xr, ur, work_arrays(work, cn, na), update_v, sxu, as,
+                      tile_table(ta.gather, cn.t) != 0, ns);
     }
   }
   if (tid == 0 && bad) atomicOr(status, 1);
@@ -510,9 +572,51 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
 
 constexpr int kBndThreads = kBoundaryNodesPerGroup;
 
-// Boundary node bi (partials [p0, p1)) at row i, flags at row xi: sums its
-// partials in ascending tile order from 0.0 in FP64, then the node update.
-// Returns its reaction contribution.
+// Force of a boundary node: its partials [p0, p1) in ascending tile order
+// from 0.0 in FP64.  Up to 8 partials are loaded at once, then added in
+// ascending order (the same order as one at a time); more than 8 continue
+// one by one.
+__device__ __forceinline__ void sum_partials(const float* __restrict__ partials, int64_t p0, int64_t p1, double f[3])
+{
+  constexpr int kBatch = 8;
+  float         pv[kBatch][3];
+#pragma unroll
+  for (int k = 0; k < kBatch; k++)
+    if (p0 + k < p1)
+#pragma unroll
+      for (int c = 0; c < 3; c++) pv[k][c] = partials[3 * (p0 + k) + c];
+  f[0] = f[1] = f[2] = 0.0;
+#pragma unroll
+  for (int k = 0; k < kBatch; k++)
+    if (p0 + k < p1) {
+      f[0] += (double)pv[k][0];
+      f[1] += (double)pv[k][1];
+      f[2] += (double)pv[k][2];
+    }
+  for (int64_t p = p0 + kBatch; p < p1; p++) {
+    f[0] += (double)partials[3 * p];
+    f[1] += (double)partials[3 * p + 1];
+    f[2] += (double)partials[3 * p + 2];
+  }
+}
+
+// Closure terms (UqModel::ApplyClosure, src/uq/nimble_uq.cc:327-346) with
+// separate multiply and add, as k_uq_closure rounds them
+__device__ __forceinline__ double closure_scale(double f, double c)
+{
+#pragma clang fp contract(off)
+  return f * c;
+}
+__device__ __forceinline__ void closure_add(double f[3], const double g[3], double c)
+{
+#pragma clang fp contract(off)
+  f[0] += g[0] * c;
+  f[1] += g[1] * c;
+  f[2] += g[2] * c;
+}
+
+// Boundary node bi (partials [p0, p1)) at row i, flags at row xi: its force,
+// then the node update.  Returns its reaction contribution.
 __device__ __forceinline__ double boundary_node(const TileArgs& ta, const NodeArrays& na, const BcEntry* table,
                                                 int64_t i, int64_t xi, int64_t p0, int64_t p1, const StepArgs& sa,
                                                 int rx_coord)
@@ -526,28 +630,8 @@ __device__ __forceinline__ double boundary_node(const TileArgs& ta, const NodeAr
     load3(na.v, i, v);
     m = na.mass[i];
   }
-  // up to 8 partials are loaded at once, then added in ascending order
-  // (the same order as one at a time); more than 8 continue one by one
-  constexpr int kBatch = 8;
-  float         pv[kBatch][3];
-#pragma unroll
-  for (int k = 0; k < kBatch; k++)
-    if (p0 + k < p1)
-#pragma unroll
-      for (int c = 0; c < 3; c++) pv[k][c] = ta.partials[3 * (p0 + k) + c];
-  double f[3] = {0.0, 0.0, 0.0};
-#pragma unroll
-  for (int k = 0; k < kBatch; k++)
-    if (p0 + k < p1) {
-      f[0] += (double)pv[k][0];
-      f[1] += (double)pv[k][1];
-      f[2] += (double)pv[k][2];
-    }
-  for (int64_t p = p0 + kBatch; p < p1; p++) {
-    f[0] += (double)ta.partials[3 * p];
-    f[1] += (double)ta.partials[3 * p + 1];
-    f[2] += (double)ta.partials[3 * p + 2];
-  }
+  double f[3];
+  sum_partials(ta.partials, p0, p1, f);
   const double rxs = rx_coord >= 0 && (flags & kReactionFlag) ? f[rx_coord] : 0.0;
   node_update(na, table, i, flags, f, u, v, m, sa);
   return rxs;
@@ -565,6 +649,76 @@ __global__ __launch_bounds__(kBndThreads) void k_boundary_update(TileArgs ta, No
     rxs = boundary_node(ta, na, na.bc_table, i, i, ta.bnd_ptr[bi], ta.bnd_ptr[bi + 1], sa, rx.coord);
   }
   if (rx.coord < 0) return;
+  const double s = block_sum<kBndThreads>(rxs, red);
+  if (threadIdx.x == 0) rx.partials[ta.num_tiles + g] = s;
+}
+
+// Off-nominal ensemble, one launch for every node: workgroups [0, groups)
+// take the boundary nodes, each thread its node's force and update for the
+// nominal trajectory and every exact sample, the rest the interior nodes,
+// whose forces the element launch stored.  With the trajectories' forces in
+// registers a thread then runs the closure of the approximate samples, as
+// k_uq_closure does.  One launch where a step took one boundary launch per
+// trajectory and the closure: at 48^3 with two exact and five approximate
+// samples --UQ_FIGURES--
+__global__ __launch_bounds__(kBndThreads) void k_uq_nodes(TileArgs ta, NodeArrays na, const BcEntry* sample_bc,
+                                                          UqClosure uc, int num_partials, unsigned groups,
+                                                          StepArgs sa, ReactionArgs rx)
+{
+  __shared__ double red[kBndThreads / 64];
+  const int         ne  = uc.num_exact;
+  const bool        bnd = blockIdx.x < groups;  // uniform
+  const unsigned    g   = bnd ? xcd_tile(blockIdx.x, groups) : xcd_tile(blockIdx.x - groups, gridDim.x - groups);
+  const int64_t     l   = (int64_t)g * kBndThreads + threadIdx.x;
+  const int64_t     i   = bnd ? ta.bnd_base + l : l;
+  double            rxs = 0.0;
+  if (l < (bnd ? ta.num_bnd : ta.bnd_base)) {
+    const int  flags = na.flags[i];
+    NodeArrays ns    = na;  // a sample's arrays
+    ns.bc_table      = sample_bc;
+    const auto of    = [&](int s) {
+      double* b = uc.state + 4 * (int64_t)s * uc.stride;
+      ns.u      = b;
+      ns.v      = b + uc.stride;
+      ns.a      = b + 2 * uc.stride;
+      ns.f      = b + 3 * uc.stride;
+    };
+    double fn[3], fe[kUqCachedExact][3];
+    if (bnd) {
+      const int64_t p0 = ta.bnd_ptr[l], p1 = ta.bnd_ptr[l + 1];
+      sum_partials(ta.partials, p0, p1, fn);
+      if (rx.coord >= 0 && (flags & kReactionFlag)) rxs = fn[rx.coord];
+      double u[3];
+      if (sa.update_v) load3(na.u, i, u);
+      node_step(na, i, flags, fn, u, sa);
+#pragma unroll
+      for (int k = 0; k < kUqCachedExact; k++)
+        if (k < ne) {
+          const int64_t q = (int64_t)(k + 1) * num_partials;
+          sum_partials(ta.partials, q + p0, q + p1, fe[k]);
+          of(k);
+          if (sa.update_v) load3(ns.u, i, u);
+          node_step(ns, i, flags, fe[k], u, sa);
+        }
+    } else {
+      load3(uc.f_nominal, i, fn);
+#pragma unroll
+      for (int k = 0; k < kUqCachedExact; k++)
+        if (k < ne) load3(uc.state + (4 * (int64_t)k + 3) * uc.stride, i, fe[k]);
+    }
+    for (int s = 0; s < uc.num_approx; s++) {
+      const double* c    = uc.coeff + (int64_t)s * (ne + 1);
+      double        f[3] = {closure_scale(fn[0], c[0]), closure_scale(fn[1], c[0]), closure_scale(fn[2], c[0])};
+#pragma unroll
+      for (int k = 0; k < kUqCachedExact; k++)
+        if (k < ne) closure_add(f, fe[k], c[k + 1]);
+      of(ne + s);
+      double u[3];
+      if (sa.update_v) load3(ns.u, i, u);
+      node_step(ns, i, flags, f, u, sa);
+    }
+  }
+  if (rx.coord < 0 || !bnd) return;  // uniform
   const double s = block_sum<kBndThreads>(rxs, red);
   if (threadIdx.x == 0) rx.partials[ta.num_tiles + g] = s;
 }
@@ -615,12 +769,14 @@ template <int kThreads, typename Work>
 void launch_tiles(unsigned grid, const Work& work, const TileArgs& ta, const double* X, const NodeArrays& na,
                   float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t)
 {
-  if (Fip)
+  // an off-nominal ensemble's launch always holds the nominal trajectory
+  if (Fip || std::is_same<Work, UqTileWork>::value) {
     hipExtLaunchKernelGGL((k_element_tiled<kThreads, true, Work>), dim3(grid), dim3(kThreads), 0, s, t.start, t.stop,
                           0, work, ta, X, na, Fip, sip, rx, status);
-  else
+  } else if constexpr (!std::is_same<Work, UqTileWork>::value) {
     hipExtLaunchKernelGGL((k_element_tiled<kThreads, false, Work>), dim3(grid), dim3(kThreads), 0, s, t.start,
                           t.stop, 0, work, ta, X, na, Fip, sip, rx, status);
+  }
 }
 
 template <typename Work>
@@ -649,6 +805,23 @@ void launch_ens_element_tiled(const EnsTileWork& work, const TileArgs& ta, const
                               ReactionArgs rx, int* status, hipStream_t s)
 {
   launch_work(work, work.count, ta, X, na, nullptr, nullptr, rx, status, s);
+}
+
+void launch_uq_element_tiled(const UqTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,
+                             float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s,
+                             const LaunchTimer& timer)
+{
+  launch_work(work, work.count, ta, X, na, Fip, sip, rx, status, s, timer);
+}
+
+void launch_uq_nodes(const TileArgs& ta, const NodeArrays& na, const BcEntry* sample_bc, const UqClosure& uc,
+                     int num_partials, const StepArgs& sa, ReactionArgs rx, hipStream_t s, const LaunchTimer& timer)
+{
+  const unsigned groups   = boundary_grid(ta.num_bnd);
+  const unsigned interior = uc.num_approx > 0 ? boundary_grid(ta.bnd_base) : 0;
+  if (groups + interior == 0) return complete_timer(timer, s);
+  hipExtLaunchKernelGGL(k_uq_nodes, dim3(groups + interior), dim3(kBndThreads), 0, s, timer.start, timer.stop, 0, ta,
+                        na, sample_bc, uc, num_partials, groups, sa, rx);
 }
 
 int element_tiled_groups_per_cu(int tile_elems)

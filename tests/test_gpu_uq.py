@@ -204,3 +204,42 @@ def test_uq_deck_end_to_end(hip_device, tmp_path):
     u2 = run.sample(3)[0]  # sample_displacement_2
     for i, c in enumerate("xyz"):
         assert np.array_equal(vals[f"sample_displacement_2_{c}"][-1], u2[:, i])
+
+
+@pytest.mark.parametrize("tile", [64, 256])
+@pytest.mark.parametrize("approx", [0, 3])
+def test_joint_launches_match_launches_per_trajectory(hip_device, monkeypatch, tile, approx):
+    """Up to 8 exact samples a tiled model advances every trajectory in one
+    element and one node launch, above that launch by launch: the nominal
+    trajectory and the first 8 samples are the same bits either way, and so
+    are approximate samples that give the ninth force no weight."""
+    monkeypatch.setenv("NSM_TILE_ELEMS", str(tile))
+    prob = N.CubeProblem(n=9, materials=[N.problems.STEEL, N.problems.ALUMINIUM], num_steps=12, name="uq")
+    rng = np.random.default_rng(4)
+    scale = rng.uniform(0.8, 1.2, (9, 1))
+    K0 = np.array([b.material.bulk_modulus for b in prob.blocks()])
+    G0 = np.array([b.material.shear_modulus for b in prob.blocks()])
+    c = rng.uniform(-0.5, 1.0, (approx, 10))
+    c[:, 9] = 0.0
+    fields = FIELDS + ("acceleration",)
+    got = []
+    for ne in (8, 9):
+        m = prob.make_model("mixed")
+        assert m.AssemblyInfo()["tiled"] and m.AssemblyInfo()["num_tiles"] > 2
+        m.AddBoundaryCondition("prescribed_displacement", prob.node_layer(4)[:7], 1, 1e-5)
+        m.AddBoundaryCondition("initial_velocity", prob.node_layer(3), 0, 2.0)
+        m.SetUqSamples(K0 * scale[:ne], G0 * scale[:ne], c[:, :ne + 1])
+        integ = prob.make_integrator(m, output_frequency=5)
+        integ.Advance(7)
+        integ.Advance(5)
+        out = [m.GetVectorNodeData(f) for f in fields] + [m.GetReactionHistory(0, 12)]
+        out += [m.GetIntegrationPointData("stress"), m.GetIntegrationPointData("deformation_gradient")]
+        for s in list(range(8)) + [ne + k for k in range(approx)]:
+            out += [m.GetUqNodeData(s, f) for f in fields]
+        m.ComputeInternalForce()
+        out += [m.GetVectorNodeData("internal_force"), m.GetUqNodeData(2, "internal_force")]
+        got.append(out)
+        m.close()
+    assert np.linalg.norm(got[0][0]) > 0 and np.linalg.norm(got[0][-1]) > 0
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
