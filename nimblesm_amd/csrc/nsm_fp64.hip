@@ -11,6 +11,7 @@
 #include "nsm_ensemble.h"
 #include "nsm_fp64_math.h"
 #include "nsm_kernels.h"
+#include "nsm_node_step.h"
 
 namespace nsm {
 namespace {
@@ -301,37 +302,32 @@ struct Lds {
 // read from rjac (k_reference_jacobians; b depends on X only), else formed
 // here as the reference does in every call (src/nimble_element.h:442-500);
 // the same operations either way, so the same bits.
+// b^{-1} and det b of point k of element e
+__device__ __forceinline__ void load_reference(const double* __restrict__ rjac, int64_t e, int k, double bi[9],
+                                               double& detb)
+{
+  const double2* r = (const double2*)(rjac + (e * 8 + k) * 10);
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const double2 v = r[i];
+    bi[2 * i]       = v.x;
+    bi[2 * i + 1]   = v.y;
+  }
+  const double2 v = r[4];
+  bi[8]           = v.x;
+  detb            = v.y;
+}
+
+// The evaluation once the nodes are staged in lds.nodes; bi, detb from
+// load_reference when kRefTable.  Slots are [3][slot_stride].
 template <int kMode, bool kRefTable>
-__device__ __forceinline__ void element_fp64(Lds& lds, int64_t e, bool valid, double K, double G, int64_t E_total,
-                                             const int* __restrict__ conn, const double* __restrict__ X,
-                                             const double* __restrict__ u, const double* __restrict__ rjac,
-                                             double* __restrict__ Fip, double* __restrict__ sip,
-                                             double* __restrict__ slots, int* __restrict__ status)
+__device__ __forceinline__ void staged_element_fp64(Lds& lds, int64_t e, bool valid, double K, double G, double bi[9],
+                                                    double detb, double* __restrict__ Fip, double* __restrict__ sip,
+                                                    double* __restrict__ slots, int64_t slot_stride,
+                                                    int* __restrict__ status)
 {
   const int el = threadIdx.x >> 3;
   const int k  = threadIdx.x & 7;
-  double    bi[9], detb = 1.0;
-  if (kRefTable && kMode != kElementForcesFromStress && valid) {
-    const double2* r = (const double2*)(rjac + (e * 8 + k) * 10);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const double2 v = r[i];
-      bi[2 * i]       = v.x;
-      bi[2 * i + 1]   = v.y;
-    }
-    const double2 v = r[4];
-    bi[8]           = v.x;
-    detb            = v.y;
-  }
-  if (valid) {
-    const int64_t nd = conn[e * 8 + k];
-    lds.nodes.x[el][k][0] = X[3 * nd];
-    lds.nodes.x[el][k][1] = X[3 * nd + 1];
-    lds.nodes.x[el][k][2] = X[3 * nd + 2];
-    lds.nodes.xc[el][k][0] = lds.nodes.x[el][k][0] + u[3 * nd];
-    lds.nodes.xc[el][k][1] = lds.nodes.x[el][k][1] + u[3 * nd + 1];
-    lds.nodes.xc[el][k][2] = lds.nodes.x[el][k][2] + u[3 * nd + 2];
-  }
   __syncthreads();
 
   double ainv[10], sig[6];
@@ -384,18 +380,41 @@ __device__ __forceinline__ void element_fp64(Lds& lds, int64_t e, bool valid, do
   if (valid) {
     double f[3];
     node_force(k, lds.pts.ai[el], lds.pts.sg[el], f);
-    const int64_t ss = 8 * round_up8(E_total), sl = fp64_slot(e, k);  // [comp][slot]
-    slots[sl]          = f[0];
-    slots[ss + sl]     = f[1];
-    slots[2 * ss + sl] = f[2];
+    const int64_t sl            = fp64_slot(e, k);  // [comp][slot]
+    slots[sl]                   = f[0];
+    slots[slot_stride + sl]     = f[1];
+    slots[2 * slot_stride + sl] = f[2];
   }
   if (bad) atomicOr(status, 1);
+}
+
+template <int kMode, bool kRefTable>
+__device__ __forceinline__ void element_fp64(Lds& lds, int64_t e, bool valid, double K, double G, int64_t E_total,
+                                             const int* __restrict__ conn, const double* __restrict__ X,
+                                             const double* __restrict__ u, const double* __restrict__ rjac,
+                                             double* __restrict__ Fip, double* __restrict__ sip,
+                                             double* __restrict__ slots, int* __restrict__ status)
+{
+  const int el = threadIdx.x >> 3;
+  const int k  = threadIdx.x & 7;
+  double    bi[9], detb = 1.0;
+  if (kRefTable && kMode != kElementForcesFromStress && valid) load_reference(rjac, e, k, bi, detb);
+  if (valid) {
+    const int64_t nd = conn[e * 8 + k];
+    lds.nodes.x[el][k][0] = X[3 * nd];
+    lds.nodes.x[el][k][1] = X[3 * nd + 1];
+    lds.nodes.x[el][k][2] = X[3 * nd + 2];
+    lds.nodes.xc[el][k][0] = lds.nodes.x[el][k][0] + u[3 * nd];
+    lds.nodes.xc[el][k][1] = lds.nodes.x[el][k][1] + u[3 * nd + 1];
+    lds.nodes.xc[el][k][2] = lds.nodes.x[el][k][2] + u[3 * nd + 2];
+  }
+  staged_element_fp64<kMode, kRefTable>(lds, e, valid, K, G, bi, detb, Fip, sip, slots, 8 * round_up8(E_total), status);
 }
 
 // The full evaluation is held to 5 waves per SIMD (at most 96 registers):
 // more would cost occupancy, fewer spill.
 template <int kMode, bool kRefTable>
-__global__ __launch_bounds__(kThreads, kMode == kElementFull && kRefTable ? 5 : 1) void k_element_fp64(
+__global__ __launch_bounds__(kThreads, kMode == kElementFull ? 5 : 1) void k_element_fp64(
     const BlockTable<double> bt, int64_t E_total, const int* __restrict__ conn, const double* __restrict__ X,
     const double* __restrict__ u, const double* __restrict__ rjac, double* __restrict__ Fip,
     double* __restrict__ sip, double* __restrict__ slots, int* __restrict__ status)
@@ -443,6 +462,129 @@ __global__ __launch_bounds__(kThreads, 5) void k_ens_element_fp64(EnsNodes en, c
                              ens_load(Gd, (int64_t)kb), ms.num_elem, conn + 8 * (int64_t)ms.elem_base,
                              en.X + 3 * (int64_t)sm.x_base, en.u + 3 * (int64_t)sm.node_base,
                              rjac + 80 * (int64_t)ms.elem_base, nullptr, nullptr, slots + sm.slot_base, status);
+}
+
+// ---------------------------------------------------------------------------
+// Small models: a whole step in one launch.  The element kernel and the node
+// kernel each wait for a few dependent loads; on a mesh that leaves most of
+// the device idle a step is the sum of the two waits.  Here every lane, which
+// serves as node k of its element, first finishes the previous step of that
+// node itself: it sums the node's element forces of the last launch (its
+// incidence row lists their slots in ascending element order, so the sum is
+// the node kernel's) and advances u and v, the same values in every element
+// that shares the node; the lane of the node's first incidence stores them.
+// Elements still read the old state and the old slots meanwhile, so both
+// alternate between two buffers.  Every node is summed up to 8 times instead
+// of once, which larger meshes would pay for in L2 traffic.
+// Step of the 8^3 / 16^3 / 24^3 cube in two launches and in this one: 13.9 /
+// 14.7 / 19.0 us and 9.2 / 10.6 / 16.2 us.
+// ---------------------------------------------------------------------------
+
+// incidence row of (element e, node k): the slots of its node's incidences,
+// ascending element, padded with `pad` (a slot that holds zero)
+__global__ __launch_bounds__(256) void k_incidence_rows(int64_t E, const int* __restrict__ conn,
+                                                        const uint32_t* __restrict__ node_ptr,
+                                                        const uint32_t* __restrict__ node_ent, uint32_t pad,
+                                                        uint32_t* __restrict__ rows)
+{
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 8 * E) return;
+  const int      nd = conn[i];
+  const uint32_t p0 = node_ptr[nd], n = node_ptr[nd + 1] - p0;
+#pragma unroll
+  for (uint32_t j = 0; j < kMaxIncidence; j++) rows[kMaxIncidence * i + j] = j < n ? node_ent[p0 + j] : pad;
+}
+
+// Reaction partial of node tile `tile` (256 nodes) from the last launch's
+// slots, and the total of a step whose partials are complete: the sums of
+// k_node_update and reaction_total, by one wave.
+__device__ __forceinline__ void joint_reaction(const JointStep& js, int tile, double* red)
+{
+  for (int t = threadIdx.x; t < 256; t += kThreads) {
+    const int64_t i = 256 * (int64_t)tile + t;
+    double        r = 0.0;
+    if (i < js.num_nodes && (js.flags[i] & kReactionFlag)) {
+      const double* sl = js.slots_in + js.rx.coord * js.slot_stride;
+      for (uint32_t p = js.node_ptr[i]; p < js.node_ptr[i + 1]; p++) r += sl[js.node_ent[p]];
+    }
+    red[t] = r;
+  }
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    for (int t = threadIdx.x; t < w; t += kThreads) red[t] += red[t + w];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) js.rx.partials[tile] = red[0];
+}
+
+__global__ __launch_bounds__(kThreads, 4) void k_joint_step_fp64(const BlockTable<double> bt, JointStep js,
+                                                                 const int* __restrict__ conn,
+                                                                 const double* __restrict__ X,
+                                                                 const double* __restrict__ rjac,
+                                                                 double* __restrict__ Fip, double* __restrict__ sip,
+                                                                 int* __restrict__ status)
+{
+  __shared__ union {
+    Lds    lds;
+    double red[256];
+  } sh;
+  // the first workgroups form the reaction sums: one per reaction tile, then
+  // the total of the step before
+  unsigned b = blockIdx.x;
+  if (b < js.reaction_groups) {  // uniform
+    const int tiles = (int)js.reaction_groups - (js.fold.n > 0 ? 1 : 0);
+    if ((int)b < tiles) {
+      joint_reaction(js, js.reaction_tiles[b], sh.red);
+    } else {
+      const double total = reaction_total<kThreads>(js.fold.partials, js.fold.tiles, js.fold.n, sh.red);
+      if (threadIdx.x == 0) *js.fold.out = total;
+    }
+    return;
+  }
+  b -= js.reaction_groups;
+  const int     el = threadIdx.x >> 3, k = threadIdx.x & 7;
+  const int64_t e     = bt.off[0] + (int64_t)xcd_tile(b, gridDim.x - js.reaction_groups) * kEPW + el;
+  const bool    valid = e < bt.off[bt.count];
+  const int     blk   = valid ? block_of(bt, e) : 0;
+  double        bi[9], detb = 1.0;
+  if (valid) {
+    load_reference(rjac, e, k, bi, detb);
+    const int64_t nd = conn[e * 8 + k];
+    double        x[3], u[3];
+    load3(X, nd, x);
+    load3(js.u_in, nd, u);
+    if (js.kick) {  // uniform
+      uint32_t     ent[kMaxIncidence];
+      const uint4* row = (const uint4*)(js.rows + kMaxIncidence * (e * 8 + k));
+      const uint4  r0 = row[0], r1 = row[1];
+      ent[0] = r0.x, ent[1] = r0.y, ent[2] = r0.z, ent[3] = r0.w;
+      ent[4] = r1.x, ent[5] = r1.y, ent[6] = r1.z, ent[7] = r1.w;
+      double v[3];
+      load3(js.v_in, nd, v);
+      const double m     = js.mass[nd];
+      const int    flags = js.flags[nd];
+      double       s[3][kMaxIncidence];
+#pragma unroll
+      for (int j = 0; j < kMaxIncidence; j++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) s[c][j] = js.slots_in[c * js.slot_stride + ent[j]];
+      double f[3] = {0.0, 0.0, 0.0}, a[3];
+#pragma unroll
+      for (int j = 0; j < kMaxIncidence; j++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) f[c] += s[c][j];
+      node_advance(js.bc, flags & 0x7f, f, u, v, a, m, js.sa);
+      if (ent[0] == (uint32_t)fp64_slot(e, k)) {
+        store3_stream(js.f, nd, f);
+        store3(js.u_out, nd, u);
+        store3(js.v_out, nd, v);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; c++) sh.lds.nodes.xc[el][k][c] = x[c] + u[c];
+  }
+  staged_element_fp64<kElementFull, true>(sh.lds, e, valid, bt.K[blk], bt.G[blk], bi, detb, Fip, sip, js.slots_out,
+                                          js.slot_stride, status);
 }
 
 // Reference inverse Jacobian and its determinant at every point of elements
@@ -840,6 +982,24 @@ void launch_element_fp64(const BlockTable<double>& bt, int64_t E_total, const in
   else
     NSM_FP64_LAUNCH(kElementFull);
 #undef NSM_FP64_LAUNCH
+}
+
+void launch_incidence_rows(int64_t E, const int* conn, const uint32_t* node_ptr, const uint32_t* node_ent,
+                           uint32_t pad, uint32_t* rows, hipStream_t s)
+{
+  if (E <= 0) return;
+  hipLaunchKernelGGL(k_incidence_rows, dim3(grid_of(8 * E, 256)), dim3(256), 0, s, E, conn, node_ptr, node_ent, pad,
+                     rows);
+}
+
+void launch_joint_step_fp64(const BlockTable<double>& bt, JointStep js, const int* conn, const double* X,
+                            const double* rjac, double* Fip, double* sip, int* status, hipStream_t s)
+{
+  const int64_t n = bt.off[bt.count] - bt.off[0];
+  if (n <= 0) return;
+  js.reaction_groups = (unsigned)((js.rx.coord >= 0 ? js.num_reaction_tiles : 0) + (js.fold.n > 0 ? 1 : 0));
+  hipLaunchKernelGGL(k_joint_step_fp64, dim3(js.reaction_groups + grid_of(n, kEPW)), dim3(kThreads), 0, s, bt, js,
+                     conn, X, rjac, Fip, sip, status);
 }
 
 void launch_reference_jacobians(int64_t E, const int* conn, const double* X, double* out, hipStream_t s)

@@ -224,6 +224,14 @@ struct nsm_model {
   int       num_reaction_tiles = 0;
   size_t    device_bytes = 0;
 
+  // small FP64 models: a step in one launch (k_joint_step_fp64).  Incidence
+  // rows, the second buffers of u and v and two force-slot buffers, allocated
+  // at the first call that uses them.
+  bool      joint_ok    = false;  // every node has 1 to kMaxIncidence incidences, few elements
+  double*   joint_state = nullptr;  // u, v [3N] each, the slots [2][3][joint_stride()], then the rows
+  uint32_t* joint_rows  = nullptr;  // [8 E][kMaxIncidence]
+  int64_t   joint_stride() const { return 8 * nsm::round_up8(E) + 8; }
+
   // tile-local assembly (mixed precision): element tiles, device copies of
   // their arrays; integration-point arrays are stored in tile element order
   bool                 tiled = false;
@@ -851,6 +859,94 @@ bool is_output(int64_t step, int64_t num_load_steps, int64_t output_frequency)
   return step % output_frequency == 0 || step == num_load_steps - 1;
 }
 
+// Whether this call's steps run in one launch each (kernel timing asks for the
+// element and the node launch, and UQ samples need the separate ones).
+bool joint_steps(const nsm_model* md)
+{
+  return md->joint_ok && !md->timing && md->uq_samples() == 0;
+}
+
+int ensure_joint(nsm_model* md)
+{
+  if (md->joint_state) return NSM_OK;
+  const size_t state = 6 * (size_t)md->N + 6 * (size_t)md->joint_stride();
+  const size_t rows  = (size_t)(8 * md->E) * nsm::kMaxIncidence;
+  int          st    = dalloc(&md->joint_state, state + rows / 2, &md->device_bytes);
+  if (st) return st;
+  md->joint_rows = (uint32_t*)(md->joint_state + state);
+  nsm::launch_incidence_rows(md->E, md->conn, md->node_ptr, md->node_ent, (uint32_t)(md->joint_stride() - 8),
+                             md->joint_rows, md->stream);
+  NSM_LAUNCHED();
+  // the slots past the elements', the incidence rows' padding, stay zero
+  NSM_HIP(hipMemsetAsync(md->joint_state, 0, state * sizeof(double), md->stream));
+  return NSM_OK;
+}
+
+// Steps [step, step_end) of a small FP64 model, an odd number of at least
+// three (the last one's node launch then finds u and v where they belong),
+// with times cur for the first and t its end.  `*pending` as in launch_step.
+int launch_joint_steps(nsm_model* md, int64_t step, int64_t step_end, int64_t num_load_steps, int64_t output_frequency,
+                       double dt_user, nsm::StepTimes cur, double* t, int64_t* pending)
+{
+  nsm::BlockTable<double> bt{};
+  bt.count = md->num_blocks;
+  for (int b = 0; b <= md->num_blocks; b++) bt.off[b] = md->blk_off[(size_t)b];
+  for (int b = 0; b < md->num_blocks; b++) {
+    bt.K[b] = md->K[(size_t)b];
+    bt.G[b] = md->G[(size_t)b];
+  }
+  const size_t  N3        = 3 * (size_t)md->N;
+  double* const u[2]      = {md->u, md->joint_state};
+  double* const v[2]      = {md->v, md->joint_state + N3};
+  double* const slots[2]  = {md->joint_state + 2 * N3, md->joint_state + 2 * N3 + 3 * (size_t)md->joint_stride()};
+  nsm::NodeArrays na      = md->node_arrays();
+  na.slot_stride          = md->joint_stride();
+  nsm::JointStep js{};
+  js.rows               = md->joint_rows;
+  js.num_nodes          = md->N;
+  js.slot_stride        = na.slot_stride;
+  js.f                  = md->f;
+  js.mass               = md->m;
+  js.flags              = md->flags;
+  js.bc                 = md->bc_table;
+  js.node_ptr           = md->node_ptr;
+  js.node_ent           = md->node_ent;
+  js.reaction_tiles     = md->reaction_tiles;
+  js.num_reaction_tiles = md->num_reaction_tiles;
+  int64_t fold          = *pending;  // step whose partials are complete
+  for (int64_t n = step; n < step_end; n++) {
+    const int k   = (int)((n - step) & 1);
+    js.kick       = n > step;
+    js.slots_in   = slots[k ^ 1];
+    js.slots_out  = slots[k];
+    js.u_in       = js.kick ? u[k ^ 1] : u[0];
+    js.v_in       = v[k ^ 1];
+    js.u_out      = u[k];
+    js.v_out      = v[k];
+    js.rx         = nsm::ReactionArgs{-1, nullptr};
+    js.fold       = reaction_fold(md, fold);
+    fold          = -1;
+    if (js.kick) {
+      const nsm::StepTimes prev = cur;
+      cur                       = step_times(t, dt_user);
+      js.sa = nsm::StepArgs{prev, cur, (int)is_output(n - 1, num_load_steps, output_frequency), 1, 0, 1, 1};
+      if (reaction_args(md, n - 1, &js.rx)) fold = n - 1;
+    }
+    nsm::launch_joint_step_fp64(bt, js, md->conn, md->X, md->rjac, (double*)md->Fip, (double*)md->sip, md->status,
+                                md->stream);
+    NSM_LAUNCHED();
+  }
+  const int64_t           last = step_end - 1;
+  const nsm::StepArgs     sa{cur, cur, (int)is_output(last, num_load_steps, output_frequency), 0, 1, 1, 1};
+  nsm::ReactionArgs       rx;
+  const bool              want_rx = reaction_args(md, last, &rx);
+  const nsm::ReactionFold rf      = reaction_fold(md, fold);
+  nsm::launch_node_update<double>(na, slots[(last - step) & 1], sa, rx, rf, md->stream);
+  NSM_LAUNCHED();
+  *pending = want_rx ? last : -1;
+  return NSM_OK;
+}
+
 // device node array with w values per node -> host array in mesh node order
 // device staging array of at least `need` values
 int ensure_stage(nsm_model* md, size_t need)
@@ -1039,6 +1135,12 @@ bool use_reference_table(int64_t E)
   return E > 0 && 640 * E <= kRefTableBytes;
 }
 
+// Largest FP64 model whose steps run in one launch each.  Microseconds per
+// step, two launches / one: 16^3 14.7 / 10.6, 24^3 19.0 / 16.2, 32^3 29.4 /
+// 28.1, 36^3 38.2 / 33.6, 40^3 45.9 / 43.0, 48^3 67 / 76 (the eightfold node
+// sums then cost more than the second launch).
+constexpr int64_t kJointElems = 1 << 16;
+
 // Element-tile size of a mixed model: NSM_TILE_ELEMS when it names one;
 // 512 when that already gives every CU two tiles or more; otherwise the
 // autotuner's choice from a few timed steps of a model built with each
@@ -1203,6 +1305,14 @@ int model_create(int64_t num_nodes, const double* reference_coordinates, int num
           (uint32_t)(grouped ? nsm::fp64_slot(k >> 3, (int)(k & 7)) : (k & 7) * E + (k >> 3));
   }
 
+  if (precision == NSM_FP64 && use_reference_table(E) && E <= kJointElems && num_blocks <= nsm::kMaxLaunchBlocks) {
+    md->joint_ok = true;
+    for (int64_t i = 0; i < num_nodes; i++) {
+      const uint32_t n = ptr[(size_t)i + 1] - ptr[(size_t)i];
+      md->joint_ok     = md->joint_ok && n >= 1 && n <= nsm::kMaxIncidence;
+    }
+  }
+
   const size_t N3 = 3 * (size_t)num_nodes;
   const size_t ipw = precision == NSM_FP64 ? sizeof(double) : sizeof(float);
   size_t&      tot = md->device_bytes;
@@ -1293,6 +1403,7 @@ int nsm_model_destroy(nsm_model* md)
   free_dev(md->sip);
   free_dev(md->slots);
   free_dev(md->rjac);
+  free_dev(md->joint_state);
   free_dev(md->elem_tmp);
   free_dev(md->wg_min);
   free_dev(md->status);
@@ -1669,7 +1780,19 @@ int nsm_model_explicit_steps(nsm_model* md, int64_t step_begin, int64_t step_end
     NSM_LAUNCHED();
   }
   int64_t pending = -1;  // step whose reaction total is not yet summed
+  // small FP64 models: all steps in joint launches but the first of an even
+  // number
+  int64_t joint_from = step_end;
+  if (joint_steps(md) && step_end - step_begin >= 3) {
+    if ((st = ensure_joint(md))) return st;
+    joint_from = step_begin + ((step_end - step_begin + 1) & 1);
+  }
   for (int64_t step = step_begin; step < step_end; step++) {
+    if (step == joint_from) {
+      if ((st = launch_joint_steps(md, step, step_end, num_load_steps, output_frequency, dt_user, cur, &t, &pending)))
+        return st;
+      break;
+    }
     const bool     last = step + 1 == step_end;
     double         tn   = t;
     nsm::StepTimes nxt  = cur;

@@ -20,6 +20,34 @@ struct StepArgs {
   int       write_f;    // store the internal force (always when update_v is 0)
 };
 
+// One launch of a small FP64 model's step (k_joint_step_fp64): the previous
+// step of every node from the slots of the launch before (kick; the first
+// launch of a sequence takes u as it is), then this step's element forces.
+constexpr uint32_t kMaxIncidence = 8;  // elements at a node
+struct JointStep {
+  const uint32_t* rows;  // [8 E][kMaxIncidence] (launch_incidence_rows)
+  int64_t         num_nodes, slot_stride;
+  const double *  slots_in, *u_in, *v_in;
+  double *        slots_out, *u_out, *v_out, *f;
+  const double*   mass;
+  const uint8_t*  flags;
+  const BcEntry*  bc;
+  StepArgs        sa;    // of the previous step, with this step's first half
+  int             kick;
+  const uint32_t *node_ptr, *node_ent;
+  const int*      reaction_tiles;
+  int             num_reaction_tiles;
+  ReactionArgs    rx;    // of the previous step (coord -1: none)
+  ReactionFold    fold;  // of the step before it
+  unsigned        reaction_groups;  // set by the launcher
+};
+// rows[8 (8 e + k) + j]: slot of the j-th incidence of node k of element e
+// (ascending element), `pad` past the last
+void launch_incidence_rows(int64_t E, const int* conn, const uint32_t* node_ptr, const uint32_t* node_ent,
+                           uint32_t pad, uint32_t* rows, hipStream_t s);
+void launch_joint_step_fp64(const BlockTable<double>& bt, JointStep js, const int* conn, const double* X,
+                            const double* rjac, double* Fip, double* sip, int* status, hipStream_t s);
+
 // ApplyKinematicBC for the explicit scheme
 // (src/nimble_boundary_condition_manager.h:136-217), resolved per node.
 __device__ __forceinline__ void apply_bc(const BcEntry* table, int code, double v[3], const double u[3],
@@ -72,20 +100,15 @@ __device__ __forceinline__ void store3_stream(double* p, int64_t i, const double
   __builtin_nontemporal_store(r[2], p + 3 * i + 2);
 }
 
-// Node i with assembled internal force f, current displacement u, velocity v
-// and lumped mass m: store f, then a = (1/m)(f + f_ext) with f_ext = 0, second
-// half kick, BCs on output steps, and (fused) the next step's half kick, BC,
-// drift, BC.  Performs stores only (table may live in LDS).
-__device__ __forceinline__ void node_update(const NodeArrays& na, const BcEntry* table, int64_t i, int flags,
-                                            const double f[3], double u[3], double v[3], double m,
-                                            const StepArgs& sa)
+// The second half of a step for a node with internal force f, displacement
+// u, velocity v and lumped mass m: a = (1/m)(f + f_ext) with f_ext = 0, half
+// kick, BCs on output steps, and (fused) the next step's half kick, BC,
+// drift, BC.
+__device__ __forceinline__ void node_advance(const BcEntry* table, int code, const double f[3], double u[3],
+                                             double v[3], double a[3], double m, const StepArgs& sa)
 {
 #pragma clang fp contract(off)
-  if (sa.write_f || !sa.update_v) store3_stream(na.f, i, f);
-  if (!sa.update_v) return;
-  const int    code     = flags & 0x7f;
   const double oneOverM = 1.0 / m;
-  double       a[3];
   a[0] = oneOverM * (f[0] + 0.0);
   a[1] = oneOverM * (f[1] + 0.0);
   a[2] = oneOverM * (f[2] + 0.0);
@@ -97,8 +120,20 @@ __device__ __forceinline__ void node_update(const NodeArrays& na, const BcEntry*
     apply_bc(table, code, v, u, delta_t);
     kick(u, v, sa.nxt.dt);
     apply_bc(table, code, v, u, delta_t);
-    store3(na.u, i, u);
   }
+}
+
+// node_advance of node i, its internal force and new state stored.  Performs
+// stores only (table may live in LDS).
+__device__ __forceinline__ void node_update(const NodeArrays& na, const BcEntry* table, int64_t i, int flags,
+                                            const double f[3], double u[3], double v[3], double m,
+                                            const StepArgs& sa)
+{
+  if (sa.write_f || !sa.update_v) store3_stream(na.f, i, f);
+  if (!sa.update_v) return;
+  double a[3];
+  node_advance(table, flags & 0x7f, f, u, v, a, m, sa);
+  if (sa.fuse) store3(na.u, i, u);
   store3(na.v, i, v);
   if (sa.write_a) store3(na.a, i, a);
 }

@@ -455,3 +455,36 @@ def test_node_fields_of_every_copy_size(hip_device, num_nodes):
     for k in range(2):
         assert len(got[k]) == 3 and all(np.array_equal(g, fields[k]) for g in got[k])
         models[k].close()
+
+
+@pytest.mark.parametrize("n,scattered", [(1, False), (3, True), (7, False), (9, True)])
+def test_joint_steps_match_separate_launches(hip_device, n, scattered):
+    """A small FP64 model advances in one launch per step; with kernel timing
+    enabled it takes the element and the node launch: every field and the
+    reaction history are the same bits, whatever number of steps a call
+    takes, with conditions of every kind, output steps, two blocks and
+    reaction nodes in every node tile."""
+    mats = [N.problems.STEEL, N.problems.ALUMINIUM] if n > 1 else [N.problems.STEEL]
+    prob = N.CubeProblem(n=n, materials=mats, num_steps=20, name="joint").build()
+    nodes = np.arange(0, prob.num_nodes, 3, dtype=np.int32) if scattered else prob.top
+    u0 = 1e-3 * np.sin(3 * prob.X) * prob.X[:, 2:3]
+    got = []
+    for separate in (False, True):
+        m = prob.make_model("fp64")
+        m.AddBoundaryCondition("prescribed_displacement", prob.top[:5], 1, 1e-5)
+        m.AddBoundaryCondition("initial_velocity", prob.top, 0, 2.0)
+        m.SetReactionNodes(nodes, 1)
+        if separate:
+            m.EnableKernelTiming(True, every=1000)
+        integ = prob.make_integrator(m, output_frequency=4)
+        m.SetVectorNodeData("displacement", u0)
+        out = []
+        for steps in (1, 2, 3, 4, 9, 1):
+            integ.Advance(steps)
+            out += [m.GetVectorNodeData(f) for f in ("displacement", "velocity", "acceleration", "internal_force")]
+            out += [m.GetIntegrationPointData("stress"), m.GetReactionHistory(0, integ.step)]
+        got.append(out)
+        m.close()
+    assert np.linalg.norm(got[0][-1]) > 0
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
