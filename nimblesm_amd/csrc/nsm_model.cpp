@@ -224,10 +224,20 @@ struct nsm_model {
   int       num_reaction_tiles = 0;
   size_t    device_bytes = 0;
 
+  bool joint_ok = false;  // the model's steps may run in one launch each
+
+  // small tiled models: a step in one launch (JointTileWork).  Second buffers
+  // of the shared nodes' u and v (rows of num_bnd nodes each) and of the
+  // partials, three buffers of reaction partials and the slots' partial
+  // ranges, allocated at the first call that uses them.
+  double* joint_bnd      = nullptr;  // u, v [3 num_bnd] each, then the reaction partials [3][reaction_stride]
+  int2*   joint_slots    = nullptr;
+  float*  joint_partials = nullptr;
+  int     num_bnd_reaction_groups = 0;  // entries of reaction_tiles past the element tiles'
+
   // small FP64 models: a step in one launch (k_joint_step_fp64).  Incidence
   // rows, the second buffers of u and v and two force-slot buffers, allocated
   // at the first call that uses them.
-  bool      joint_ok    = false;  // every node has 1 to kMaxIncidence incidences, few elements
   double*   joint_state = nullptr;  // u, v [3N] each, the slots [2][3][joint_stride()], then the rows
   uint32_t* joint_rows  = nullptr;  // [8 E][kMaxIncidence]
   int64_t   joint_stride() const { return 8 * nsm::round_up8(E) + 8; }
@@ -490,6 +500,7 @@ int rebuild_bcs(nsm_model* md)
                         hipMemcpyHostToDevice));
   }
   std::vector<int> tiles;
+  md->num_bnd_reaction_groups = 0;
   const bool       have_rx = md->reaction_mask.size() == code.size();
   for (size_t i = 0; i < code.size(); i++)  // device node order
     if (have_rx && md->reaction_mask[(size_t)mesh_node(md, (int64_t)i)]) {
@@ -511,7 +522,7 @@ int rebuild_bcs(nsm_model* md)
     for (size_t b = 0; b < ts.bnd_nodes.size(); b++)
       if (md->reaction_mask[(size_t)mesh_node(md, ts.bnd_nodes[b])]) {
         const int g = ts.num_tiles + (int)(b / nsm::kBoundaryNodesPerGroup);
-        if (tiles.empty() || tiles.back() != g) tiles.push_back(g);
+        if (tiles.empty() || tiles.back() != g) tiles.push_back(g), md->num_bnd_reaction_groups++;
       }
   }
   NSM_HIP(hipMemcpy(md->flags, code.data(), code.size(), hipMemcpyHostToDevice));
@@ -832,6 +843,12 @@ int setup_tiles(nsm_model* md)
   if ((st = dalloc(&partials, std::max<size_t>(3 * ts.bnd_ent.size(), 1), &md->device_bytes))) return st;
   md->tile_bufs.push_back((void*)partials);
   ta.partials = partials;
+  // Steps in one launch: one workgroup per tile, all of them on the device at
+  // once (larger models need the persistent kernel's prefetch), shared nodes that a second launch would wait for,
+  // each of them in some tile.
+  md->joint_ok = md->num_blocks <= nsm::kMaxLaunchBlocks && ts.num_tiles <= ta.resident_groups && ta.num_bnd > 0;
+  for (int b = 0; b < ta.num_bnd && md->joint_ok; b++)
+    md->joint_ok = ts.bnd_ptr[(size_t)b + 1] > ts.bnd_ptr[(size_t)b];
   md->blk_tile_off.assign((size_t)md->num_blocks + 1, 0);
   for (int b = 0; b <= md->num_blocks; b++)
     md->blk_tile_off[(size_t)b] =
@@ -868,6 +885,18 @@ bool joint_steps(const nsm_model* md)
 
 int ensure_joint(nsm_model* md)
 {
+  if (md->tiled) {
+    if (md->joint_bnd) return NSM_OK;
+    const size_t bnd   = 6 * (size_t)md->tile_args.num_bnd + 3 * (size_t)md->reaction_stride;
+    const size_t slots = md->tiles.nodes.size(), values = 3 * md->tiles.bnd_ent.size();
+    int          st    = dalloc(&md->joint_bnd, bnd + slots + (values + 1) / 2, &md->device_bytes);
+    if (st) return st;
+    md->joint_slots    = (int2*)(md->joint_bnd + bnd);
+    md->joint_partials = (float*)(md->joint_slots + slots);
+    nsm::launch_slot_partials(md->tile_args, (int)slots, md->joint_slots, md->stream);
+    NSM_LAUNCHED();
+    return NSM_OK;
+  }
   if (md->joint_state) return NSM_OK;
   const size_t state = 6 * (size_t)md->N + 6 * (size_t)md->joint_stride();
   const size_t rows  = (size_t)(8 * md->E) * nsm::kMaxIncidence;
@@ -879,6 +908,71 @@ int ensure_joint(nsm_model* md)
   NSM_LAUNCHED();
   // the slots past the elements', the incidence rows' padding, stay zero
   NSM_HIP(hipMemsetAsync(md->joint_state, 0, state * sizeof(double), md->stream));
+  return NSM_OK;
+}
+
+// Steps [step, step_end) of a small tiled model; see launch_joint_steps.
+int launch_joint_tiled_steps(nsm_model* md, int64_t step, int64_t step_end, int64_t num_load_steps,
+                             int64_t output_frequency, double dt_user, nsm::StepTimes cur, double* t,
+                             int64_t* pending)
+{
+  const nsm::NodeArrays na = md->node_arrays();
+  nsm::TileArgs         ta[2] = {md->tile_args, md->tile_args};
+  ta[1].partials              = md->joint_partials;
+  // row i of a shared node at 3 i in both buffers
+  const ptrdiff_t base   = 3 * (ptrdiff_t)md->tile_args.bnd_base;
+  double* const   bu[2]  = {md->u, md->joint_bnd - base};
+  double* const   bv[2]  = {md->v, md->joint_bnd + 3 * (ptrdiff_t)md->tile_args.num_bnd - base};
+  double* const   rx3    = md->joint_bnd + 6 * (size_t)md->tile_args.num_bnd;
+  const int64_t   last   = step_end - 1;
+  // a step's partials are written in two launches and summed in the one
+  // after: three buffers; the last step's go where the caller sums them
+  const auto partials_of = [&](int64_t n) {
+    return n == last ? reaction_partials_of(md, n) : rx3 + (n % 3) * md->reaction_stride;
+  };
+  const bool want_rx = wants_reaction(md, step);
+  int64_t    fold    = *pending;
+  const double* fold_partials = fold >= 0 ? reaction_partials_of(md, fold) : nullptr;
+  nsm::JointTileWork w{};
+  w.bt            = float_table(md, 0, md->num_blocks, -1);
+  w.t_count       = md->tiles.num_tiles;
+  w.slot_partials = md->joint_slots;
+  w.coord         = md->reaction_coord;
+  w.groups        = md->reaction_tiles + (md->num_reaction_tiles - md->num_bnd_reaction_groups);
+  for (int64_t n = step; n < step_end; n++) {
+    const int            k    = (int)((n - step) & 1);
+    const nsm::StepTimes prev = w.sa.cur;
+    const nsm::StepTimes nxt  = n < last ? step_times(t, dt_user) : cur;
+    w.kick                    = n > step;
+    w.prev = nsm::StepArgs{prev, cur, (int)is_output(n - 1, num_load_steps, output_frequency), 1, 0, 1, 1};
+    w.sa   = nsm::StepArgs{cur, nxt, (int)is_output(n, num_load_steps, output_frequency), (int)(n < last),
+                           (int)(n == last), 1, 1};
+    w.partials_in     = ta[k ^ 1].partials;
+    w.bu_in           = w.kick ? bu[k ^ 1] : bu[0];
+    w.bv_in           = bv[k ^ 1];
+    w.bu_out          = bu[k];
+    w.bv_out          = bv[k];
+    w.fold            = nsm::ReactionFold{fold_partials, md->reaction_tiles, fold >= 0 ? md->num_reaction_tiles : 0,
+                               md->reaction_hist + std::max<int64_t>(fold, 0)};
+    w.prev_rx         = w.kick && want_rx ? partials_of(n - 1) : nullptr;
+    w.reaction_groups = (unsigned)((w.prev_rx ? md->num_bnd_reaction_groups : 0) + (w.fold.n > 0 ? 1 : 0));
+    const nsm::ReactionArgs rx{want_rx ? md->reaction_coord : -1, want_rx ? partials_of(n) : nullptr};
+    nsm::launch_joint_element_tiled(w, ta[k], md->X, na, (float*)md->Fip, (float*)md->sip, rx, md->status,
+                                    md->stream);
+    NSM_LAUNCHED();
+    fold          = w.kick && want_rx ? n - 1 : -1;
+    fold_partials = fold >= 0 ? partials_of(fold) : nullptr;
+    cur           = nxt;
+  }
+  const nsm::ReactionArgs rx{want_rx ? md->reaction_coord : -1, want_rx ? partials_of(last) : nullptr};
+  nsm::launch_boundary_update(ta[(last - step) & 1], na, w.sa, rx, md->stream);
+  NSM_LAUNCHED();
+  if (fold >= 0 && md->num_reaction_tiles > 0) {
+    nsm::launch_reaction_finalize(fold_partials, md->reaction_tiles, md->num_reaction_tiles, md->reaction_hist + fold,
+                                  md->stream);
+    NSM_LAUNCHED();
+  }
+  *pending = want_rx ? last : -1;
   return NSM_OK;
 }
 
@@ -1404,6 +1498,7 @@ int nsm_model_destroy(nsm_model* md)
   free_dev(md->slots);
   free_dev(md->rjac);
   free_dev(md->joint_state);
+  free_dev(md->joint_bnd);
   free_dev(md->elem_tmp);
   free_dev(md->wg_min);
   free_dev(md->status);
@@ -1780,8 +1875,7 @@ int nsm_model_explicit_steps(nsm_model* md, int64_t step_begin, int64_t step_end
     NSM_LAUNCHED();
   }
   int64_t pending = -1;  // step whose reaction total is not yet summed
-  // small FP64 models: all steps in joint launches but the first of an even
-  // number
+  // small models: all steps in joint launches but the first of an even number
   int64_t joint_from = step_end;
   if (joint_steps(md) && step_end - step_begin >= 3) {
     if ((st = ensure_joint(md))) return st;
@@ -1789,8 +1883,11 @@ int nsm_model_explicit_steps(nsm_model* md, int64_t step_begin, int64_t step_end
   }
   for (int64_t step = step_begin; step < step_end; step++) {
     if (step == joint_from) {
-      if ((st = launch_joint_steps(md, step, step_end, num_load_steps, output_frequency, dt_user, cur, &t, &pending)))
-        return st;
+      st = md->tiled ? launch_joint_tiled_steps(md, step, step_end, num_load_steps, output_frequency, dt_user, cur, &t,
+                                                &pending)
+                     : launch_joint_steps(md, step, step_end, num_load_steps, output_frequency, dt_user, cur, &t,
+                                          &pending);
+      if (st) return st;
       break;
     }
     const bool     last = step + 1 == step_end;

@@ -69,6 +69,33 @@ struct EnsTileWork {
   EnsFold          fold;
 };
 
+// Small models, a whole step in one launch (one workgroup per tile): while
+// staging its nodes a tile first finishes the previous step of the shared
+// ones from the partials of the launch before, in every tile that holds the
+// node, the first of them storing the result; the shared nodes' u and v and
+// the partials alternate between two buffers meanwhile.  Bound by latency:
+// us per step in two launches / this one, 128-element tiles, 6^3 16.3 / 13.1,
+// 25^3 17.4 / 14.7, 40^3 21.3 / 18.0, 48^3 (864 of 1024 resident tiles) 25.7 /
+// 23.3.
+struct JointTileWork {
+  BlockTable<float> bt;
+  int               t_begin, t_count;
+  StepArgs          sa;       // this step
+  StepArgs          prev;     // the previous step, with this step's first half
+  int               kick;     // 0: the shared nodes are up to date (a sequence's first launch)
+  const int2*       slot_partials;  // per tile-node slot: its shared node's first partial and their count
+  const float*      partials_in;
+  const double *    bu_in, *bv_in;  // row i of a shared node at 3 i (i its node id)
+  double *          bu_out, *bv_out;
+  // the first workgroups: reaction partials of the previous step's shared
+  // nodes (groups of 256), then the total of the step before it
+  unsigned          reaction_groups;
+  int               coord;
+  const int*        groups;   // partial indices of the groups holding reaction nodes
+  double*           prev_rx;  // the previous step's partials
+  ReactionFold      fold;
+};
+
 // Off-nominal ensemble: the tiles [t_begin, t_begin + t_count) of the nominal
 // trajectory (s = 0) and of every exact sample (s >= 1) of one model in one
 // launch, work item i being tile t_begin + i % t_count of trajectory
@@ -115,6 +142,10 @@ void launch_ens_element_tiled(const EnsTileWork& work, const TileArgs& ta, const
 // sample; reaction partial of group g at rx.partials[rx_base + g].
 void launch_ens_boundary_update(const TileArgs& ta, const EnsNodes& en, const EnsRange* groups, int num_groups,
                                 EnsStep es, ReactionArgs rx, int rx_base, hipStream_t s);
+// slot_partials of JointTileWork
+void launch_slot_partials(const TileArgs& ta, int num_slots, int2* out, hipStream_t s);
+void launch_joint_element_tiled(const JointTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,
+                                float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s);
 // Every trajectory's tiles of an off-nominal ensemble; then the shared nodes
 // of every trajectory from their partials and, for every node, the closure
 // forces of the approximate samples (as launch_uq_closure) with their update.

@@ -160,7 +160,8 @@ struct NodeState {
 template <int kThreads>
 __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const double (&xr)[2][3],
                                       const double (&ur)[2][3], const NodeArrays& na, int update_v,
-                                      double (*sxu)[6], Assembly<kThreads>& as, bool gather, NodeState& ns)
+                                      double (*sxu)[6], Assembly<kThreads>& as, bool gather, NodeState& ns,
+                                      bool load_state = true)
 {
   if (gather && threadIdx.x < 24) as.g.ef[threadIdx.x][kThreads] = 0.0f;
 #pragma unroll
@@ -178,7 +179,7 @@ __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const dou
 #pragma unroll
         for (int c = 0; c < 3; c++) as.acc[ln][c] = 0.0;
     }
-    if (ids.dst[k] == kInterior) {
+    if (load_state && ids.dst[k] == kInterior) {
       ns.flg[k] = na.flags[ids.gid[k] + x_delta];
       if (update_v) {
         load3(na.v, ids.gid[k], ns.v[k]);
@@ -192,9 +193,11 @@ __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const dou
 __device__ __forceinline__ int work_count(const ModelTileWork& w) { return w.t_count; }
 __device__ __forceinline__ int work_count(const EnsTileWork& w) { return w.count; }
 __device__ __forceinline__ int work_count(const UqTileWork& w) { return w.count; }
+__device__ __forceinline__ int work_count(const JointTileWork& w) { return w.t_count; }
 __device__ __forceinline__ int work_update_v(const ModelTileWork& w) { return w.sa.update_v; }
 __device__ __forceinline__ int work_update_v(const EnsTileWork& w) { return w.es.update_v; }
 __device__ __forceinline__ int work_update_v(const UqTileWork& w) { return w.sa.update_v; }
+__device__ __forceinline__ int work_update_v(const JointTileWork&) { return 1; }
 
 __device__ __forceinline__ TileCtx tile_ctx(const ModelTileWork& w, int i)
 {
@@ -208,6 +211,10 @@ __device__ __forceinline__ TileCtx tile_ctx(const EnsTileWork& w, int i)
                  uniform(sm.partial_base), uniform(sm.bc_base), uniform(sm.kg_base)};
 }
 
+__device__ __forceinline__ TileCtx tile_ctx(const JointTileWork& w, int i)
+{
+  return TileCtx{w.t_begin + i, 0, 0, 0, 0, 0, 0};
+}
 __device__ __forceinline__ TileCtx tile_ctx(const UqTileWork& w, int i)
 {
   int s = 0;
@@ -251,10 +258,12 @@ __device__ __forceinline__ bool item_output(const UqTileWork&, const TileCtx& c)
 
 __device__ __forceinline__ const BcEntry* work_bc(const ModelTileWork&) { return nullptr; }
 __device__ __forceinline__ const BcEntry* work_bc(const UqTileWork&) { return nullptr; }
+__device__ __forceinline__ const BcEntry* work_bc(const JointTileWork&) { return nullptr; }
 __device__ __forceinline__ const BcEntry* work_bc(const EnsTileWork& w) { return w.bc; }
 
 // moduli of the tile's block (tiles never straddle blocks)
-__device__ __forceinline__ void tile_moduli(const ModelTileWork& w, const TileCtx&, int e0, float& K, float& G)
+template <typename Work>
+__device__ __forceinline__ void tile_moduli(const Work& w, const TileCtx&, int e0, float& K, float& G)
 {
   const int b = uniform(block_of(w.bt, (int64_t)e0));
   K           = w.bt.K[b];
@@ -276,6 +285,7 @@ __device__ __forceinline__ void tile_moduli(const UqTileWork& w, const TileCtx& 
 
 __device__ __forceinline__ StepArgs tile_step(const ModelTileWork& w, const TileCtx&) { return w.sa; }
 __device__ __forceinline__ StepArgs tile_step(const UqTileWork& w, const TileCtx&) { return w.sa; }
+__device__ __forceinline__ StepArgs tile_step(const JointTileWork& w, const TileCtx&) { return w.sa; }
 __device__ __forceinline__ StepArgs tile_step(const EnsTileWork& w, const TileCtx& c)
 {
   return ens_step_args(w.es, c.s);
@@ -284,6 +294,7 @@ __device__ __forceinline__ StepArgs tile_step(const EnsTileWork& w, const TileCt
 // index of the tile's reaction partial
 __device__ __forceinline__ int tile_rx_slot(const ModelTileWork&, const TileCtx& c, int) { return c.t; }
 __device__ __forceinline__ int tile_rx_slot(const UqTileWork&, const TileCtx& c, int) { return c.t; }
+__device__ __forceinline__ int tile_rx_slot(const JointTileWork&, const TileCtx& c, int) { return c.t; }
 __device__ __forceinline__ int tile_rx_slot(const EnsTileWork&, const TileCtx&, int i) { return i; }
 
 // A previous step's reaction total(s): workgroup 0 sums the model's
@@ -307,6 +318,120 @@ __device__ __forceinline__ void fold_previous(const EnsTileWork& w, double*)
     const int    p0    = f.ptr[s];
     const double total = wave_reaction_total(f.partials, f.idx + p0, f.ptr[s + 1] - p0);
     if ((threadIdx.x & 63) == 0) f.hist[(int64_t)s * f.hist_stride + f.step] = total;
+  }
+}
+
+// Force of a boundary node: its partials [p0, p1) in ascending tile order
+// from 0.0 in FP64.  Up to 8 partials are loaded at once, then added in
+// ascending order (the same order as one at a time); more than 8 continue
+// one by one.
+__device__ __forceinline__ void sum_partials(const float* __restrict__ partials, int64_t p0, int64_t p1, double f[3])
+{
+  constexpr int kBatch = 8;
+  float         pv[kBatch][3];
+#pragma unroll
+  for (int k = 0; k < kBatch; k++)
+    if (p0 + k < p1)
+#pragma unroll
+      for (int c = 0; c < 3; c++) pv[k][c] = partials[3 * (p0 + k) + c];
+  f[0] = f[1] = f[2] = 0.0;
+#pragma unroll
+  for (int k = 0; k < kBatch; k++)
+    if (p0 + k < p1) {
+      f[0] += (double)pv[k][0];
+      f[1] += (double)pv[k][1];
+      f[2] += (double)pv[k][2];
+    }
+  for (int64_t p = p0 + kBatch; p < p1; p++) {
+    f[0] += (double)partials[3 * p];
+    f[1] += (double)partials[3 * p + 1];
+    f[2] += (double)partials[3 * p + 2];
+  }
+}
+
+// Joint steps: the reaction partial of the boundary group `group` (256 shared
+// nodes) of the previous step, as k_boundary_update sums it.
+template <int kThreads>
+__device__ __forceinline__ void joint_reaction(const JointTileWork& w, const TileArgs& ta, const NodeArrays& na,
+                                               int group, double* red)
+{
+  for (int t0 = 0; t0 < kBoundaryNodesPerGroup; t0 += kThreads) {
+    const int t = t0 + (int)threadIdx.x;
+    if (t >= kBoundaryNodesPerGroup) break;  // whole waves
+    const int bi = (group - ta.num_tiles) * kBoundaryNodesPerGroup + t;
+    double    v  = 0.0;
+    if (bi < ta.num_bnd && (na.flags[ta.bnd_base + bi] & kReactionFlag)) {
+      double f[3];
+      sum_partials(w.partials_in, ta.bnd_ptr[bi], ta.bnd_ptr[bi + 1], f);
+      v = f[w.coord];
+    }
+#pragma unroll
+    for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m, 64);
+    if ((t & 63) == 0) red[t >> 6] = v;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int q = 0; q < kBoundaryNodesPerGroup / 64; q++) s += red[q];
+    w.prev_rx[group] = s;
+  }
+}
+
+// Joint steps: u of the thread's slots, the shared nodes' after their
+// previous step (see JointTileWork), and the flags, mass and v of its
+// interior nodes (left in ns).  Every load of both slots is issued before the
+// first is used, whatever kind of slot it is (an interior slot's partials are
+// entry 0, not used): a branch around them would make the kernel wait for one
+// slot's chain after the other's.  table (LDS) is staged in the meantime.
+template <int kThreads>
+__device__ __forceinline__ void joint_nodes(const JointTileWork& w, const TileArgs& ta, const TileCtx& c,
+                                            const SlotIds& ids, const NodeArrays& na, const BcEntry* table,
+                                            double (&ur)[2][3], NodeState& ns)
+{
+  constexpr int kBatch = 8;
+  const int     n0 = tile_table(ta.node_off, c.t), nn = tile_table(ta.node_off, c.t + 1) - n0;
+  int2          p[2];
+  float         pv[2][kBatch][3];
+#pragma unroll
+  for (int k = 0; k < 2; k++) p[k] = w.slot_partials[n0 + min((int)threadIdx.x + k * kThreads, nn - 1)];
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const bool own = ids.dst[k] == kInterior;
+    const int  i   = ids.gid[k];
+    load3(own ? na.u : w.bu_in, i, ur[k]);
+    load3(own ? na.v : w.bv_in, i, ns.v[k]);
+    ns.flg[k] = na.flags[i];
+    ns.m[k]   = na.mass[i];
+  }
+  if (w.kick)  // uniform
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int j = 0; j < kBatch; j++)
+#pragma unroll
+        for (int cc = 0; cc < 3; cc++) pv[k][j][cc] = w.partials_in[3 * (p[k].x + max(min(j, p[k].y - 1), 0)) + cc];
+  __syncthreads();  // table
+  if (!w.kick) return;
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    if (ids.dst[k] == kInterior || ids.dst[k] == kAbsent) continue;
+    double f[3] = {0.0, 0.0, 0.0}, v[3] = {ns.v[k][0], ns.v[k][1], ns.v[k][2]}, a[3];
+#pragma unroll
+    for (int j = 0; j < kBatch; j++)
+      if (j < p[k].y)
+#pragma unroll
+        for (int cc = 0; cc < 3; cc++) f[cc] += (double)pv[k][j][cc];
+    for (int64_t q = p[k].x + kBatch; q < p[k].x + p[k].y; q++)
+#pragma unroll
+      for (int cc = 0; cc < 3; cc++) f[cc] += (double)w.partials_in[3 * q + cc];
+    const int i = ids.gid[k];
+    node_advance(table, ns.flg[k] & 0x7f, f, ur[k], v, a, ns.m[k], w.prev);
+    if (ids.dst[k] == p[k].x) {  // the node's first tile
+      store3_stream(na.f, i, f);
+      store3(w.bu_out, i, ur[k]);
+      store3(w.bv_out, i, v);
+    }
   }
 }
 
@@ -334,6 +459,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
   constexpr int  kNodes      = 2 * kThreads;
   constexpr bool kEnsemble   = std::is_same<Work, EnsTileWork>::value;
   constexpr bool kUq         = std::is_same<Work, UqTileWork>::value;
+  constexpr bool kJoint      = std::is_same<Work, JointTileWork>::value;  // one item per workgroup, no prefetch
   // ensembles stage each tile's sample's kinematic-condition entries (one
   // 8-byte word per thread)
   constexpr int  kTileBcWords = kBcWords * kEnsMaxBcCodes;
@@ -347,15 +473,31 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
   __shared__ int     bad;
   __shared__ double  fold_red[256];
 
-  fold_previous<kThreads>(work, fold_red);
+  unsigned block = blockIdx.x, blocks = gridDim.x;
+  if constexpr (kJoint) {
+    if (block < work.reaction_groups) {  // uniform
+      const bool last = work.fold.n > 0 && block == work.reaction_groups - 1;
+      if (last) {
+        const double total = reaction_total<kThreads>(work.fold.partials, work.fold.tiles, work.fold.n, fold_red);
+        if (threadIdx.x == 0) *work.fold.out = total;
+      } else {
+        joint_reaction<kThreads>(work, ta, na, work.groups[block], fold_red);
+      }
+      return;
+    }
+    block -= work.reaction_groups;
+    blocks -= work.reaction_groups;
+  } else {
+    fold_previous<kThreads>(work, fold_red);
+  }
 
   // Workgroup w (numbered so that each XCD holds a contiguous run of w)
   // processes work items w, w + G, w + 2G, ... (G workgroups): at any time
   // the grid works on one window of G consecutive tiles, so the F and sigma
   // rows are written in one narrow address range and each XCD's L2 sees
   // neighbouring tiles.
-  const int G        = (int)gridDim.x;
-  const int w        = (int)xcd_tile(blockIdx.x, gridDim.x);
+  const int G        = (int)blocks;
+  const int w        = (int)xcd_tile(block, blocks);
   const int count    = work_count(work);
   const int update_v = work_update_v(work);
   const int ib       = uniform(w);
@@ -374,17 +516,19 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     reinterpret_cast<uint64_t*>(sbc)[tid] =
         reinterpret_cast<const uint64_t*>(work_bc(work) + c_first.bc_base)[tid];
   SlotIds ids      = load_ids<kThreads>(ta, c_first);
-  SlotIds ids_next = load_ids<kThreads>(ta, tile_ctx(work, next(ib)));
+  ElemData  cur = load_elem<kThreads>(ta, c_first.t);
+  NodeState ns;
+  SlotIds   ids_next{};
+  if (!kJoint) ids_next = load_ids<kThreads>(ta, tile_ctx(work, next(ib)));
   double  xr[2][3], ur[2][3];
 #pragma unroll
   for (int k = 0; k < 2; k++) {
     load3(X, ids.gid[k] + c_first.x_delta, xr[k]);
-    load3(work_arrays(work, c_first, na).u, ids.gid[k], ur[k]);
+    if (!kJoint) load3(work_arrays(work, c_first, na).u, ids.gid[k], ur[k]);
   }
-  ElemData  cur = load_elem<kThreads>(ta, c_first.t);
-  NodeState ns;
+  if constexpr (kJoint) joint_nodes<kThreads>(work, ta, c_first, ids, na, sbc, ur, ns);
   stage<kThreads>(ids, c_first.x_delta, xr, ur, work_arrays(work, c_first, na), update_v, sxu, as,
-                  tile_table(ta.gather, c_first.t) != 0, ns);
+                  tile_table(ta.gather, c_first.t) != 0, ns, !kJoint);
   // every prologue load complete (vmcnt(0); lgkmcnt and expcnt at their
   // maximum, gfx9 encoding): the loop's waits then depend on its body only
   __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -401,13 +545,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     // ---- prefetch (clamped to this workgroup's last item): the next
     // item's nodes and elements, the node ids of the one after, and (in
     // ensembles) the next item's sample's condition entries
+    ElemData el_next   = cur;
+    SlotIds  ids_after = ids;
+    if (!kJoint) {
 #pragma unroll
-    for (int k = 0; k < 2; k++) {
-      load3(X, ids_next.gid[k] + cn.x_delta, xr[k]);
-      load3(work_arrays(work, cn, na).u, ids_next.gid[k], ur[k]);
+      for (int k = 0; k < 2; k++) {
+        load3(X, ids_next.gid[k] + cn.x_delta, xr[k]);
+        load3(work_arrays(work, cn, na).u, ids_next.gid[k], ur[k]);
+      }
+      el_next   = load_elem<kThreads>(ta, cn.t);
+      ids_after = load_ids<kThreads>(ta, tile_ctx(work, next(next(i))));
     }
-    const ElemData el_next   = load_elem<kThreads>(ta, cn.t);
-    const SlotIds  ids_after = load_ids<kThreads>(ta, tile_ctx(work, next(next(i))));
     uint64_t       bc_next   = 0;
     if (kEnsemble)
       bc_next = reinterpret_cast<const uint64_t*>(work_bc(work) + cn.bc_base)[min(tid, kTileBcWords - 1)];
@@ -571,34 +719,6 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
 }
 
 constexpr int kBndThreads = kBoundaryNodesPerGroup;
-
-// Force of a boundary node: its partials [p0, p1) in ascending tile order
-// from 0.0 in FP64.  Up to 8 partials are loaded at once, then added in
-// ascending order (the same order as one at a time); more than 8 continue
-// one by one.
-__device__ __forceinline__ void sum_partials(const float* __restrict__ partials, int64_t p0, int64_t p1, double f[3])
-{
-  constexpr int kBatch = 8;
-  float         pv[kBatch][3];
-#pragma unroll
-  for (int k = 0; k < kBatch; k++)
-    if (p0 + k < p1)
-#pragma unroll
-      for (int c = 0; c < 3; c++) pv[k][c] = partials[3 * (p0 + k) + c];
-  f[0] = f[1] = f[2] = 0.0;
-#pragma unroll
-  for (int k = 0; k < kBatch; k++)
-    if (p0 + k < p1) {
-      f[0] += (double)pv[k][0];
-      f[1] += (double)pv[k][1];
-      f[2] += (double)pv[k][2];
-    }
-  for (int64_t p = p0 + kBatch; p < p1; p++) {
-    f[0] += (double)partials[3 * p];
-    f[1] += (double)partials[3 * p + 1];
-    f[2] += (double)partials[3 * p + 2];
-  }
-}
 
 // Closure terms (UqModel::ApplyClosure, src/uq/nimble_uq.cc:327-346) with
 // separate multiply and add, as k_uq_closure rounds them
@@ -770,12 +890,25 @@ void launch_tiles(unsigned grid, const Work& work, const TileArgs& ta, const dou
                   float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t)
 {
   // an off-nominal ensemble's launch always holds the nominal trajectory
-  if (Fip || std::is_same<Work, UqTileWork>::value) {
+  constexpr bool kStores = std::is_same<Work, UqTileWork>::value || std::is_same<Work, JointTileWork>::value;
+  if (Fip || kStores) {
     hipExtLaunchKernelGGL((k_element_tiled<kThreads, true, Work>), dim3(grid), dim3(kThreads), 0, s, t.start, t.stop,
                           0, work, ta, X, na, Fip, sip, rx, status);
-  } else if constexpr (!std::is_same<Work, UqTileWork>::value) {
+  } else if constexpr (!kStores) {
     hipExtLaunchKernelGGL((k_element_tiled<kThreads, false, Work>), dim3(grid), dim3(kThreads), 0, s, t.start,
                           t.stop, 0, work, ta, X, na, Fip, sip, rx, status);
+  }
+}
+
+template <typename Work>
+void launch_grid(const Work& work, unsigned grid, const TileArgs& ta, const double* X, const NodeArrays& na,
+                 float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t)
+{
+  switch (ta.tile_elems) {
+    case 64: launch_tiles<64>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    case 128: launch_tiles<128>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    case 512: launch_tiles<512>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    default: launch_tiles<256>(grid, work, ta, X, na, Fip, sip, rx, status, s, t);
   }
 }
 
@@ -784,13 +917,7 @@ void launch_work(const Work& work, int count, const TileArgs& ta, const double* 
                  float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t = LaunchTimer{})
 {
   if (count <= 0) return complete_timer(t, s);
-  const unsigned grid = (unsigned)std::min(count, std::max(ta.resident_groups, 1));
-  switch (ta.tile_elems) {
-    case 64: launch_tiles<64>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    case 128: launch_tiles<128>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    case 512: launch_tiles<512>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    default: launch_tiles<256>(grid, work, ta, X, na, Fip, sip, rx, status, s, t);
-  }
+  launch_grid(work, (unsigned)std::min(count, std::max(ta.resident_groups, 1)), ta, X, na, Fip, sip, rx, status, s, t);
 }
 
 void launch_element_tiled(const BlockTable<float>& bt, const TileArgs& ta, int t_begin, int t_count,
@@ -805,6 +932,32 @@ void launch_ens_element_tiled(const EnsTileWork& work, const TileArgs& ta, const
                               ReactionArgs rx, int* status, hipStream_t s)
 {
   launch_work(work, work.count, ta, X, na, nullptr, nullptr, rx, status, s);
+}
+
+__global__ __launch_bounds__(256) void k_slot_partials(TileArgs ta, int num_slots, int2* __restrict__ out)
+{
+  const int s = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (s >= num_slots) return;
+  int2 r = make_int2(0, 0);
+  if (ta.slot_dst[s] >= 0) {
+    const int b = ta.nodes[s] - ta.bnd_base;
+    r.x         = ta.bnd_ptr[b];
+    r.y         = ta.bnd_ptr[b + 1] - r.x;
+  }
+  out[s] = r;
+}
+
+void launch_slot_partials(const TileArgs& ta, int num_slots, int2* out, hipStream_t s)
+{
+  if (num_slots <= 0) return;
+  hipLaunchKernelGGL(k_slot_partials, dim3((unsigned)((num_slots + 255) / 256)), dim3(256), 0, s, ta, num_slots, out);
+}
+
+void launch_joint_element_tiled(const JointTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,
+                                float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s)
+{
+  if (work.t_count <= 0) return;
+  launch_grid(work, work.reaction_groups + (unsigned)work.t_count, ta, X, na, Fip, sip, rx, status, s, LaunchTimer{});
 }
 
 void launch_uq_element_tiled(const UqTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,

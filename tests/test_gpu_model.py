@@ -458,19 +458,21 @@ def test_node_fields_of_every_copy_size(hip_device, num_nodes):
 
 
 @pytest.mark.parametrize("n,scattered", [(1, False), (3, True), (7, False), (9, True)])
-def test_joint_steps_match_separate_launches(hip_device, n, scattered):
-    """A small FP64 model advances in one launch per step; with kernel timing
+@pytest.mark.parametrize("precision,tile", [("fp64", 0), ("mixed", 64), ("mixed", 512)])
+def test_joint_steps_match_separate_launches(hip_device, monkeypatch, precision, tile, n, scattered):
+    """A small model advances in one launch per step; with kernel timing
     enabled it takes the element and the node launch: every field and the
     reaction history are the same bits, whatever number of steps a call
     takes, with conditions of every kind, output steps, two blocks and
     reaction nodes in every node tile."""
+    monkeypatch.setenv("NSM_TILE_ELEMS", str(tile or "auto"))
     mats = [N.problems.STEEL, N.problems.ALUMINIUM] if n > 1 else [N.problems.STEEL]
     prob = N.CubeProblem(n=n, materials=mats, num_steps=20, name="joint").build()
     nodes = np.arange(0, prob.num_nodes, 3, dtype=np.int32) if scattered else prob.top
     u0 = 1e-3 * np.sin(3 * prob.X) * prob.X[:, 2:3]
     got = []
     for separate in (False, True):
-        m = prob.make_model("fp64")
+        m = prob.make_model(precision)
         m.AddBoundaryCondition("prescribed_displacement", prob.top[:5], 1, 1e-5)
         m.AddBoundaryCondition("initial_velocity", prob.top, 0, 2.0)
         m.SetReactionNodes(nodes, 1)
