@@ -41,7 +41,10 @@ __device__ __forceinline__ double refined_rcp(double d)
   return __builtin_fma(r, t, r);
 }
 
-// n / d given r = refined_rcp(d), for operands that pass plain_operand
+// whether ok holds in every active lane of the wave: uniform
+__device__ __forceinline__ bool whole_wave(bool ok) { return __ballot(!ok) == 0; }
+
+// n / d given r = refined_rcp(d), for operands that pass divide_by's test
 __device__ __forceinline__ double div_shared(double n, double d, double r)
 {
   const double q = n * r;
@@ -49,21 +52,21 @@ __device__ __forceinline__ double div_shared(double n, double d, double r)
   return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(e, r, q, false), d, n);
 }
 
-// zero, infinite, NaN, or |x| in [2^-300, 2^300) (frexp exponent of
-// zero, infinity and NaN is 0)
-__device__ __forceinline__ bool plain_operand(double x)
-{
-  return (unsigned)(__builtin_amdgcn_frexp_exp(x) + 299) < 600u;
-}
-
-// q[i] = n[i] / d for i < kN, bit for bit as kN separate divisions
+// q[i] = n[i] / d for i < kN, bit for bit as kN separate divisions: shared
+// where every operand is zero, infinite, NaN or of magnitude in
+// [2^-300, 2^300) (the frexp exponent of the first three is 0), from the least
+// and the largest exponent
 template <int kN>
 __device__ __forceinline__ void divide_by(const double (&n)[kN], double d, double (&q)[kN])
 {
-  bool plain = plain_operand(d);
+  int lo = __builtin_amdgcn_frexp_exp(d), hi = lo;
 #pragma unroll
-  for (int i = 0; i < kN; i++) plain = plain && plain_operand(n[i]);
-  if (__builtin_expect(__ballot(!plain) == 0, 1)) {  // uniform across the wave
+  for (int i = 0; i < kN; i++) {
+    const int e = __builtin_amdgcn_frexp_exp(n[i]);
+    lo          = min(lo, e);
+    hi          = max(hi, e);
+  }
+  if (__builtin_expect(whole_wave((lo >= -299) & (hi <= 300)), 1)) {
     const double r = refined_rcp(d);
 #pragma unroll
     for (int i = 0; i < kN; i++) q[i] = div_shared(n[i], d, r);
@@ -71,6 +74,86 @@ __device__ __forceinline__ void divide_by(const double (&n)[kN], double d, doubl
 #pragma unroll
     for (int i = 0; i < kN; i++) q[i] = n[i] / d;
   }
+}
+
+// ---------------------------------------------------------------------------
+// Quotients and roots of operands of ordinary size.  For d (and n) far from
+// the ends of the range, finite and not zero, the scale steps and div_fixup
+// of a division change nothing, and neither do those of a square root,
+//   s = x scaled, r = rsq(s), g = s r, h = r / 2, e = fma(-h, g, 1/2),
+//   g = fma(g, e, g), h = fma(h, e, h), twice g = fma(fma(-g, g, s), h, g),
+//   g unscaled, s itself where it is zero or infinite:
+// left out, the same operations on the same values remain and give the same
+// bits.  8 of 11 instructions of a quotient (7 of a reciprocal) and 10 of 18
+// of a root stay; testing operands takes two each, or four for three.  A
+// wave that holds another operand takes the full sequence.  The kernels here
+// are bound by issuing vector instructions: stresses of 500 009 elements'
+// points 128.6 -> 113.9 us.
+// ---------------------------------------------------------------------------
+
+// x positive, in [2^-700, 2^700): its high word, sign and exponent, in a range
+constexpr uint32_t kPlainLo = (1023u - 700u) << 20, kPlainHi = (1023u + 700u) << 20;
+
+__device__ __forceinline__ uint32_t high_word(double x)
+{
+  return (uint32_t)(__builtin_bit_cast(uint64_t, x) >> 32);
+}
+
+__device__ __forceinline__ bool plain(double x) { return high_word(x) - kPlainLo < kPlainHi - kPlainLo; }
+
+__device__ __forceinline__ bool plain3(double x, double y, double z)
+{
+  const uint32_t lo = min(min(high_word(x), high_word(y)), high_word(z));
+  const uint32_t hi = max(max(high_word(x), high_word(y)), high_word(z));
+  return (lo >= kPlainLo) & (hi < kPlainHi);
+}
+
+// n / d for |d| plain and |n| within [2^-300, 2^300], or |n| plain and d near 1
+__device__ __forceinline__ double div_plain(double n, double d)
+{
+  const double r = refined_rcp(d);
+  const double q = n * r;
+  return __builtin_fma(__builtin_fma(-d, q, n), r, q);
+}
+
+// 1 / d for |d| plain
+__device__ __forceinline__ double rcp_plain(double d)
+{
+  const double r = refined_rcp(d);
+  return __builtin_fma(__builtin_fma(-d, r, 1.0), r, r);
+}
+
+// x / 3 for x plain: 1/3 to nearest is a constant; the quotient from it and
+// one residual is the correctly rounded one (Markstein, IBM J. Res. Dev. 34,
+// 1990), which the division's is too
+__device__ __forceinline__ double third_plain(double x)
+{
+  constexpr double r = 1.0 / 3.0;
+  const double     q = x * r;
+  return __builtin_fma(__builtin_fma(-3.0, q, x), r, q);
+}
+
+__device__ __forceinline__ double third(double x)
+{
+  return __builtin_expect(whole_wave(plain(x)), 1) ? third_plain(x) : x / 3.0;
+}
+
+__device__ __forceinline__ double reciprocal(double d)
+{
+  return __builtin_expect(whole_wave(plain(d)), 1) ? rcp_plain(d) : 1.0 / d;
+}
+
+// sqrt(x) for x plain
+__device__ __forceinline__ double sqrt_plain(double x)
+{
+  const double r = __builtin_amdgcn_rsq(x);
+  double       g = x * r;
+  double       h = r * 0.5;
+  const double e = __builtin_fma(-h, g, 0.5);
+  g              = __builtin_fma(g, e, g);
+  h              = __builtin_fma(h, e, h);
+  g              = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
 }
 
 // Invert3x3 on a row-major 3x3 (src/nimble_utils.h:1229-1268); returns det.
@@ -140,11 +223,15 @@ __device__ __forceinline__ double invert_full33(const double* a, double* inv)
 // arguments near 1 are 1-3 ulp off), and NimbleSM's stress calls it
 // (src/nimble_material.cc:274), so the parity path evaluates the same steps
 // with the same constants to reproduce the reference's FP64 bits.
+// kPlain: x is plain, and one reduction serves |x| = x.  A wave whose
+// arguments are all in [0.5, 2) (a volume ratio's) takes the remainder and
+// the quotient of xe by 3 from xe = 0 or 1 directly.
+template <bool kPlain>
 __device__ __forceinline__ double cbrt_ref(double x)
 {
-  if (x == 0.0 || isnan(x) || isinf(x)) return x + x;
-  int          xe;
-  const double xm = frexp(fabs(x), &xe);
+  if (!kPlain && (x == 0.0 || isnan(x) || isinf(x))) return x + x;
+  const int    xe = __builtin_amdgcn_frexp_exp(x);
+  const double xm = __builtin_amdgcn_frexp_mant(kPlain ? x : fabs(x));
   const double u  = (0.354895765043919860 +
                     ((1.50819193781584896 +
                       ((-2.11499494167371287 +
@@ -156,9 +243,12 @@ __device__ __forceinline__ double cbrt_ref(double x)
   const double t2  = u * u * u;
   const double cb2 = 1.2599210498948731648;   // 2^(1/3)
   const double sq2 = 1.5874010519681994748;   // 2^(2/3)
+  // numerator and denominator within [0.1, 10]
+  const double y   = div_plain(u * (t2 + 2.0 * xm), 2.0 * t2 + xm);
+  if (kPlain && __builtin_expect(whole_wave((unsigned)xe < 2u), 1)) return y * (xe == 0 ? 1.0 : cb2);
   const int    r   = xe % 3;                  // C remainder: -2..2
   const double fac = r == -2 ? 1.0 / sq2 : r == -1 ? 1.0 / cb2 : r == 0 ? 1.0 : r == 1 ? cb2 : sq2;
-  const double ym  = u * (t2 + 2.0 * xm) / (2.0 * t2 + xm) * fac;
+  const double ym  = y * fac;
   return ldexp(x > 0.0 ? ym : -ym, xe / 3);
 }
 
@@ -182,7 +272,7 @@ __device__ __forceinline__ double cos_acos_div3(double x)
   const double den = 1.0 + 2.26376989330935617 * x +
                      ((1.80461009751278976 + 0.603976798217196003 * x) * x2 +
                       (0.0783255761115461708 + 0.00268525944538021629 * x) * x4);
-  return num / den;
+  return div_plain(num, den);  // both within [0.8, 6]
 }
 
 // Closed-form eigen-decomposition of a symmetric 3x3 with column-pivoted QR
@@ -193,7 +283,7 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
   double       cxx = t[S_XX], cyy = t[S_YY], czz = t[S_ZZ];
   const double cxy = t[S_XY], cyz = t[S_YZ], czx = t[S_ZX];
 
-  const double c1 = (cxx + cyy + czz) / 3.0;
+  const double c1 = third(cxx + cyy + czz);
   cxx -= c1;
   cyy -= c1;
   czz -= c1;
@@ -205,8 +295,17 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
 
   const double c2 = cxx_cyy + cyy * czz + czz * cxx - cxy_cxy - cyz_cyz - czx_czx;
 
-  const double three_over_a      = -3.0 / c2;
-  const double sqrt_three_over_a = sqrt(three_over_a);
+  // c2 of ordinary size: then so are -3 / c2 and its root, by which the
+  // cosine is divided below
+  const bool plain_c2          = whole_wave(plain(-c2));
+  double     three_over_a, sqrt_three_over_a;
+  if (__builtin_expect(plain_c2, 1)) {
+    three_over_a      = div_plain(-3.0, c2);
+    sqrt_three_over_a = sqrt_plain(three_over_a);
+  } else {
+    three_over_a      = -3.0 / c2;
+    sqrt_three_over_a = sqrt(three_over_a);
+  }
 
   const double c3 = cxx * cyz_cyz + cyy * czx_czx - 2.0 * cxy * cyz * czx + czz * (cxy_cxy - cxx_cyy);
   const double rr = -0.5 * c3 * three_over_a * sqrt_three_over_a;
@@ -215,7 +314,11 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
   const double cth  = cos_acos_div3(arg);
   const double tcth = 2.0 * mult_sign(cth, rr);
 
-  double eval2 = tcth / sqrt_three_over_a;
+  double eval2;
+  if (__builtin_expect(plain_c2, 1))
+    eval2 = div_plain(tcth, sqrt_three_over_a);
+  else
+    eval2 = tcth / sqrt_three_over_a;
 
   const double r0[3] = {cxx - eval2, cxy, czx};
   const double r1[3] = {cxy, cyy - eval2, cyz};
@@ -239,7 +342,7 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
   for (int i = 0; i < 3; i++) ra[i] = k0l ? r1[i] : r0[i];
   for (int i = 0; i < 3; i++) rb[i] = k2l ? r1[i] : r2[i];
 
-  const double ki_ki = 1.0 / (k0l ? k0 : k1l ? k1 : k2);  // k0, k1, k2: sums of squares, never -0.0
+  const double ki_ki = reciprocal(k0l ? k0 : k1l ? k1 : k2);  // k0, k1, k2: sums of squares, never -0.0
 
   const double ki_dpr1 = ki_ki * (kr[0] * ra[0] + kr[1] * ra[1] + kr[2] * ra[2]);
   const double ki_dpr2 = ki_ki * (kr[0] * rb[0] + kr[1] * rb[1] + kr[2] * rb[2]);
@@ -252,7 +355,7 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
   const bool a0lea1 = a0 <= a1;
   double     ar[3];
   for (int i = 0; i < 3; i++) ar[i] = a0lea1 ? rb[i] : ra[i];
-  const double ai_ai = 1.0 / (a0lea1 ? a1 : a0);
+  const double ai_ai = reciprocal(a0lea1 ? a1 : a0);
 
   e2[0] = kr[1] * ar[2] - kr[2] * ar[1];
   e2[1] = kr[2] * ar[0] - kr[0] * ar[2];
@@ -272,7 +375,8 @@ __device__ __forceinline__ void eigen_sym33(const double t[6], double ev[3], dou
 
   // Wilkinson shift
   const double b     = 0.5 * (rm2xx - rm2yy);
-  const double sterm = mult_sign(sqrt(b * b + rm2xy_rm2xy), b);
+  const double bb    = b * b + rm2xy_rm2xy;
+  const double sterm = mult_sign(__builtin_expect(whole_wave(plain(bb)), 1) ? sqrt_plain(bb) : sqrt(bb), b);
   double       eval0 = rm2yy + b - sterm;
   double       eval1 = rm2xx + rm2yy - eval0;
 
@@ -344,9 +448,25 @@ __device__ __forceinline__ void left_stretch(const double* F, double V[6])
   const double l2 = v2[0] * v2[0] + v2[1] * v2[1] + v2[2] * v2[2];
   const double l3 = v3[0] * v3[0] + v3[1] * v3[1] + v3[2] * v3[2];
 
-  const double xi = 1.0 / (sqrt(ev[0]) * l1);
-  const double yi = 1.0 / (sqrt(ev[1]) * l2);
-  const double zi = 1.0 / (sqrt(ev[2]) * l3);
+  double xi, yi, zi;
+  if (__builtin_expect(whole_wave(plain3(ev[0], ev[1], ev[2])), 1)) {
+    xi = sqrt_plain(ev[0]) * l1;
+    yi = sqrt_plain(ev[1]) * l2;
+    zi = sqrt_plain(ev[2]) * l3;
+  } else {
+    xi = sqrt(ev[0]) * l1;
+    yi = sqrt(ev[1]) * l2;
+    zi = sqrt(ev[2]) * l3;
+  }
+  if (__builtin_expect(whole_wave(plain3(xi, yi, zi)), 1)) {
+    xi = rcp_plain(xi);
+    yi = rcp_plain(yi);
+    zi = rcp_plain(zi);
+  } else {
+    xi = 1.0 / xi;
+    yi = 1.0 / yi;
+    zi = 1.0 / zi;
+  }
 
   V[S_XX] = xi * v1[0] * v1[0] + yi * v2[0] * v2[0] + zi * v3[0] * v3[0];
   V[S_YY] = xi * v1[1] * v1[1] + yi * v2[1] * v2[1] + zi * v3[1] * v3[1];
@@ -365,8 +485,14 @@ __device__ __forceinline__ void neohookean_stress(double K, double G, const doub
   const double xj = v[S_XX] * v[S_YY] * v[S_ZZ] + 2.0 * v[S_XY] * v[S_YZ] * v[S_ZX] - v[S_XX] * v[S_YZ] * v[S_YZ] -
                     v[S_YY] * v[S_ZX] * v[S_ZX] - v[S_ZZ] * v[S_XY] * v[S_XY];
 
-  const double cj  = cbrt_ref(xj);
-  const double fac = 1.0 / (cj * cj);
+  double fac;
+  if (__builtin_expect(whole_wave(plain(xj)), 1)) {
+    const double cj = cbrt_ref<true>(xj);
+    fac             = rcp_plain(cj * cj);
+  } else {
+    const double cj = cbrt_ref<false>(xj);
+    fac             = 1.0 / (cj * cj);
+  }
 
   double bxx = v[S_XX] * v[S_XX] + v[S_XY] * v[S_XY] + v[S_ZX] * v[S_ZX];
   double byy = v[S_XY] * v[S_XY] + v[S_YY] * v[S_YY] + v[S_YZ] * v[S_YZ];
@@ -383,9 +509,10 @@ __device__ __forceinline__ void neohookean_stress(double K, double G, const doub
   bzx = fac * bzx;
 
   const double trace = bxx + byy + bzz;
-  bxx = bxx - trace / 3.0;
-  byy = byy - trace / 3.0;
-  bzz = bzz - trace / 3.0;
+  const double mean  = third(trace);
+  bxx = bxx - mean;
+  byy = byy - mean;
+  bzz = bzz - mean;
 
   // 1/xj of the pressure and the six quotients of the deviator share xj
   const double n[7] = {1.0, G * bxx, G * byy, G * bzz, G * bxy, G * byz, G * bzx};

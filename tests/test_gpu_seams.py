@@ -244,3 +244,38 @@ def test_seams_at_the_edges_of_a_wavefront(hip_device, elems, E):
             call(_dev(X, hip_device))
         assert ei.value.status == 3
         call(Xd)
+
+
+@pytest.mark.parametrize("run", [1, 3, 64, 200])
+def test_ordinary_and_special_operands_share_waves(hip_device, elems, run):
+    """Quotients and roots leave the scale and fix-up steps out where every
+    lane of a wave holds operands of ordinary size.  Points of each kind --
+    general, undeformed, rotated only, nearly undeformed, with two equal
+    stretches, with volume ratios outside [0.5, 2), with very large, very
+    small, zero, infinite and NaN entries -- in runs of one, three, a wave
+    and more: the oracle's bits each (NaN where it has NaN)."""
+    import torch
+
+    rng = np.random.default_rng(7)
+    rot = np.linalg.qr(rng.standard_normal((3, 3)))[0]
+    rot *= np.linalg.det(rot)
+    ravel = lambda m: np.array([m[i][j] for i, j in  # noqa: E731
+                                [(0, 0), (1, 1), (2, 2), (0, 1), (1, 2), (2, 0), (1, 0), (2, 1), (0, 2)]])
+    eye = np.eye(3)
+    noise = rng.standard_normal((3, 3))
+    special = [eye, rot, eye + 1e-9 * noise, eye + 1e-15 * noise, eye + 1e-30 * noise, np.diag([1.1, 1.1, 0.9]),
+               np.diag([1.0, 1.0, 1.01]), rot @ np.diag([1.2, 1.2, 1.2]), 3.0 * (eye + 0.1 * noise),
+               0.3 * (eye + 0.1 * noise), 2.0 ** 240 * eye, 2.0 ** -240 * eye, 2.0 ** 120 * (eye + 0.1 * noise),
+               np.zeros((3, 3)), np.diag([1.0, 1.0, np.inf]), np.diag([1.0, np.nan, 1.0]), -eye]
+    general = O.deformation_gradients(*elems).reshape(-1, 9)[: 40 * run]
+    rows = []
+    for k in range(40):
+        rows += list(general[k * run:(k + 1) * run]) + [ravel(special[k % len(special)])] * run
+    F = np.array(rows)
+    F = F[: len(F) // 8 * 8].reshape(-1, 8, 9)
+    with np.errstate(all="ignore"):
+        want = O.stress(1.6e11, 0.8e11, F)
+    s = torch.zeros(want.shape, dtype=torch.float64, device=hip_device)
+    N.NeohookeanMaterial(7800.0, 1.6e11, 0.8e11).GetStress(_dev(F, hip_device), s)
+    torch.cuda.synchronize()
+    assert np.array_equal(s.cpu().numpy(), want, equal_nan=True)
