@@ -843,10 +843,23 @@ int setup_tiles(nsm_model* md)
   if ((st = dalloc(&partials, std::max<size_t>(3 * ts.bnd_ent.size(), 1), &md->device_bytes))) return st;
   md->tile_bufs.push_back((void*)partials);
   ta.partials = partials;
-  // Steps in one launch: one workgroup per tile, all of them on the device at
-  // once (larger models need the persistent kernel's prefetch), shared nodes that a second launch would wait for,
-  // each of them in some tile.
-  md->joint_ok = md->num_blocks <= nsm::kMaxLaunchBlocks && ts.num_tiles <= ta.resident_groups && ta.num_bnd > 0;
+  // Steps in one launch, one workgroup per tile: shared nodes that a second
+  // launch would wait for, each of them in some tile, and
+  // either all tiles on the device at once, or a few windows of them of which
+  // the persistent kernel's last one is at most 7/10 full.  Its workgroups
+  // take equally many tiles each, so it then waits for the few that have one
+  // more; near a full window its prefetch wins, and so it does with
+  // 512-element tiles (one workgroup per CU, nothing else to run during its
+  // loads) and where redundant shared-node updates add up.  us per step, two
+  // launches / one, 128-element tiles (1024 at once): 1.07 windows 36.9 /
+  // 30.1, 1.65 42.8 / 40.1, 1.82 49.1 / 48.9, 2.0 42.0 / 46.2, 2.2 55.0 /
+  // 49.2, 4.2 88.0 / 82.1; 256: 1.07 38.4 / 30.8, 1.65 40.5 / 39.5, 1.91
+  // 44.9 / 48.3, 3.1 71.2 / 63.7, 4.2 88.9 / 87.4, 4.85 88.7 / 89.8; 512: 2.4
+  // 59.2 / 60.1, 3.1 70.9 / 76.6.
+  const int64_t tiles = ts.num_tiles, window = ta.resident_groups;
+  const bool    few   = tiles <= window || (ts.tile_elems < 512 && tiles <= 5 * window && tiles % window != 0 &&
+                                          10 * (tiles % window) <= 7 * window);
+  md->joint_ok        = md->num_blocks <= nsm::kMaxLaunchBlocks && few && ta.num_bnd > 0;
   for (int b = 0; b < ta.num_bnd && md->joint_ok; b++)
     md->joint_ok = ts.bnd_ptr[(size_t)b + 1] > ts.bnd_ptr[(size_t)b];
   md->blk_tile_off.assign((size_t)md->num_blocks + 1, 0);
@@ -876,7 +889,7 @@ bool is_output(int64_t step, int64_t num_load_steps, int64_t output_frequency)
   return step % output_frequency == 0 || step == num_load_steps - 1;
 }
 
-// Whether this call's steps run in one launch each (kernel timing asks for the
+// Whether this call's steps may run in one launch each (kernel timing asks for the
 // element and the node launch, and UQ samples need the separate ones).
 bool joint_steps(const nsm_model* md)
 {
@@ -1878,8 +1891,15 @@ int nsm_model_explicit_steps(nsm_model* md, int64_t step_begin, int64_t step_end
   // small models: all steps in joint launches but the first of an even number
   int64_t joint_from = step_end;
   if (joint_steps(md) && step_end - step_begin >= 3) {
-    if ((st = ensure_joint(md))) return st;
-    joint_from = step_begin + ((step_end - step_begin + 1) & 1);
+    st = ensure_joint(md);
+    if (st == NSM_ERR_NOMEM) {  // no memory for the second buffers: separate launches
+      (void)hipGetLastError();
+      md->joint_ok = false;
+    } else if (st) {
+      return st;
+    } else {
+      joint_from = step_begin + ((step_end - step_begin + 1) & 1);
+    }
   }
   for (int64_t step = step_begin; step < step_end; step++) {
     if (step == joint_from) {

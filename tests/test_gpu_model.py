@@ -457,8 +457,11 @@ def test_node_fields_of_every_copy_size(hip_device, num_nodes):
         models[k].close()
 
 
-@pytest.mark.parametrize("n,scattered", [(1, False), (3, True), (7, False), (9, True)])
-@pytest.mark.parametrize("precision,tile", [("fp64", 0), ("mixed", 64), ("mixed", 512)])
+@pytest.mark.parametrize("precision,tile,n,scattered",
+                         [(p, t, n, s) for p, t in [("fp64", 0), ("mixed", 64), ("mixed", 512)]
+                          for n, s in [(1, False), (3, True), (7, False), (9, True)]]
+                         # more tiles than the device holds at once
+                         + [("mixed", 64, 49, True), ("mixed", 128, 66, False)])
 def test_joint_steps_match_separate_launches(hip_device, monkeypatch, precision, tile, n, scattered):
     """A small model advances in one launch per step; with kernel timing
     enabled it takes the element and the node launch: every field and the
