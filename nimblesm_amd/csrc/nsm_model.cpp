@@ -844,21 +844,18 @@ int setup_tiles(nsm_model* md)
   md->tile_bufs.push_back((void*)partials);
   ta.partials = partials;
   // Steps in one launch, one workgroup per tile: shared nodes that a second
-  // launch would wait for, each of them in some tile, and
-  // either all tiles on the device at once, or a few windows of them of which
-  // the persistent kernel's last one is at most 7/10 full.  Its workgroups
-  // take equally many tiles each, so it then waits for the few that have one
-  // more; near a full window its prefetch wins, and so it does with
-  // 512-element tiles (one workgroup per CU, nothing else to run during its
-  // loads) and where redundant shared-node updates add up.  us per step, two
-  // launches / one, 128-element tiles (1024 at once): 1.07 windows 36.9 /
-  // 30.1, 1.65 42.8 / 40.1, 1.82 49.1 / 48.9, 2.0 42.0 / 46.2, 2.2 55.0 /
-  // 49.2, 4.2 88.0 / 82.1; 256: 1.07 38.4 / 30.8, 1.65 40.5 / 39.5, 1.91
-  // 44.9 / 48.3, 3.1 71.2 / 63.7, 4.2 88.9 / 87.4, 4.85 88.7 / 89.8; 512: 2.4
-  // 59.2 / 60.1, 3.1 70.9 / 76.6.
+  // launch would wait for, each of them in some tile, and all tiles on the
+  // device at once, or a few windows of them with a last one that a
+  // persistent grid would fill too little.  Tiles update the shared nodes
+  // they read each for themselves, which adds up with more windows.  us per
+  // step, persistent / one workgroup per tile / the same and one launch:
+  // 128-element tiles 1.07 windows 36.2 / 31.6 / 30.1, 1.65 42.8 / 41.2 /
+  // 40.1, 2.2 54.8 / 50.4 / 49.2, 2.4 55.3 / 51.1 / 51.7, 4.2 88.0 / 79.7 /
+  // 82.1; 256: 1.07 37.7 / 32.4 / 30.8, 2.4 56.2 / 51.4 / 50.4, 4.2 89.9 /
+  // 84.0 / 87.4.
   const int64_t tiles = ts.num_tiles, window = ta.resident_groups;
-  const bool    few   = tiles <= window || (ts.tile_elems < 512 && tiles <= 5 * window && tiles % window != 0 &&
-                                          10 * (tiles % window) <= 7 * window);
+  const bool    few =
+      tiles <= window || (2 * tiles <= 5 * window && nsm::last_window_partial(tiles, ta, 7));
   md->joint_ok        = md->num_blocks <= nsm::kMaxLaunchBlocks && few && ta.num_bnd > 0;
   for (int b = 0; b < ta.num_bnd && md->joint_ok; b++)
     md->joint_ok = ts.bnd_ptr[(size_t)b + 1] > ts.bnd_ptr[(size_t)b];

@@ -119,6 +119,9 @@ struct UqTileWork {
 // boundary nodes per workgroup of the boundary kernel (one per thread)
 constexpr int kBoundaryNodesPerGroup = 256;
 unsigned      boundary_grid(int num_bnd);
+// whether windows of all resident workgroups leave a last one of the items
+// that is filled to at most tenths / 10
+bool          last_window_partial(int64_t items, const TileArgs& ta, int tenths);
 
 // Tiles [t_begin, t_begin + t_count) (all inside the blocks of bt): element
 // arithmetic, force assembly in LDS, the step of the tile-interior nodes,

@@ -137,16 +137,34 @@ __device__ __forceinline__ ElemData load_elem(const TileArgs& ta, int t)
 // the writes and for the gathers of neighbouring slots), so a slot sums its
 // at most 8 contributions in ascending corner order after one barrier.
 // Column kThreads of ef is zero (absent corners read it); staging a gather
-// tile rewrites it, since a colour tile's accumulators overlap it.
+// tile rewrites it, since a colour tile's accumulators overlap it.  kLean: a
+// slot's elements take the place of its X once every element has read that
+// (NodeRow).
 constexpr uint16_t kNoElement = 0xffff;
-template <int kThreads>
+template <int kThreads, bool kLean>
 union Assembly {
   double acc[2 * kThreads][3];
   struct {
-    uint16_t inv[2 * kThreads][8];
+    uint16_t inv[kLean ? 1 : 2 * kThreads][8];
     float    ef[24][kThreads + 1];
   } g;
 };
+
+// X and u of a node slot side by side (48 bytes): an element reads each of
+// its nodes with three 16-byte LDS reads
+union NodeRow {
+  double   xu[6];
+  uint16_t inv[8];
+};
+
+template <int kThreads, bool kLean>
+__device__ __forceinline__ uint16_t* slot_elements(NodeRow* rows, Assembly<kThreads, kLean>& as, int ln)
+{
+  if constexpr (kLean)
+    return rows[ln].inv;
+  else
+    return as.g.inv[ln];
+}
 
 // Staging of one tile: its nodes' X and u into LDS, cleared assembly slots,
 // and the loads of its interior nodes' flags (and v, m when the step updates
@@ -157,10 +175,24 @@ struct NodeState {
   double v[2][3], m[2];
 };
 
-template <int kThreads>
+__device__ __forceinline__ void load_node_state(const SlotIds& ids, int x_delta, const NodeArrays& na, int update_v,
+                                                NodeState& ns)
+{
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+    if (ids.dst[k] == kInterior) {
+      ns.flg[k] = na.flags[ids.gid[k] + x_delta];
+      if (update_v) {
+        load3(na.v, ids.gid[k], ns.v[k]);
+        ns.m[k] = na.mass[ids.gid[k]];
+      }
+    }
+}
+
+template <int kThreads, bool kLean>
 __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const double (&xr)[2][3],
                                       const double (&ur)[2][3], const NodeArrays& na, int update_v,
-                                      double (*sxu)[6], Assembly<kThreads>& as, bool gather, NodeState& ns,
+                                      NodeRow* rows, Assembly<kThreads, kLean>& as, bool gather, NodeState& ns,
                                       bool load_state = true)
 {
   if (gather && threadIdx.x < 24) as.g.ef[threadIdx.x][kThreads] = 0.0f;
@@ -170,23 +202,17 @@ __device__ __forceinline__ void stage(const SlotIds& ids, int x_delta, const dou
     if (ids.dst[k] != kAbsent) {
 #pragma unroll
       for (int c = 0; c < 3; c++) {
-        sxu[ln][c]     = xr[k][c];
-        sxu[ln][3 + c] = ur[k][c];
+        rows[ln].xu[c]     = xr[k][c];
+        rows[ln].xu[3 + c] = ur[k][c];
       }
-      if (gather)
-        *reinterpret_cast<uint4*>(as.g.inv[ln]) = make_uint4(~0u, ~0u, ~0u, ~0u);
-      else
+      if (!gather)
 #pragma unroll
         for (int c = 0; c < 3; c++) as.acc[ln][c] = 0.0;
-    }
-    if (load_state && ids.dst[k] == kInterior) {
-      ns.flg[k] = na.flags[ids.gid[k] + x_delta];
-      if (update_v) {
-        load3(na.v, ids.gid[k], ns.v[k]);
-        ns.m[k] = na.mass[ids.gid[k]];
-      }
+      else if (!kLean)
+        *reinterpret_cast<uint4*>(as.g.inv[ln]) = make_uint4(~0u, ~0u, ~0u, ~0u);
     }
   }
+  if (load_state) load_node_state(ids, x_delta, na, update_v, ns);
 }
 
 // ---- the two kinds of element-launch work (nsm_tiled.h) ----
@@ -435,7 +461,8 @@ __device__ __forceinline__ void joint_nodes(const JointTileWork& w, const TileAr
   }
 }
 
-// Persistent workgroups, each walking every G-th tile.  kThreads elements
+// Persistent workgroups, each walking every G-th tile, or (kOne) a workgroup
+// per work item, which loads nothing ahead.  kThreads elements
 // and at most 2*kThreads nodes per tile.  While tile t computes, X, u and
 // element data of its next tile and node ids of the one after are in flight;
 // the next tile is staged into LDS at the end of the iteration.
@@ -450,8 +477,20 @@ __device__ __forceinline__ void joint_nodes(const JointTileWork& w, const TileAr
 // pair has and spills.  The launch bound
 // holds the kernel to two waves per SIMD (at most 256 registers): left free,
 // the scheduler takes more for the gather assembly and halves occupancy.
-template <int kThreads, bool kStoreIp, typename Work>
-__global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, TileArgs ta,
+//
+// kLeanTiles: ensembles with a workgroup per item run three waves per SIMD,
+// in 168 registers and a third less LDS: no next item in registers, the
+// nodes' state loaded after the element arithmetic, the slots' elements where
+// their X was.  With no element data to store the arithmetic's issue bounds
+// them, and a third wave fills what two left idle: 64 meshes of 32^3 elements
+// 8.56 -> 6.72 ms per 40 steps, 128 of 24^3 in 64-element tiles 8.94 -> 5.91.
+// Kernels that store element data gain nothing from it (52^3 elements,
+// 128-element tiles, 29.9 / 29.5 us, 74^3 63.4 / 69.8, 16 windows 314 / 374).
+template <int kThreads, bool kOne, typename Work>
+constexpr bool kLeanTiles = kOne && kThreads < 512 && std::is_same<Work, EnsTileWork>::value;
+
+template <int kThreads, bool kStoreIp, bool kOne, typename Work>
+__global__ __launch_bounds__(kThreads, (kLeanTiles<kThreads, kOne, Work> ? 3 : 2)) void k_element_tiled(const Work work, TileArgs ta,
                                                             const double* __restrict__ X, NodeArrays na,
                                                             float* __restrict__ Fip, float* __restrict__ sip,
                                                             ReactionArgs rx, int* __restrict__ status)
@@ -459,17 +498,17 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
   constexpr int  kNodes      = 2 * kThreads;
   constexpr bool kEnsemble   = std::is_same<Work, EnsTileWork>::value;
   constexpr bool kUq         = std::is_same<Work, UqTileWork>::value;
-  constexpr bool kJoint      = std::is_same<Work, JointTileWork>::value;  // one item per workgroup, no prefetch
+  constexpr bool kJoint      = std::is_same<Work, JointTileWork>::value;
+  static_assert(!kJoint || kOne, "a joint step's grid holds every tile");
   // ensembles stage each tile's sample's kinematic-condition entries (one
   // 8-byte word per thread)
   constexpr int  kTileBcWords = kBcWords * kEnsMaxBcCodes;
   static_assert(!kEnsemble || kTileBcWords <= kThreads, "one condition word per thread");
-  // X and u of a node slot side by side (48 bytes): an element reads each
-  // of its nodes with three 16-byte LDS reads
-  __shared__ __attribute__((aligned(16))) double sxu[kNodes][6];
-  __shared__ __attribute__((aligned(16))) Assembly<kThreads> as;
+  constexpr bool kLean       = kLeanTiles<kThreads, kOne, Work>;
+  __shared__ __attribute__((aligned(16))) NodeRow rows[kNodes];
+  __shared__ __attribute__((aligned(16))) Assembly<kThreads, kLean> as;
   __shared__ double  red[kThreads / 64];
-  __shared__ BcEntry sbc[kMaxBcEntries];
+  __shared__ BcEntry sbc[kEnsemble ? kEnsMaxBcCodes : kMaxBcEntries];
   __shared__ int     bad;
   __shared__ double  fold_red[256];
 
@@ -519,7 +558,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
   ElemData  cur = load_elem<kThreads>(ta, c_first.t);
   NodeState ns;
   SlotIds   ids_next{};
-  if (!kJoint) ids_next = load_ids<kThreads>(ta, tile_ctx(work, next(ib)));
+  if (!kOne) ids_next = load_ids<kThreads>(ta, tile_ctx(work, next(ib)));
   double  xr[2][3], ur[2][3];
 #pragma unroll
   for (int k = 0; k < 2; k++) {
@@ -527,8 +566,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     if (!kJoint) load3(work_arrays(work, c_first, na).u, ids.gid[k], ur[k]);
   }
   if constexpr (kJoint) joint_nodes<kThreads>(work, ta, c_first, ids, na, sbc, ur, ns);
-  stage<kThreads>(ids, c_first.x_delta, xr, ur, work_arrays(work, c_first, na), update_v, sxu, as,
-                  tile_table(ta.gather, c_first.t) != 0, ns, !kJoint);
+  stage<kThreads, kLean>(ids, c_first.x_delta, xr, ur, work_arrays(work, c_first, na), update_v, rows, as,
+                  tile_table(ta.gather, c_first.t) != 0, ns, !kJoint && !kLean);
   // every prologue load complete (vmcnt(0); lgkmcnt and expcnt at their
   // maximum, gfx9 encoding): the loop's waits then depend on its body only
   __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -547,7 +586,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
     // ensembles) the next item's sample's condition entries
     ElemData el_next   = cur;
     SlotIds  ids_after = ids;
-    if (!kJoint) {
+    if (!kOne) {
 #pragma unroll
       for (int k = 0; k < 2; k++) {
         load3(X, ids_next.gid[k] + cn.x_delta, xr[k]);
@@ -557,7 +596,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       ids_after = load_ids<kThreads>(ta, tile_ctx(work, next(next(i))));
     }
     uint64_t       bc_next   = 0;
-    if (kEnsemble)
+    if (kEnsemble && !kOne)
       bc_next = reinterpret_cast<const uint64_t*>(work_bc(work) + cn.bc_base)[min(tid, kTileBcWords - 1)];
 
     // ---- element arithmetic (every thread; see load_elem)
@@ -579,8 +618,8 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       for (int j = 0; j < 8; j++)
 #pragma unroll
         for (int c = 0; c < 3; c++) {
-          Xe[j][c] = sxu[lc[j]][c];
-          ue[j][c] = sxu[lc[j]][3 + c];
+          Xe[j][c] = rows[lc[j]].xu[c];
+          ue[j][c] = rows[lc[j]].xu[3 + c];
         }
       float Kt, Gt;
       tile_moduli(work, c, e0, Kt, Gt);
@@ -619,14 +658,23 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       if (!mixed::element(Xe, ue, Kt, Gt, store, f)) bad = 1;
     }
 
+    if constexpr (kLean) load_node_state(ids, c.x_delta, work_arrays(work, c, na), update_v, ns);
+
     const bool gather = tile_table(ta.gather, t) != 0;  // uniform
     if (gather) {
       // ---- gather tiles: every element publishes its forces and, for each
       // corner j, itself as the slot's corner-j element (no other element of
       // the tile holds that slot at corner j)
+      if constexpr (kLean) {
+        __syncthreads();  // every element has read its nodes
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+          *reinterpret_cast<uint4*>(rows[tid + k * kThreads].inv) = make_uint4(~0u, ~0u, ~0u, ~0u);
+        __syncthreads();
+      }
       if (tid < ntl) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) as.g.inv[lc[j]][j] = (uint16_t)tid;
+        for (int j = 0; j < 8; j++) slot_elements<kThreads, kLean>(rows, as, lc[j])[j] = (uint16_t)tid;
 #pragma unroll
         for (int j = 0; j < 8; j++)
 #pragma unroll
@@ -672,7 +720,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       double fn[3];
       if (gather) {
         // the slot's contributions in ascending corner order, from 0.0
-        const uint4    iv   = *reinterpret_cast<const uint4*>(as.g.inv[ln]);
+        const uint4    iv   = *reinterpret_cast<const uint4*>(slot_elements<kThreads, kLean>(rows, as, ln));
         const unsigned wd[4] = {iv.x, iv.y, iv.z, iv.w};
         fn[0] = fn[1] = fn[2] = 0.0;
 #pragma unroll
@@ -688,7 +736,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       }
       if (ids.dst[k] == kInterior) {
         if (rx.coord >= 0 && (ns.flg[k] & kReactionFlag)) rxs += fn[rx.coord];
-        double un[3] = {sxu[ln][3], sxu[ln][4], sxu[ln][5]};
+        double un[3] = {rows[ln].xu[3], rows[ln].xu[4], rows[ln].xu[5]};
         node_update(nac, sbc, ids.gid[k], ns.flg[k], fn, un, ns.v[k], ns.m[k], sa);
       } else {
         float* const pp = ta.partials + 3 * (int64_t)ids.dst[k];
@@ -701,6 +749,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       const double s = block_sum<kThreads>(rxs, red);
       if (threadIdx.x == 0) rx.partials[tile_rx_slot(work, c, i)] = s;
     }
+    if (kOne) break;
     __syncthreads();  // tile t's LDS reads done
 
     // ---- stage the next item
@@ -711,7 +760,7 @@ __global__ __launch_bounds__(kThreads, 2) void k_element_tiled(const Work work, 
       if (kEnsemble && tid < kTileBcWords) reinterpret_cast<uint64_t*>(sbc)[tid] = bc_next;
       if (kUq && update_v && (c.s > 0) != (cn.s > 0))  // the next item's conditions (once per launch)
         for (int b = tid; b < na.num_bc; b += kThreads) sbc[b] = item_bc(work, cn, na)[b];
-      stage<kThreads>(ids, cn.x_delta, xr, ur, work_arrays(work, cn, na), update_v, sxu, as,
+      stage<kThreads, kLean>(ids, cn.x_delta, xr, ur, work_arrays(work, cn, na), update_v, rows, as,
                       tile_table(ta.gather, cn.t) != 0, ns);
     }
   }
@@ -885,31 +934,50 @@ __global__ __launch_bounds__(kBndThreads) void k_ens_boundary_update(TileArgs ta
 
 unsigned boundary_grid(int num_bnd) { return (unsigned)((num_bnd + kBndThreads - 1) / kBndThreads); }
 
-template <int kThreads, typename Work>
+template <int kThreads, bool kOne, typename Work>
 void launch_tiles(unsigned grid, const Work& work, const TileArgs& ta, const double* X, const NodeArrays& na,
                   float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t)
 {
-  // an off-nominal ensemble's launch always holds the nominal trajectory
-  constexpr bool kStores = std::is_same<Work, UqTileWork>::value || std::is_same<Work, JointTileWork>::value;
-  if (Fip || kStores) {
-    hipExtLaunchKernelGGL((k_element_tiled<kThreads, true, Work>), dim3(grid), dim3(kThreads), 0, s, t.start, t.stop,
-                          0, work, ta, X, na, Fip, sip, rx, status);
-  } else if constexpr (!kStores) {
-    hipExtLaunchKernelGGL((k_element_tiled<kThreads, false, Work>), dim3(grid), dim3(kThreads), 0, s, t.start,
-                          t.stop, 0, work, ta, X, na, Fip, sip, rx, status);
-  }
+  const auto launch = [&](auto kernel) {
+    hipExtLaunchKernelGGL(kernel, dim3(grid), dim3(kThreads), 0, s, t.start, t.stop, 0, work, ta, X, na, Fip, sip, rx,
+                          status);
+  };
+  // an off-nominal ensemble's launch always holds the nominal trajectory; a
+  // batched ensemble keeps no element data
+  if constexpr (std::is_same<Work, EnsTileWork>::value)
+    launch(k_element_tiled<kThreads, false, kOne, Work>);
+  else if (std::is_same<Work, UqTileWork>::value || std::is_same<Work, JointTileWork>::value || Fip)
+    launch(k_element_tiled<kThreads, true, kOne, Work>);
+  else if constexpr (std::is_same<Work, ModelTileWork>::value)
+    launch(k_element_tiled<kThreads, false, kOne, Work>);
 }
 
-template <typename Work>
+template <bool kOne, typename Work>
 void launch_grid(const Work& work, unsigned grid, const TileArgs& ta, const double* X, const NodeArrays& na,
                  float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t)
 {
   switch (ta.tile_elems) {
-    case 64: launch_tiles<64>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    case 128: launch_tiles<128>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    case 512: launch_tiles<512>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
-    default: launch_tiles<256>(grid, work, ta, X, na, Fip, sip, rx, status, s, t);
+    case 64: launch_tiles<64, kOne>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    case 128: launch_tiles<128, kOne>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    case 512: launch_tiles<512, kOne>(grid, work, ta, X, na, Fip, sip, rx, status, s, t); break;
+    default: launch_tiles<256, kOne>(grid, work, ta, X, na, Fip, sip, rx, status, s, t);
   }
+}
+
+// One workgroup per item where the last window of a persistent grid is little
+// filled.  The persistent workgroups take equally many items each, the next
+// one's loads behind the current one's arithmetic, and in the last window
+// most of them have run out; a workgroup per item starts as another ends, but
+// waits out its loads.  us per step, persistent / per item, models of
+// 256-element tiles (512 at once): 1.07 windows 37.7 / 32.4, 1.65 40.4 / 41.5,
+// 2.0 42.2 / 44.3, 3.1 69.9 / 64.7, 4.2 89.9 / 84.0.  512-element tiles fill a
+// CU with one workgroup, so nothing runs during those loads: 3.1 windows 70.5
+// / 73.6.  Ensembles' tiles (kLeanTiles) go one per workgroup at any number:
+// 1.7 windows 1597 / 1378 us per 40 steps, 5.0 3205 / 2701, 16.0 8580 / 6720.
+bool last_window_partial(int64_t items, const TileArgs& ta, int tenths)
+{
+  const int64_t window = std::max(ta.resident_groups, 1);
+  return ta.tile_elems < kTileElems && items % window != 0 && 10 * (items % window) <= tenths * window;
 }
 
 template <typename Work>
@@ -917,7 +985,12 @@ void launch_work(const Work& work, int count, const TileArgs& ta, const double* 
                  float* sip, ReactionArgs rx, int* status, hipStream_t s, const LaunchTimer& t = LaunchTimer{})
 {
   if (count <= 0) return complete_timer(t, s);
-  launch_grid(work, (unsigned)std::min(count, std::max(ta.resident_groups, 1)), ta, X, na, Fip, sip, rx, status, s, t);
+  const int window = std::max(ta.resident_groups, 1);
+  const bool each  = kLeanTiles<64, true, Work> && ta.tile_elems < kTileElems;
+  if (each || count <= window || last_window_partial(count, ta, 6))
+    launch_grid<true>(work, (unsigned)count, ta, X, na, Fip, sip, rx, status, s, t);
+  else
+    launch_grid<false>(work, (unsigned)window, ta, X, na, Fip, sip, rx, status, s, t);
 }
 
 void launch_element_tiled(const BlockTable<float>& bt, const TileArgs& ta, int t_begin, int t_count,
@@ -957,7 +1030,7 @@ void launch_joint_element_tiled(const JointTileWork& work, const TileArgs& ta, c
                                 float* Fip, float* sip, ReactionArgs rx, int* status, hipStream_t s)
 {
   if (work.t_count <= 0) return;
-  launch_grid(work, work.reaction_groups + (unsigned)work.t_count, ta, X, na, Fip, sip, rx, status, s, LaunchTimer{});
+  launch_grid<true>(work, work.reaction_groups + (unsigned)work.t_count, ta, X, na, Fip, sip, rx, status, s, LaunchTimer{});
 }
 
 void launch_uq_element_tiled(const UqTileWork& work, const TileArgs& ta, const double* X, const NodeArrays& na,
@@ -982,16 +1055,16 @@ int element_tiled_groups_per_cu(int tile_elems)
   int n = 0;
   switch (tile_elems) {
     case 64:
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<64, true, ModelTileWork>, 64, 0);
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<64, true, false, ModelTileWork>, 64, 0);
       break;
     case 128:
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<128, true, ModelTileWork>, 128, 0);
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<128, true, false, ModelTileWork>, 128, 0);
       break;
     case 512:
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<512, true, ModelTileWork>, 512, 0);
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<512, true, false, ModelTileWork>, 512, 0);
       break;
     default:
-      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<256, true, ModelTileWork>, 256, 0);
+      (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_element_tiled<256, true, false, ModelTileWork>, 256, 0);
   }
   return n;
 }

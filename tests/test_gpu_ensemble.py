@@ -314,3 +314,35 @@ def test_reference_deck_meshes_in_one_ensemble(hip_device, precision, tile):
         else:
             os.environ["NSM_TILE_ELEMS"] = old
     ens.close()
+
+
+@pytest.mark.parametrize("tile,samples", [(64, 40), (128, 36), (256, 64), (512, 33), (512, 64)])
+def test_more_tiles_than_resident_workgroups(hip_device, tile, samples):
+    """Tiles past one window of resident workgroups, a last window little and
+    entirely filled: the first, a middle and the last sample are the bits of a
+    model alone."""
+    n, steps = 16, 6
+    rng = np.random.default_rng(11)
+    prob = N.CubeProblem(n=n, materials=[N.problems.STEEL], num_steps=steps).build()
+    ens = N.Ensemble("mixed", tile)
+    mid = ens.AddMesh(prob.X, [b.conn for b in prob.blocks()])
+    for kind, nodes, c, _ in prob.bc_list():
+        ens.AddBoundaryCondition(mid, kind, nodes, c)
+    ens.SetReactionNodes(mid, prob.top, 2)
+    mats = [(E, nu, rho) for E, nu, rho in zip(rng.uniform(50e9, 250e9, samples), rng.uniform(0.22, 0.42, samples),
+                                               rng.uniform(2000, 9000, samples))]
+    v = rng.uniform(0.5, 2.0, samples)
+    nm = [N.NeohookeanMaterial.from_young(rho, E, nu) for E, nu, rho in mats]
+    mag = np.zeros((samples, 4))
+    mag[:, 3] = v
+    ens.AddSamples(mid, [[x.density] for x in nm], [[x.bulk_modulus] for x in nm], [[x.shear_modulus] for x in nm], mag)
+    ens.Setup()
+    dts = ens.CriticalTimeSteps()
+    ens.Run(steps, steps * (0.5 * dts), use_graph=False)
+    for s in (0, samples // 2, samples - 1):
+        _, m = single_model(n, [mats[s]], float(v[s]), steps, "mixed", tile)
+        for f in FIELDS:
+            assert np.array_equal(ens.GetNodeData(s, f), m.GetVectorNodeData(f)), (s, f)
+        assert np.array_equal(ens.GetReactionHistory(s), m.GetReactionHistory(0, steps)), s
+        m.close()
+    ens.close()
