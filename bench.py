@@ -69,9 +69,9 @@ VALU_PEAK_TFLOPS = {"mixed": 157.3, "fp64": 78.6}
 COUNTED_FLOPS_PER_ELEMENT_STEP = 9840
 # The FP64 element kernel is bound by VALU issue, not HBM: its VALU
 # instructions per element (8 lanes per element; rocprofv3 SQ_INSTS_VALU on
-# the 128^3 cube, 1,897 per lane) and the issue peak those are measured
+# the 128^3 cube, 1,717 per lane) and the issue peak those are measured
 # against: 1024 SIMDs, one wave64 FP64 instruction per 4 cycles, 2.4 GHz
-FP64_VALU_INSTS_PER_ELEMENT = 8 * 1897
+FP64_VALU_INSTS_PER_ELEMENT = 8 * 1717
 VALU_ISSUE_PEAK_PER_S = 1024 * 2.4e9 / 4
 # the same for the tiled mixed element kernel (one lane per element; SQ_INSTS_VALU
 # per wave of 64 elements on the 128^3 cube, 512-element tiles)

@@ -25,7 +25,8 @@ enum { F_XX = 0, F_YY = 1, F_ZZ = 2, F_XY = 3, F_YZ = 4, F_ZX = 5, F_YX = 6, F_Z
 // are finite, nonzero and normal with exponents far from the ends of the
 // range -- here: frexp exponents in [-299, 300] -- and div_fixup settles
 // zero, infinite and NaN operands from d and n alone, whatever quotient it
-// is given.  So for such operands r depends on d only, and the quotients
+// is given; div_fmas with vcc = 0 is a plain fma, without the wait for vcc.
+// So for such operands r depends on d only, and the quotients
 // over one denominator share it: the same operations on the same values,
 // hence the same bits as dividing one by one, with one reciprocal (a
 // quarter-rate instruction) and its refinement per denominator instead of
@@ -49,7 +50,7 @@ __device__ __forceinline__ double div_shared(double n, double d, double r)
 {
   const double q = n * r;
   const double e = __builtin_fma(-d, q, n);
-  return __builtin_amdgcn_div_fixup(__builtin_amdgcn_div_fmas(e, r, q, false), d, n);
+  return __builtin_amdgcn_div_fixup(__builtin_fma(e, r, q), d, n);
 }
 
 // q[i] = n[i] / d for i < kN, bit for bit as kN separate divisions: shared
