@@ -366,7 +366,7 @@ __device__ __forceinline__ void staged_element_fp64(Lds& lds, int64_t e, bool va
     }
   }
   if (kMode == kElementDefGrad) {
-    if (bad) atomicOr(status, 1);
+    if (bad) raise(status);
     return;
   }
   __syncthreads();  // node data no longer needed
@@ -385,7 +385,7 @@ __device__ __forceinline__ void staged_element_fp64(Lds& lds, int64_t e, bool va
     slots[slot_stride + sl]     = f[1];
     slots[2 * slot_stride + sl] = f[2];
   }
-  if (bad) atomicOr(status, 1);
+  if (bad) raise(status);
 }
 
 template <int kMode, bool kRefTable>
@@ -655,13 +655,6 @@ __device__ __forceinline__ void store_range(const double* s, int n, double* __re
     if ((int)threadIdx.x + i * kThreads < n) g[threadIdx.x + i * kThreads] = r[i];
 }
 
-// A seam's status word is host memory the device writes only when an element
-// is inverted; it is read after the stream has been waited for.
-__device__ __forceinline__ void raise(int* status)
-{
-  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
 __global__ __launch_bounds__(kThreads, 4) void k_seam_defgrad(int64_t E, const double* __restrict__ Xg,
                                                            const double* __restrict__ ug, double* __restrict__ F,
                                                            int* __restrict__ status)
@@ -878,7 +871,7 @@ __global__ __launch_bounds__(kThreads) void k_element_mass(int64_t e_begin, int6
     double a[9], b[9], bi[9];
     jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
-    if (det[el][k] <= 0.0) atomicOr(status, 1);
+    if (det[el][k] <= 0.0) raise(status);
   }
   __syncthreads();
   if (e < e_end) lumped_row(k, rho, det[el], &elem_mass[grouped ? fp64_slot(e, k) : (int64_t)k * E_total + e]);
@@ -912,7 +905,7 @@ __global__ __launch_bounds__(kThreads) void k_ens_element_mass(EnsNodes en, cons
     double a[9], b[9], bi[9];
     jacobians(shape_row(k), xs[el], zs[el], a, b);
     det[el][k] = invert3x3(b, bi);
-    if (det[el][k] <= 0.0) atomicOr(status, 1);
+    if (det[el][k] <= 0.0) raise(status);
   }
   __syncthreads();
   if (ok)

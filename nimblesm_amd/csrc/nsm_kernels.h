@@ -110,6 +110,13 @@ struct BlockTable {
   Real    G[kMaxLaunchBlocks];
 };
 
+// An inverted element.  The word may be host memory, which is written only
+// then, and read after the stream has been waited for.
+__device__ __forceinline__ void raise(int* status)
+{
+  __hip_atomic_store(status, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // block of element e (blocks ascending, e inside the table's range)
 template <typename Real>
 __device__ __forceinline__ int block_of(const BlockTable<Real>& bt, int64_t e)

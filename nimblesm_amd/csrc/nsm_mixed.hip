@@ -68,7 +68,7 @@ __global__ __launch_bounds__(kThreads) NSM_MIXED_WAVES_ATTR void k_element_mixed
   for (int n = 0; n < 8; n++)
 #pragma unroll
     for (int c = 0; c < 3; c++) slots[(int64_t)(c * 8 + n) * E_total + e] = f[n][c];
-  if (!ok) atomicOr(status, 1);
+  if (!ok) raise(status);
 }
 
 }  // namespace

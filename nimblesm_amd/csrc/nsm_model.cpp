@@ -70,17 +70,17 @@ namespace {
     if (_e != hipSuccess) return fail(NSM_ERR_HIP, "kernel launch: %s", hipGetErrorString(_e));    \
   } while (0)
 
-// Status words of the stateless seam entry points: pinned host memory every
-// device can write, one word per call in flight (a cache line each), taken
-// from a free list for the length of the call, so calls on different threads
-// and streams do not share one.  A word holds 0 unless a kernel of its call
-// met an inverted element.  The call waits for its stream and reads the word
-// where it lies: clearing a device word before the kernel and copying it to
-// the host after it cost a call two more stream operations.
-// A call on 343 elements: 20 -> 13 us.
-class SeamStatus {
+// Status words: pinned host memory every device can write, one word (a cache
+// line each) per model, and per call in flight of the stateless seam entry
+// points, from a free list, so calls on different threads and streams do not
+// share one.  A word holds 0 unless a kernel met an inverted element.  A call
+// waits for its stream and reads the word where it lies: clearing a device
+// word before the kernel and copying it to the host after it cost a seam two
+// more stream operations (343 elements: 20 -> 13 us), and the copy alone a
+// model's call 20 to 35 us (20 steps of 64^3 elements: 956 -> 920).
+class StatusWord {
  public:
-  // the call's word, 0 on entry
+  // a word that holds 0
   static int take(int** out)
   {
     std::lock_guard<std::mutex> lk(mutex());
@@ -135,7 +135,7 @@ int run_seam(int64_t n, void* stream, Launch&& launch)
   if (n < 0) return fail(NSM_ERR_ARG, "negative size");
   if (n == 0) return NSM_OK;
   int* status = nullptr;
-  int  st     = SeamStatus::take(&status);
+  int  st     = StatusWord::take(&status);
   if (st) return st;
   launch(status, (hipStream_t)stream);
   hipError_t e = hipGetLastError();
@@ -143,7 +143,7 @@ int run_seam(int64_t n, void* stream, Launch&& launch)
   if (e == hipSuccess) e = done;
   const int h = *(volatile int*)status;
   // a word whose kernel may still be running is not used again
-  if (done == hipSuccess) SeamStatus::give_back(status);
+  if (done == hipSuccess) StatusWord::give_back(status);
   if (e != hipSuccess) return fail(NSM_ERR_HIP, "element seam: %s", hipGetErrorString(e));
   if (h) return fail(NSM_ERR_NEG_JACOBIAN, "non-positive Jacobian determinant (Invert3x3)");
   return NSM_OK;
@@ -210,7 +210,7 @@ struct nsm_model {
   double*   elem_tmp = nullptr;  // [8][E] setup scratch (element masses)
   double*   wg_min = nullptr;
   int64_t   wg_min_len = 0;
-  int*      status = nullptr;
+  int*      status = nullptr;  // StatusWord
   uint8_t*  flags = nullptr;  // [N] bc table index + 1 | reaction bit
   nsm::BcEntry* bc_table = nullptr;
   int64_t   num_reaction_nodes = 0;
@@ -542,12 +542,10 @@ int rebuild_bcs(nsm_model* md)
 
 int check_status(nsm_model* md)
 {
-  int h = 0;
-  NSM_HIP(hipMemcpyAsync(&h, md->status, sizeof(int), hipMemcpyDeviceToHost, md->stream));
   NSM_HIP(hipStreamSynchronize(md->stream));
-  if (h) {
-    NSM_HIP(hipMemsetAsync(md->status, 0, sizeof(int), md->stream));
-    NSM_HIP(hipStreamSynchronize(md->stream));
+  volatile int* const word = md->status;
+  if (*word) {
+    *word = 0;
     return fail(NSM_ERR_NEG_JACOBIAN, "non-positive Jacobian determinant in an element (Invert3x3)");
   }
   return NSM_OK;
@@ -1436,7 +1434,7 @@ int model_create(int64_t num_nodes, const double* reference_coordinates, int num
       (st = dalloc((char**)&md->sip, 48 * E_ip * ipw, &tot)) ||
       (st = dalloc((char**)&md->slots, num_slots * ipw, &tot)) ||
       (st = dalloc(&md->rjac, precision == NSM_FP64 && use_reference_table(E) ? (size_t)(80 * E) : 0, &tot)) ||
-      (st = dalloc(&md->status, 1, &tot)) || (st = dalloc(&md->flags, (size_t)num_nodes, &tot)) ||
+      (st = StatusWord::take(&md->status)) || (st = dalloc(&md->flags, (size_t)num_nodes, &tot)) ||
       (st = dalloc(&md->reaction_partials, 2 * std::max<size_t>(num_partials, 1), &tot)) ||
       (md->tiled && (st = setup_tiles(md))))
     return cleanup(st);
@@ -1458,7 +1456,6 @@ int model_create(int64_t num_nodes, const double* reference_coordinates, int num
   NSM_HIP_C(hipMemsetAsync(md->a, 0, N3 * sizeof(double), s));
   NSM_HIP_C(hipMemsetAsync(md->f, 0, N3 * sizeof(double), s));
   NSM_HIP_C(hipMemsetAsync(md->m, 0, (size_t)num_nodes * sizeof(double), s));
-  NSM_HIP_C(hipMemsetAsync(md->status, 0, sizeof(int), s));
   NSM_HIP_C(hipMemsetAsync(md->flags, 0, (size_t)num_nodes, s));
   if (md->rjac) {
     nsm::launch_reference_jacobians(E, md->conn, md->X, md->rjac, s);
@@ -1493,7 +1490,9 @@ int nsm_model_destroy(nsm_model* md)
 {
   if (!md) return NSM_OK;
   (void)hipSetDevice(md->device);
-  if (md->stream) (void)hipStreamSynchronize(md->stream);
+  // a word whose kernels may still be running is not used again
+  if (md->stream && hipStreamSynchronize(md->stream) == hipSuccess && md->status) StatusWord::give_back(md->status);
+  md->status = nullptr;
   free_dev(md->X);
   free_dev(md->u);
   free_dev(md->v);
@@ -1511,7 +1510,6 @@ int nsm_model_destroy(nsm_model* md)
   free_dev(md->joint_bnd);
   free_dev(md->elem_tmp);
   free_dev(md->wg_min);
-  free_dev(md->status);
   free_dev(md->flags);
   free_dev(md->bc_table);
   free_dev(md->reaction_hist);

@@ -764,7 +764,7 @@ __global__ __launch_bounds__(kThreads, (kLeanTiles<kThreads, kOne, Work> ? 3 : 2
                       tile_table(ta.gather, cn.t) != 0, ns);
     }
   }
-  if (tid == 0 && bad) atomicOr(status, 1);
+  if (tid == 0 && bad) raise(status);
 }
 
 constexpr int kBndThreads = kBoundaryNodesPerGroup;

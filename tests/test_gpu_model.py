@@ -493,3 +493,36 @@ def test_joint_steps_match_separate_launches(hip_device, monkeypatch, precision,
     assert np.linalg.norm(got[0][-1]) > 0
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision,n", [("fp64", 3), ("mixed", 3), ("mixed", 20), ("fp64", 42)])
+def test_inverted_element_is_one_models_own(hip_device, precision, n):
+    """An inverted element fails the call that met it -- an evaluation and a
+    run of several steps -- and no call of another model, no later call of its
+    own and no later model."""
+    prob = N.CubeProblem(n=n, materials=[N.problems.STEEL], num_steps=20).build()
+    bad, good = prob.make_model(precision), prob.make_model(precision)
+    u = np.zeros_like(prob.X)
+    u[prob.top[0], 2] = -5.0
+    for m in (bad, good):
+        m.ComputeLumpedMass()
+    dt = 0.5 * good.GetCriticalTimeStep()
+    for call in (lambda m: m.ComputeInternalForce(), lambda m: m.ExplicitSteps(0, 5, 5, 0, dt, 0.0)):
+        bad.SetVectorNodeData("displacement", u)
+        bad.SetVectorNodeData("velocity", 0 * u)
+        good.SetVectorNodeData("displacement", 0 * u)
+        with pytest.raises(N.NimbleError) as ei:
+            call(bad)
+        assert ei.value.status == 3
+        call(good)
+        for f in ("displacement", "velocity", "acceleration"):  # the whole state a step starts from
+            bad.SetVectorNodeData(f, 0 * u)
+        call(bad)
+    bad.SetVectorNodeData("displacement", u)
+    with pytest.raises(N.NimbleError):
+        bad.ComputeInternalForce()
+    bad.close()
+    again = prob.make_model(precision)
+    again.ComputeInternalForce()
+    again.close()
+    good.close()
