@@ -2019,8 +2019,15 @@ int nsm_model_set_uq_samples(nsm_model* md, int num_exact, const double* bulk_mo
   md->uq_G.assign(shear_modulus, shear_modulus + nk);
   md->uq_exact  = num_exact;
   md->uq_approx = num_approx;
+  // Joint launches up to 12 windows of resident workgroups: beyond, a
+  // trajectory's partials and nodes no longer wait in the caches for the node
+  // launch of all.  us per step with two exact and five approximate samples,
+  // trajectory by trajectory / joint: 48^3 (2.5 windows) 122 / 73, 64^3 154 / 139,
+  // 80^3 (11.7) 272-280 / 258-270, 96^3 (20) 467-481 / 465-480, 112^3 717 / 721,
+  // 128^3 (48) 1031 / 1057.
+  constexpr int64_t kUqJointWindows = 12;
   if (md->tiled && num_exact <= nsm::kUqCachedExact && (num_exact + 1) * (int64_t)md->tiles.bnd_ent.size() < INT32_MAX &&
-      (num_exact + 1) * (int64_t)md->tiles.num_tiles < INT32_MAX) {
+      (num_exact + 1) * (int64_t)md->tiles.num_tiles <= kUqJointWindows * md->tile_args.resident_groups) {
     const size_t                   T = (size_t)num_exact + 1, nb = (size_t)md->num_blocks;
     std::vector<nsm::UqTrajectory> traj(T);
     std::vector<float>             moduli(2 * T * nb);
