@@ -2022,7 +2022,7 @@ int nsm_model_set_uq_samples(nsm_model* md, int num_exact, const double* bulk_mo
   // Joint launches up to 12 windows of resident workgroups: beyond, a
   // trajectory's partials and nodes no longer wait in the caches for the node
   // launch of all.  us per step with two exact and five approximate samples,
-  // trajectory by trajectory / joint: 48^3 (2.5 windows) 122 / 73, 64^3 154 / 139,
+  // trajectory by trajectory / joint: 48^3 (2.5 windows) 122 / 72, 64^3 154 / 139,
   // 80^3 (11.7) 272-280 / 258-270, 96^3 (20) 467-481 / 465-480, 112^3 717 / 721,
   // 128^3 (48) 1031 / 1057.
   constexpr int64_t kUqJointWindows = 12;

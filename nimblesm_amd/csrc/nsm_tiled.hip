@@ -490,10 +490,9 @@ template <int kThreads, bool kOne, typename Work>
 constexpr bool kLeanTiles = kOne && kThreads < 512 && std::is_same<Work, EnsTileWork>::value;
 
 template <int kThreads, bool kStoreIp, bool kOne, typename Work>
-__global__ __launch_bounds__(kThreads, (kLeanTiles<kThreads, kOne, Work> ? 3 : 2)) void k_element_tiled(const Work work, TileArgs ta,
-                                                            const double* __restrict__ X, NodeArrays na,
-                                                            float* __restrict__ Fip, float* __restrict__ sip,
-                                                            ReactionArgs rx, int* __restrict__ status)
+__global__ __launch_bounds__(kThreads, (kLeanTiles<kThreads, kOne, Work> ? 3 : 2)) void k_element_tiled(
+    const Work work, TileArgs ta, const double* __restrict__ X, NodeArrays na, float* __restrict__ Fip,
+    float* __restrict__ sip, ReactionArgs rx, int* __restrict__ status)
 {
   constexpr int  kNodes      = 2 * kThreads;
   constexpr bool kEnsemble   = std::is_same<Work, EnsTileWork>::value;
@@ -829,7 +828,7 @@ __global__ __launch_bounds__(kBndThreads) void k_boundary_update(TileArgs ta, No
 // registers a thread then runs the closure of the approximate samples, as
 // k_uq_closure does.  One launch where a step took one boundary launch per
 // trajectory and the closure: at 48^3 with two exact and five approximate
-// samples 122 -> 75 us per step (element 47, this 28).
+// samples 122 -> 72 us per step (element 43, this 28).
 __global__ __launch_bounds__(kBndThreads) void k_uq_nodes(TileArgs ta, NodeArrays na, const BcEntry* sample_bc,
                                                           UqClosure uc, int num_partials, unsigned groups,
                                                           StepArgs sa, ReactionArgs rx)
