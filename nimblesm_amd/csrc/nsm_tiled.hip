@@ -101,7 +101,7 @@ __device__ __forceinline__ SlotIds load_ids(const TileArgs& ta, const TileCtx& c
 #pragma unroll
   for (int k = 0; k < 2; k++) {
     const int ln = (int)threadIdx.x + k * kThreads;
-    const int sl = n0 + min(ln, nn - 1);
+    const int sl = n0 + staged_slot(ln, nn);
     r.gid[k]     = ta.nodes[sl] + c.node_base;
     const int d  = ta.slot_dst[sl];
     r.dst[k]     = ln < nn ? (d >= 0 ? d + c.partial_base : d) : kAbsent;
@@ -408,8 +408,9 @@ __device__ __forceinline__ void joint_reaction(const JointTileWork& w, const Til
 // previous step (see JointTileWork), and the flags, mass and v of its
 // interior nodes (left in ns).  Every load of both slots is issued before the
 // first is used, whatever kind of slot it is (an interior slot's partials are
-// entry 0, not used): a branch around them would make the kernel wait for one
-// slot's chain after the other's.  table (LDS) is staged in the meantime.
+// entry 0, not used; a slot past the tile's last loads that one's values,
+// from the arrays that hold its node): a branch around them would make the
+// kernel wait for one slot's chain after the other's.  table (LDS) is staged in the meantime.
 template <int kThreads>
 __device__ __forceinline__ void joint_nodes(const JointTileWork& w, const TileArgs& ta, const TileCtx& c,
                                             const SlotIds& ids, const NodeArrays& na, const BcEntry* table,
@@ -420,13 +421,13 @@ __device__ __forceinline__ void joint_nodes(const JointTileWork& w, const TileAr
   int2          p[2];
   float         pv[2][kBatch][3];
 #pragma unroll
-  for (int k = 0; k < 2; k++) p[k] = w.slot_partials[n0 + min((int)threadIdx.x + k * kThreads, nn - 1)];
+  for (int k = 0; k < 2; k++) p[k] = w.slot_partials[n0 + staged_slot((int)threadIdx.x + k * kThreads, nn)];
 #pragma unroll
   for (int k = 0; k < 2; k++) {
-    const bool own = ids.dst[k] == kInterior;
-    const int  i   = ids.gid[k];
-    load3(own ? na.u : w.bu_in, i, ur[k]);
-    load3(own ? na.v : w.bv_in, i, ns.v[k]);
+    const int  i      = ids.gid[k];
+    const bool shared = has_boundary_row(i, ta.bnd_base);
+    load3(shared ? w.bu_in : na.u, i, ur[k]);
+    load3(shared ? w.bv_in : na.v, i, ns.v[k]);
     ns.flg[k] = na.flags[i];
     ns.m[k]   = na.mass[i];
   }

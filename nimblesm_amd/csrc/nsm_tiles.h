@@ -55,6 +55,16 @@ struct TileSet {
   std::vector<int32_t>  int_off;        // [T+1]
 };
 
+// Slot, of a tile's nn, that thread-slot ln of its workgroup stages: past the
+// last one it takes that one again, so that every load runs.
+constexpr int staged_slot(int ln, int nn) { return ln < nn ? ln : nn - 1; }
+
+// Whether arrays that hold the boundary nodes only (rows from num_interior
+// on) have node id's row.  The id decides, not the slot's kind: a slot that
+// repeats a tile's last one is an interior node's where the tile has no
+// boundary node, as a body of its own that fits in one tile.
+constexpr bool has_boundary_row(int id, int num_interior) { return id >= num_interior; }
+
 // Builds the tiles of blocks given by element offsets blk_off (conn in
 // original element and node numbering, [E][8]) and renumbers the nodes (see
 // TileSet::node_new).  Returns false with a message when a tile
