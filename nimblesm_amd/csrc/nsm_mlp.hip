@@ -398,9 +398,11 @@ __global__ __launch_bounds__(256) void k_adam(Adam o, const float* __restrict__ 
 //
 // Weights are kept twice, in BF16 and padded to multiples of 32 with zeros:
 // wf [np][kp] with k along the input (forward), wt [kp][np] with k along the
-// output (input gradients), each in MFMA operand order (operand_index).  Padded columns of a layer's output are 0 (zero weights
-// and bias, gelu(0) = 0).  Rows past the batch, up to Bp (a multiple of 32),
-// are stored as 0 in H and D.
+// output (input gradients), each in MFMA operand order (operand_index).
+// Padded columns of a layer's output and of its gradient are 0 by selection:
+// their zero weights make a NaN of an infinite value, which the next product
+// would carry to every column.  Rows past the batch, up to Bp (a multiple of
+// 32), are stored as 0 in H and D.
 //
 // Training iteration of the 4-256-256-256-64 network, layer by layer and
 // here: batch 64 54 -> 19 us, 512 66 -> 23 us, 1024 100 -> 29 us, 2048 185 ->
@@ -544,7 +546,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(RowArgs a)
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
           const bool  ok = b0 + rl + r < a.B;
-          const float z  = acc[t][r] + (col < y.dout ? bias[l] : 0.0f);
+          const float z  = col < y.dout ? acc[t][r] + bias[l] : 0.0f;
           if (l + 1 < kL) {
             if (kTrain) gp[l][t][r] = gelu_grad(z);
             const bf16 h                  = (bf16)gelu(z);
@@ -603,7 +605,7 @@ __global__ __launch_bounds__(kRowThreads) void k_rows(RowArgs a)
         fvec          gv;
 #pragma unroll
         for (int r = 0; r < kPer; r++) {
-          gv[r] = b0 + rl + r < a.B ? acc[t][r] * gp[l > 0 ? l - 1 : 0][t][r] : 0.0f;
+          gv[r] = b0 + rl + r < a.B && col < y.din ? acc[t][r] * gp[l > 0 ? l - 1 : 0][t][r] : 0.0f;
           dv[r] = (bf16)gv[r];
           act[from ^ 1][rl + r][col] = dv[r];
         }

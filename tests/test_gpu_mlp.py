@@ -194,3 +194,32 @@ def test_forward_sees_trained_parameters(hip_device, B):
     assert np.array_equal(y, b.forward(x[:50]))
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("widths", [(1, 1, 1), (4, 48, 40, 8), (33, 7, 70, 31)])
+def test_infinite_values_stay_in_their_place(hip_device, widths):
+    """Widths that are no multiples of 32, all weights and inputs positive:
+    an infinite input makes its row's outputs infinite, an infinite target
+    the gradients that the oracle says; nothing turns NaN, and other rows
+    and columns keep their values (tolerances as above)."""
+    net = MLP(widths, seed=3)
+    rng = np.random.default_rng(4)
+    p = rng.uniform(0.01, 0.1, M.layout(widths)[1]).astype(np.float32)
+    net.set_parameters(p)
+    x, t = (np.abs(v) for v in data(widths, 37, 5))
+    y = net.forward(x)
+    xi = x.copy()
+    xi[11, 0] = np.inf
+    yi = net.forward(xi)
+    assert np.all(yi[11] == np.inf)
+    assert np.array_equal(np.delete(yi, 11, 0), np.delete(y, 11, 0))
+    t[11, -1] = np.inf
+    loss, g = net.loss_gradients(x, t)
+    rl, rg = M.loss_and_grad(p, widths, x, t, bf16=True)
+    assert loss == rl == np.inf
+    inf = np.isinf(rg)
+    assert np.all(rg[inf] == -np.inf) and inf.any()
+    assert np.all(g[inf] == -np.inf)
+    if not inf.all():
+        assert np.linalg.norm((g - rg)[~inf]) <= 5e-3 * np.linalg.norm(rg[~inf])
+    net.close()
