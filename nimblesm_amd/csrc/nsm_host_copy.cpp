@@ -3,8 +3,8 @@
 // hipMemcpy stages such a copy without overlap, and into fresh memory (a
 // result array just allocated) it reaches 10-14 GB/s where the link moves 57:
 // the 51.5 MB node field of the 128^3 cube took 5.0 ms.  Here the copy goes
-// in 1 MB chunks through pinned slots; while the host empties one (about 40
-// us, the page faults of fresh memory included), the device fills the next
+// in chunks through pinned slots; while the host empties one (about 40 us per
+// MB, the page faults of fresh memory included), the device fills the next
 // ones.  A kernel writes the slots: a copy-engine transfer and its event cost
 // about 20 us per chunk.
 //
@@ -14,16 +14,20 @@
 // thread may first wait a scheduler tick (4 ms) for a CPU, so nobody waits for
 // one: chunks are claimed one at a time, the caller carries whatever the
 // helpers do not, and a helper that starts late finds none left.
-// Into fresh memory, hipMemcpy / caller alone / with helpers: 2.8 MB 202 / 154
-// us, 6.6 MB 459 / 346 us, 21.9 MB 1.52 / 1.19 / 0.96 ms, 51.5 MB 5.0 / 4.2 /
-// 1.6 ms.  (Host to device the runtime already reaches 29-37 GB/s: those
-// copies stay with it.)
+// Into fresh memory, hipMemcpy / here: 2.8 MB 193 / 143 us, 6.6 MB 465 / 322,
+// 15 MB 1.04 / 0.73 ms, 21.9 MB 1.53 / 1.00, 30 MB 2.14 / 1.31, 45 MB 4.36 /
+// 1.33, 51.5 MB 5.03 / 1.51; into memory the caller keeps, 2.8 MB 157 / 121
+// us, 21.9 MB 1.25 / 0.63 ms, 51.5 MB 2.94 / 1.31.  (Host to device the
+// runtime already reaches 29-37 GB/s: those copies stay with it.)
 //
 // Memory that the device can write itself (pinned by the caller, managed, or
 // device memory) gets one copy at the link's rate instead; through the slots
 // it took twice that: 2.8 MB 58 / 118 us, 15 MB 271 / 625 us, 51.5 MB 0.91 /
 // 1.30 ms.  Asking for the kind of memory takes 0.4 us.
 #include "nsm_host_copy.h"
+
+#include "nsm_copy_plan.h"
+#include "nsm_kernels.h"
 
 #include <algorithm>
 #include <atomic>
@@ -37,27 +41,16 @@
 namespace nsm {
 namespace {
 
-constexpr size_t kChunk      = (size_t)1 << 20;
-constexpr int    kCopyGroups = 64;  // workgroups of a slot's transfer
-constexpr size_t kShared     = (size_t)16 << 20;
-constexpr int    kHelpers    = 7;
-constexpr int    kOwnSlots = 4, kHelperSlots = 2;  // slots of the caller and of a helper
-constexpr int    kMaxSlots = kOwnSlots + kHelpers * kHelperSlots;
-
-// n doubles to pinned host memory: the device writes it over the link itself
-__global__ __launch_bounds__(256) void k_copy_out(const double* __restrict__ src, double* __restrict__ dst, int n)
-{
-  for (int i = (int)(blockIdx.x * 256 + threadIdx.x); i < n; i += (int)gridDim.x * 256) dst[i] = src[i];
-}
-
 // pinned slots of one copy at a time
 struct Ring {
   int        device = -1, slots = 0;
+  size_t     bytes  = 0;
   char*      base   = nullptr;
   hipEvent_t done[kMaxSlots] = {};
 };
 
-// Idle rings: at most kIdle (4 or 18 MB each), given back with the last holder.
+// Idle rings: at most kIdle (at most 18 MB each), the largest of those given
+// back, since a small ring is soon made again; released with the last holder.
 constexpr int kIdle = 2;
 struct Pool {
   std::mutex m;
@@ -79,13 +72,15 @@ void destroy(Ring* r)
   delete r;
 }
 
-Ring* take(int device, int slots)
+Ring* take(int device, const CopyPlan& plan)
 {
+  const int    slots = plan.slots();
+  const size_t bytes = plan.pinned();
   {
     Pool&                       p = pool();
     std::lock_guard<std::mutex> lk(p.m);
     for (int i = 0; i < p.idle; i++)
-      if (p.ring[i]->device == device && p.ring[i]->slots >= slots) {
+      if (p.ring[i]->device == device && p.ring[i]->slots >= slots && p.ring[i]->bytes >= bytes) {
         Ring* r   = p.ring[i];
         p.ring[i] = p.ring[--p.idle];
         return r;
@@ -95,7 +90,8 @@ Ring* take(int device, int slots)
   if (!r) return nullptr;
   r->device = device;
   r->slots  = slots;
-  bool ok   = hipHostMalloc((void**)&r->base, (size_t)slots * kChunk, hipHostMallocDefault) == hipSuccess;
+  r->bytes  = bytes;
+  bool ok   = hipHostMalloc((void**)&r->base, bytes, hipHostMallocDefault) == hipSuccess;
   for (int i = 0; i < slots; i++)
     ok = ok && hipEventCreateWithFlags(&r->done[i], hipEventDisableTiming) == hipSuccess;
   if (ok) return r;
@@ -106,12 +102,17 @@ Ring* take(int device, int slots)
 
 void give_back(Ring* r)
 {
+  const auto smaller = [](const Ring* a, const Ring* b) { return a->bytes < b->bytes; };
   {
     Pool&                       p = pool();
     std::lock_guard<std::mutex> lk(p.m);
     if (p.holders > 0 && p.idle < kIdle) {
       p.ring[p.idle++] = r;
       return;
+    }
+    if (p.holders > 0) {
+      Ring*& least = *std::min_element(p.ring, p.ring + kIdle, smaller);
+      if (least->bytes < r->bytes) std::swap(least, r);
     }
   }
   destroy(r);
@@ -122,6 +123,7 @@ void give_back(Ring* r)
 // is active, nobody touches the ring or the caller's memory again.
 struct Copy {
   Ring*               ring;
+  CopyPlan            plan;
   hipStream_t         stream;
   char*               dst;
   const char*         src;
@@ -140,16 +142,17 @@ struct Copy {
 // Carries chunks through slots [slot0, slot0 + n) until none is left.
 void carry(Copy& c, int slot0, int n)
 {
-  size_t     held[kOwnSlots];  // chunk in each slot, in the order of the slots
+  size_t     held[kMaxOwnSlots];  // chunk in each slot, in the order of the slots
   int        first = 0, count = 0;
   hipError_t e     = hipSuccess;
-  const auto size  = [&](size_t k) { return std::min(kChunk, c.bytes - k * kChunk); };
+  const size_t chunk = c.plan.chunk;
+  const auto   size  = [&](size_t k) { return std::min(chunk, c.bytes - k * chunk); };
   const auto fill  = [&] {  // the next chunk into the slot after the last held one
     const size_t k = c.claim();
     if (k >= c.chunks) return false;
     const int i = (first + count) % n;
-    hipLaunchKernelGGL(k_copy_out, dim3(kCopyGroups), dim3(256), 0, c.stream, (const double*)(c.src + k * kChunk),
-                       (double*)(c.ring->base + (size_t)(slot0 + i) * kChunk), (int)(size(k) / sizeof(double)));
+    launch_copy_out((const double*)(c.src + k * chunk), (double*)(c.ring->base + (size_t)(slot0 + i) * chunk),
+                    (int)(size(k) / sizeof(double)), c.stream);
     e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(c.ring->done[slot0 + i], c.stream);
     held[i] = k;
@@ -161,7 +164,7 @@ void carry(Copy& c, int slot0, int n)
   while (count > 0 && e == hipSuccess) {
     const int i = first;
     if ((e = hipEventSynchronize(c.ring->done[slot0 + i])) != hipSuccess) break;
-    std::memcpy(c.dst + held[i] * kChunk, c.ring->base + (size_t)(slot0 + i) * kChunk, size(held[i]));
+    std::memcpy(c.dst + held[i] * chunk, c.ring->base + (size_t)(slot0 + i) * chunk, size(held[i]));
     first = (first + 1) % n;
     count--;
     if (more) more = fill();
@@ -187,24 +190,26 @@ bool direct(const void* dst)
   return a.type != hipMemoryTypeUnregistered;
 }
 
-hipError_t staged(int device, hipStream_t stream, char* dst, const char* src, size_t bytes, Ring* ring, int helpers)
+hipError_t staged(int device, hipStream_t stream, char* dst, const char* src, size_t bytes, Ring* ring,
+                  const CopyPlan& plan)
 {
-  const std::shared_ptr<Copy> c(new Copy{ring, stream, dst, src, bytes, (bytes + kChunk - 1) / kChunk});
+  const std::shared_ptr<Copy> c(
+      new Copy{ring, plan, stream, dst, src, bytes, (bytes + plan.chunk - 1) / plan.chunk});
   try {
-    for (int h = 0; h < helpers; h++)
+    for (int h = 0; h < plan.helpers; h++)
       std::thread([c, h, device] {
         c->active.fetch_add(1);
         if (c->next.load() < c->chunks) {
           const hipError_t e = hipSetDevice(device);
           if (e == hipSuccess)
-            carry(*c, kOwnSlots + h * kHelperSlots, kHelperSlots);
+            carry(*c, c->plan.own + h * kHelperSlots, kHelperSlots);
         }
         c->active.fetch_sub(1);
       }).detach();
   } catch (const std::exception&) {
     // no further thread: the caller carries the rest
   }
-  carry(*c, 0, kOwnSlots);
+  carry(*c, 0, plan.own);
   while (c->active.load() > 0) std::this_thread::yield();
   return (hipError_t)c->error.load();
 }
@@ -214,14 +219,13 @@ hipError_t staged(int device, hipStream_t stream, char* dst, const char* src, si
 hipError_t device_to_host(int device, hipStream_t stream, double* dst, const double* src, size_t count)
 {
   const size_t bytes = count * sizeof(double);
-  // below two chunks there is nothing to overlap and hipMemcpy is as fast
-  if (bytes < 2 * kChunk || direct(dst)) return plain(stream, dst, src, bytes);
-  const int   helpers = bytes >= kShared ? kHelpers : 0;
-  Ring* const ring    = take(device, kOwnSlots + helpers * kHelperSlots);
+  if (bytes < kStaged || direct(dst)) return plain(stream, dst, src, bytes);
+  const CopyPlan plan = copy_plan(bytes);
+  Ring* const    ring = take(device, plan);
   if (!ring) return plain(stream, dst, src, bytes);
   hipError_t e;
   try {
-    e = staged(device, stream, (char*)dst, (const char*)src, bytes, ring, helpers);
+    e = staged(device, stream, (char*)dst, (const char*)src, bytes, ring, plan);
   } catch (const std::exception&) {  // no memory for the shared record: nothing was started
     e = plain(stream, dst, src, bytes);
   }

@@ -242,5 +242,9 @@ void launch_ip_gather(const void* src, const IpLayout& layout, int64_t e_begin, 
 // (map[n] = device index of mesh node n, a permutation of [0, N))
 void launch_permute_nodes(const double* src, const int32_t* map, int64_t N, int w, bool to_device, double* dst,
                           hipStream_t s);
+// n doubles to pinned host memory, written over the link by the kernel itself
+// (here, among kernels a model has run by then: the first launch of a
+// source's kernels loads its code, which would cost the first copy 0.5 ms)
+void launch_copy_out(const double* src, double* dst, int n, hipStream_t s);
 
 }  // namespace nsm

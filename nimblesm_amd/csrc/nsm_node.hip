@@ -189,6 +189,15 @@ __global__ __launch_bounds__(kNodeThreads) void k_permute_nodes(const double* __
     for (int c = 0; c < w; c++) dst[n * w + c] = src[d * w + c];
 }
 
+// a slot of a staged host copy (nsm_host_copy.cpp): 64 workgroups for 1 MB
+constexpr int kCopyGroups = 64;
+__global__ __launch_bounds__(kNodeThreads) void k_copy_out(const double* __restrict__ src, double* __restrict__ dst,
+                                                           int n)
+{
+  for (int i = (int)(blockIdx.x * kNodeThreads + threadIdx.x); i < n; i += (int)gridDim.x * kNodeThreads)
+    dst[i] = src[i];
+}
+
 // One value per thread, written in output order.
 __global__ __launch_bounds__(kNodeThreads) void k_ip_gather(const void* __restrict__ src, IpLayout L,
                                                             int64_t e_begin, int64_t count, double* __restrict__ dst)
@@ -472,6 +481,11 @@ void launch_permute_nodes(const double* src, const int32_t* map, int64_t N, int 
   if (N <= 0) return;
   hipLaunchKernelGGL(k_permute_nodes, dim3((unsigned)((N + kNodeThreads - 1) / kNodeThreads)), dim3(kNodeThreads), 0,
                      s, src, map, N, w, (int)to_device, dst);
+}
+
+void launch_copy_out(const double* src, double* dst, int n, hipStream_t s)
+{
+  hipLaunchKernelGGL(k_copy_out, dim3(kCopyGroups), dim3(kNodeThreads), 0, s, src, dst, n);
 }
 
 void launch_ens_fold(EnsFold fold, hipStream_t s)

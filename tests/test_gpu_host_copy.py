@@ -56,3 +56,33 @@ def test_pinned_and_device_destinations(hip_device, num_nodes):
 
     assert best(lambda: get(pinned.data_ptr())) <= 1.25 * best(runtime)
     m.close()
+
+
+@pytest.mark.parametrize("sizes", [(699050, 699051, 1747626), (1747627, 100000, 2500000)])
+def test_copies_of_every_cut_in_turn(hip_device, sizes):
+    """Fields on both sides of the sizes at which the cut changes (16 and 40
+    MB), read by three threads at once, each in its own order: every value
+    arrives, whichever pinned slots a copy finds."""
+    import threading
+
+    models = [model(n) for n in sizes]
+    bad = []
+
+    def read(k):
+        for r in range(6):
+            i = (k + r) % len(models)
+            m, v = models[i]
+            with locks[i]:  # one call of a model at a time
+                got = m.GetVectorNodeData("velocity")
+            if not np.array_equal(got, v):
+                bad.append((k, i))
+
+    locks = [threading.Lock() for _ in models]
+    threads = [threading.Thread(target=read, args=(k,)) for k in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for m, _ in models:
+        m.close()
