@@ -891,31 +891,40 @@ bool joint_steps(const nsm_model* md)
   return md->joint_ok && !md->timing && md->uq_samples() == 0;
 }
 
+// The joint steps' buffers, which become the model's once the work that fills
+// their tables is accepted: after a call that failed before, a later one
+// starts anew instead of running on tables without content.
 int ensure_joint(nsm_model* md)
 {
+  if (md->joint_bnd || md->joint_state) return NSM_OK;
+  double* buf   = nullptr;
+  size_t  bytes = 0;
   if (md->tiled) {
-    if (md->joint_bnd) return NSM_OK;
     const size_t bnd   = 6 * (size_t)md->tile_args.num_bnd + 3 * (size_t)md->reaction_stride;
     const size_t slots = md->tiles.nodes.size(), values = 3 * md->tiles.bnd_ent.size();
-    int          st    = dalloc(&md->joint_bnd, bnd + slots + (values + 1) / 2, &md->device_bytes);
+    const int    st    = dalloc(&buf, bnd + slots + (values + 1) / 2, &bytes);
     if (st) return st;
-    md->joint_slots    = (int2*)(md->joint_bnd + bnd);
+    md->joint_slots    = (int2*)(buf + bnd);
     md->joint_partials = (float*)(md->joint_slots + slots);
     nsm::launch_slot_partials(md->tile_args, (int)slots, md->joint_slots, md->stream);
-    NSM_LAUNCHED();
-    return NSM_OK;
+  } else {
+    const size_t state = 6 * (size_t)md->N + 6 * (size_t)md->joint_stride();
+    const size_t rows  = (size_t)(8 * md->E) * nsm::kMaxIncidence;
+    const int    st    = dalloc(&buf, state + rows / 2, &bytes);
+    if (st) return st;
+    md->joint_rows = (uint32_t*)(buf + state);
+    nsm::launch_incidence_rows(md->E, md->conn, md->node_ptr, md->node_ent, (uint32_t)(md->joint_stride() - 8),
+                               md->joint_rows, md->stream);
+    // the slots past the elements', the incidence rows' padding, stay zero
+    (void)hipMemsetAsync(buf, 0, state * sizeof(double), md->stream);
   }
-  if (md->joint_state) return NSM_OK;
-  const size_t state = 6 * (size_t)md->N + 6 * (size_t)md->joint_stride();
-  const size_t rows  = (size_t)(8 * md->E) * nsm::kMaxIncidence;
-  int          st    = dalloc(&md->joint_state, state + rows / 2, &md->device_bytes);
-  if (st) return st;
-  md->joint_rows = (uint32_t*)(md->joint_state + state);
-  nsm::launch_incidence_rows(md->E, md->conn, md->node_ptr, md->node_ent, (uint32_t)(md->joint_stride() - 8),
-                             md->joint_rows, md->stream);
-  NSM_LAUNCHED();
-  // the slots past the elements', the incidence rows' padding, stay zero
-  NSM_HIP(hipMemsetAsync(md->joint_state, 0, state * sizeof(double), md->stream));
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    free_dev(buf);
+    return fail(NSM_ERR_HIP, "tables of the joint steps: %s", hipGetErrorString(e));
+  }
+  (md->tiled ? md->joint_bnd : md->joint_state) = buf;
+  md->device_bytes += bytes;
   return NSM_OK;
 }
 

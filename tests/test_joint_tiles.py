@@ -105,3 +105,34 @@ def test_separate_bodies_match_separate_launches(hip_device, monkeypatch, sizes,
     assert np.linalg.norm(got[0][-1]) > 0
     for a, b in zip(*got):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision,n", [("fp64", 1), ("fp64", 5), ("mixed", 5)])
+def test_second_buffers_in_used_memory(hip_device, monkeypatch, precision, n):
+    """The buffers of the joint launches may lie where other data was: models
+    made after memory full of NaN has been given back advance to the bits of
+    separate launches."""
+    import torch
+
+    monkeypatch.setenv("NSM_TILE_ELEMS", "64")
+    X, conn, _ = bodies((n,))
+    got = []
+    for separate in (False, True):
+        m = N.ModelData(X, [N.Block(1, conn, N.NeohookeanMaterial.from_young(7800.0, 200e9, 0.3))], precision=precision)
+        m.ComputeLumpedMass()
+        dt = 0.5 * m.GetCriticalTimeStep()
+        m.SetVectorNodeData("displacement", 1e-3 * np.sin(3 * X) * X[:, 2:3])
+        if separate:
+            m.EnableKernelTiming(True, every=1000)
+        used = [torch.full((k,), float("nan"), device=hip_device) for k in (1 << 10, 1 << 14, 1 << 18, 1 << 22)]
+        torch.cuda.synchronize()
+        del used
+        torch.cuda.empty_cache()
+        before = m.Info()["device_bytes"]
+        m.ExplicitSteps(0, 5, 5, 0, dt, 0.0)
+        assert (m.Info()["device_bytes"] > before) == (not separate)
+        got.append([m.GetVectorNodeData(f) for f in ("displacement", "velocity", "acceleration", "internal_force")])
+        m.close()
+    for a, b in zip(*got):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
