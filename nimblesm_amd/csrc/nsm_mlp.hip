@@ -1083,25 +1083,26 @@ int forward_rows(nsm_mlp* net, int64_t B)
 // hardly depends on its rows), then 8, then 16.
 int train_group(int64_t B) { return B <= 1024 ? 4 : B <= 2048 ? 8 : 16; }
 
-int64_t row_partials(int64_t B) { return (B + 31) / 32 * 32 / train_group(B); }
+int64_t row_padded(int64_t B) { return (B + 31) / 32 * 32; }
 
-// One pass over the B rows in x32, t32: squared-error partials
+int64_t row_partials(int64_t B) { return row_padded(B) / train_group(B); }
+
+// activations and gradients of a training pass of B rows
+int ensure_row_batch(nsm_mlp* net, int64_t B)
+{
+  int64_t per_row = 0;  // bytes
+  for (const RowLayer& y : net->row) per_row += 2 * y.kp + 6 * y.np;
+  return ensure_rows(&net->row_batch, &net->row_cap, row_padded(B), per_row);
+}
+
+// One pass over the B rows in x32, t32 (after ensure_row_batch): squared-error partials
 // (row_partials(B) of them) and gradients, which go to net->g, or through
 // Adam when `adam` is given.
 int train_rows(nsm_mlp* net, int64_t B, double* partial, const Adam* adam)
 {
   int st = pack_rows(net);
   if (st) return st;
-  const int64_t Bp = (B + 31) / 32 * 32;
-  if (Bp > net->row_cap) {
-    int64_t per_row = 0;  // bytes
-    for (const RowLayer& y : net->row) per_row += 2 * y.kp + 6 * y.np;
-    if (net->row_batch) MLP_HIP(hipFree(net->row_batch));
-    net->row_batch = nullptr;
-    net->row_cap   = 0;
-    MLP_HIP(hipMalloc((void**)&net->row_batch, (size_t)(per_row * Bp)));
-    net->row_cap = Bp;
-  }
+  const int64_t Bp = row_padded(B);
   char* q = net->row_batch;  // every array a multiple of 64 bytes
   for (RowLayer& y : net->row) {
     y.ht = (bf16*)q, q += 2 * y.kp * Bp;
@@ -1320,10 +1321,11 @@ int nsm_mlp_loss_gradients(nsm_mlp* net, int64_t batch, const float* x, const fl
   const int64_t n = batch * net->width.back();
   const bool    rows     = net->rows && batch <= kRowBatch;
   const int64_t per_pass = rows ? row_partials(batch) : kMseBlocks;
-  if ((st = ensure_loss(net, 1, per_pass))) return st;
+  if ((st = ensure_loss(net, 1, per_pass)) || (st = rows ? ensure_row_batch(net, batch) : ensure_batch(net, batch)))
+    return st;
   if (rows)
     st = train_rows(net, batch, net->loss_part, nullptr);
-  else if (!(st = ensure_batch(net, batch)) && !(st = forward(net, batch)))
+  else if (!(st = forward(net, batch)))
     st = backward(net, batch, net->loss_part);
   if (st) return st;
   hipLaunchKernelGGL(k_mse_total, dim3(1), dim3(64), 0, net->stream, net->loss_part, (int)per_pass, n, net->loss);
@@ -1346,8 +1348,10 @@ int nsm_mlp_train(nsm_mlp* net, int64_t batch, const float* x, const float* t, i
   if (st) return st;
   const bool    rows     = net->rows && batch <= kRowBatch;
   const int64_t per_pass = rows ? row_partials(batch) : kMseBlocks;
-  if ((st = ensure_loss(net, iterations, per_pass))) return st;
-  if (!rows && (st = ensure_batch(net, batch))) return st;
+  // every buffer before the first step: a call without memory trains nothing
+  if ((st = ensure_loss(net, iterations, per_pass)) ||
+      (st = rows ? ensure_row_batch(net, batch) : ensure_batch(net, batch)))
+    return st;
   const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
   for (int it = 0; it < iterations; it++) {
     // cosine decay from lr to lr_final
