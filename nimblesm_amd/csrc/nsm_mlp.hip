@@ -1000,6 +1000,13 @@ int backward(nsm_mlp* net, int64_t B, double* partial)
 // Training batches up to kRowBatch rows, the largest measured (205 us per
 // iteration against 693); longer ones, and other networks, run layer by layer.
 constexpr int64_t kRowBatch = 16384;
+// A prediction of more rows goes layer by layer where no width passes 32: then
+// 2 of k_rows' 16 waves have columns, and with every CU busy that costs more
+// than the launches.  Layer by layer / k_rows: 3-16-1, 16,384 rows 46 / 47 us,
+// 60,000 81 / 92, 1e6 829 / 1059; 4-32-32-8, 16,384 76 / 74, 60,000 200 / 213,
+// 1e6 3.05 / 3.40 ms; 8-33-33-33-4, 60,000 198 / 188 us, 1e6 3.17 / 3.20 ms;
+// 4-64-64-8, 60,000 215 / 215 us, 1e6 3.41 / 3.41 ms.
+constexpr int kNarrow = 32;
 
 bool fits_rows(const std::vector<int>& width)
 {
@@ -1303,9 +1310,10 @@ int nsm_mlp_forward(nsm_mlp* net, int64_t batch, const float* x, float* y)
   if (batch == 0) return NSM_OK;
   MLP_HIP(hipSetDevice(net->device));
   int st = load_rows(net, batch, x, nullptr);
-  if (st || (st = net->rows ? forward_rows(net, batch) : ensure_batch(net, batch))) return st;
-  if (!net->rows && (st = forward(net, batch))) return st;
-  MLP_HIP(hipMemcpyAsync(y, net->rows ? net->y32 : net->z.back(), (size_t)(batch * net->width.back()) * sizeof(float),
+  const bool rows = net->rows && (batch <= kRowBatch || net->max_width() > kNarrow);
+  if (st || (st = rows ? forward_rows(net, batch) : ensure_batch(net, batch))) return st;
+  if (!rows && (st = forward(net, batch))) return st;
+  MLP_HIP(hipMemcpyAsync(y, rows ? net->y32 : net->z.back(), (size_t)(batch * net->width.back()) * sizeof(float),
                          hipMemcpyDeviceToHost, net->stream));
   MLP_HIP(hipStreamSynchronize(net->stream));
   return NSM_OK;

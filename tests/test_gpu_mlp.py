@@ -223,3 +223,21 @@ def test_infinite_values_stay_in_their_place(hip_device, widths):
     if not inf.all():
         assert np.linalg.norm((g - rg)[~inf]) <= 5e-3 * np.linalg.norm(rg[~inf])
     net.close()
+
+
+@pytest.mark.parametrize("widths", [(3, 16, 1), (4, 32, 32, 8), (4, 33, 8)])
+def test_long_predictions_are_their_pieces(hip_device, widths):
+    """Predictions on both sides of 16,384 rows, where narrow networks change
+    from one launch to a launch per layer, also after training on the other
+    side: every row's bits are those of a short prediction, and of a network
+    that was given the parameters."""
+    a, b = MLP(widths, seed=8), MLP(widths, seed=9)
+    x, t = data(widths, 40000, 10)
+    for B in (40000, 64):
+        a.train(x[:B], t[:B], 2, 1e-2, 1e-2)
+        b.set_parameters(a.get_parameters())
+        short = np.concatenate([b.forward(x[k:k + 8000]) for k in range(0, 40000, 8000)])
+        for n in (16384, 16385, 40000):
+            assert np.array_equal(a.forward(x[:n]), short[:n])
+    a.close()
+    b.close()
