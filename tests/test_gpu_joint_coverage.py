@@ -1,0 +1,70 @@
+"""Which of a model's launches run: the joint steps where their rule says (they
+leave second buffers behind), and the persistent form of the joint UQ element
+launch, whose workgroups pass from one trajectory's tiles to the next one's."""
+import numpy as np
+import pytest
+
+import nimblesm_amd as N
+
+pytestmark = pytest.mark.gpu
+FIELDS = ("displacement", "velocity", "acceleration", "internal_force")
+
+
+@pytest.mark.parametrize("precision,tile,n,joint",
+                         [("fp64", 0, 1, True), ("fp64", 0, 9, True), ("fp64", 0, 40, True), ("fp64", 0, 41, False),
+                          ("mixed", 64, 1, False), ("mixed", 512, 7, True), ("mixed", 512, 9, True),
+                          ("mixed", 64, 3, True), ("mixed", 64, 49, True), ("mixed", 128, 66, True),
+                          ("mixed", 128, 76, False), ("mixed", 512, 55, False)])
+def test_joint_steps_run_where_they_should(hip_device, monkeypatch, precision, tile, n, joint):
+    """One block where n is 1 (no shared nodes in a tiled model), else two."""
+    monkeypatch.setenv("NSM_TILE_ELEMS", str(tile or "auto"))
+    mats = [N.problems.STEEL, N.problems.ALUMINIUM] if n > 1 else [N.problems.STEEL]
+    prob = N.CubeProblem(n=n, materials=mats, num_steps=20, name="joint").build()
+    m = prob.make_model(precision)
+    integ = prob.make_integrator(m)
+    before = m.Info()["device_bytes"]
+    integ.Advance(2)
+    assert m.Info()["device_bytes"] == before  # too few to gain
+    integ.Advance(3)
+    assert (m.Info()["device_bytes"] > before) == joint
+    m.close()
+
+
+@pytest.mark.parametrize("tile", [64, 128, 256, 512])
+def test_persistent_joint_uq_launch(hip_device, monkeypatch, tile):
+    """Eight exact samples on a 29^3 cube: more tiles of all trajectories than
+    resident workgroups, and a last window more than 6/10 full, so the element
+    launch is persistent.  Every trajectory has the bits of launches of its
+    own (which nine samples take), with conditions that the samples do not
+    share, and so have approximate samples without weight on the ninth."""
+    import torch
+
+    monkeypatch.setenv("NSM_TILE_ELEMS", str(tile))
+    prob = N.CubeProblem(n=29, materials=[N.problems.STEEL, N.problems.ALUMINIUM], num_steps=9, name="uq")
+    rng = np.random.default_rng(4)
+    scale = rng.uniform(0.8, 1.2, (9, 1))
+    K0 = np.array([b.material.bulk_modulus for b in prob.blocks()])
+    G0 = np.array([b.material.shear_modulus for b in prob.blocks()])
+    c = rng.uniform(-0.5, 1.0, (2, 10))
+    c[:, 9] = 0.0
+    got = []
+    for ne in (8, 9):
+        m = prob.make_model("mixed")
+        window = torch.cuda.get_device_properties(0).multi_processor_count * 512 // tile
+        items = 9 * m.AssemblyInfo()["num_tiles"]
+        assert items > window and 10 * (items % window) > 6 * window and items <= 12 * window
+        m.AddBoundaryCondition("prescribed_displacement", prob.node_layer(4)[::3], 1, 1e-5)
+        m.AddBoundaryCondition("initial_velocity", prob.node_layer(3), 0, 2.0)
+        m.SetUqSamples(K0 * scale[:ne], G0 * scale[:ne], c[:, :ne + 1])
+        integ = prob.make_integrator(m, output_frequency=2)
+        integ.Advance(4)
+        integ.Advance(5)
+        out = [m.GetVectorNodeData(f) for f in FIELDS] + [m.GetReactionHistory(0, 9)]
+        out += [m.GetIntegrationPointData("stress"), m.GetIntegrationPointData("deformation_gradient")]
+        for s in list(range(8)) + [ne, ne + 1]:
+            out += [m.GetUqNodeData(s, f) for f in FIELDS]
+        got.append(out)
+        m.close()
+    assert np.linalg.norm(got[0][0]) > 0 and not np.array_equal(got[0][0], got[0][7])
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
