@@ -845,15 +845,18 @@ int setup_tiles(nsm_model* md)
   // launch would wait for, each of them in some tile, and all tiles on the
   // device at once, or a few windows of them with a last one that a
   // persistent grid would fill too little.  Tiles update the shared nodes
-  // they read each for themselves, which adds up with more windows.  us per
-  // step, persistent / one workgroup per tile / the same and one launch:
-  // 128-element tiles 1.07 windows 36.2 / 31.6 / 30.1, 1.65 42.8 / 41.2 /
-  // 40.1, 2.2 54.8 / 50.4 / 49.2, 2.4 55.3 / 51.1 / 51.7, 4.2 88.0 / 79.7 /
-  // 82.1; 256: 1.07 37.7 / 32.4 / 30.8, 2.4 56.2 / 51.4 / 50.4, 4.2 89.9 /
-  // 84.0 / 87.4.
+  // they read each for themselves, which adds up with more windows, and in
+  // 64-element tiles, where most nodes are shared, past one.  us
+  // per step, persistent / one workgroup per tile / the same and one launch:
+  // 128-element tiles 0.3 windows - / 19.8 / 18.0, 1.07 36.2 / 31.6 / 30.1, 1.65
+  // 42.8 / 41.2 / 40.1, 2.2 54.8 / 50.4 / 49.2, 2.4 55.3 / 51.2 / 51.0, 4.2 88.0
+  // / 79.7 / 82.1; 256: 0.3 - / 17.6 / 15.8, 1.07 37.7 / 32.4 / 30.8, 2.4 56.2 /
+  // 51.4 / 50.4, 4.2 89.9 / 84.0 / 87.4; 64: 0.4 - / 16.7 / 15.1, 1.23 34.4 /
+  // 30.3 / 30.3, 2.18 46.9 / 43.8 / 45.7, 2.42 49.4 / 46.5 / 47.9; 512: 0.3 - /
+  // 20.7 / 19.6, 0.96 - / 26.5 / 26.0, 2.1 57.6 in one launch, 54.3 persistent.
   const int64_t tiles = ts.num_tiles, window = ta.resident_groups;
-  const bool    few =
-      tiles <= window || (2 * tiles <= 5 * window && nsm::last_window_partial(tiles, ta, 7));
+  const bool    few   = tiles <= window || (ta.tile_elems > 64 && 2 * tiles <= 5 * window &&
+                                       nsm::last_window_partial(tiles, ta, 7));
   md->joint_ok        = md->num_blocks <= nsm::kMaxLaunchBlocks && few && ta.num_bnd > 0;
   for (int b = 0; b < ta.num_bnd && md->joint_ok; b++)
     md->joint_ok = ts.bnd_ptr[(size_t)b + 1] > ts.bnd_ptr[(size_t)b];
