@@ -13,13 +13,15 @@ constexpr int    kMaxSlots = kMaxOwnSlots + kMaxHelpers * kHelperSlots;
 
 // The caller's pinned slots and two for each helper, of a chunk each.  New
 // pinned memory costs its first touch by the host 370 us per MB, so small
-// copies use few and small slots (0.75 MB; with 4 MB the first read of a
-// process took 0.8 to 1.8 ms longer than hipMemcpy's), copies in between 5.5
-// MB, and only from kLarge on, where hipMemcpy takes 4 ms and more, 18 MB.
-// First read of a process, hipMemcpy / these: 2.2 MB 0.55 / 0.56 ms, 6.6 MB
-// 1.02 / 1.25, 15 MB 1.83 / 1.92, 18 MB 2.03 / 1.66, 32 MB 3.49 / 2.03, 51.5
-// MB 5.1 / 2.9; the first one after another model's end, 18 MB 1.17 / 0.77,
-// 32 MB 2.13 / 1.56.
+// copies use few and small slots (1 MB; with 4 MB the first read of a process
+// took 0.8 to 1.8 ms longer than hipMemcpy's), copies in between 5.5 MB, and
+// only from kLarge on, where hipMemcpy takes 4 ms and more, 18 MB.  First read
+// of a process, hipMemcpy / these: 2.2 MB 0.56 / 0.65 ms, 6.6 MB 1.02 / 1.29,
+// 15 MB 1.79 / 1.86, 18 MB 2.03 / 1.66, 32 MB 3.49 / 2.03, 51.5 MB 5.1 / 2.9;
+// the first one after another model's end, 18 MB 1.17 / 0.77, 32 MB 2.13 /
+// 1.56.  Three slots of 256 KB make the first read 0.1 ms shorter and eight
+// results of 2.8 MB that the caller keeps 1.57 ms instead of 1.41 (hipMemcpy
+// 1.68).
 struct CopyPlan {
   size_t chunk;
   int    own, helpers;
@@ -30,7 +32,7 @@ struct CopyPlan {
 
 constexpr CopyPlan copy_plan(size_t bytes)
 {
-  if (bytes < kShared) return {(size_t)256 << 10, 3, 0};
+  if (bytes < kShared) return {(size_t)512 << 10, 2, 0};
   if (bytes < kLarge) return {(size_t)512 << 10, 3, 4};
   return {(size_t)1 << 20, kMaxOwnSlots, kMaxHelpers};
 }

@@ -14,10 +14,10 @@
 // thread may first wait a scheduler tick (4 ms) for a CPU, so nobody waits for
 // one: chunks are claimed one at a time, the caller carries whatever the
 // helpers do not, and a helper that starts late finds none left.
-// Into fresh memory, hipMemcpy / here: 2.8 MB 193 / 143 us, 6.6 MB 465 / 322,
-// 15 MB 1.04 / 0.73 ms, 21.9 MB 1.53 / 1.00, 30 MB 2.14 / 1.31, 45 MB 4.36 /
-// 1.33, 51.5 MB 5.03 / 1.51; into memory the caller keeps, 2.8 MB 157 / 121
-// us, 21.9 MB 1.25 / 0.63 ms, 51.5 MB 2.94 / 1.31.  (Host to device the
+// Into fresh memory, hipMemcpy / here: 2.8 MB 188 / 133 us, 6.6 MB 456 / 277,
+// 15 MB 1.04 / 0.62 ms, 21.9 MB 1.50 / 0.95, 30 MB 2.11 / 1.33, 45 MB 4.32 /
+// 1.34, 51.5 MB 5.04 / 1.49; into memory the caller keeps, 2.8 MB 154 / 112
+// us, 21.9 MB 1.22 / 0.63 ms, 51.5 MB 2.95 / 1.30.  (Host to device the
 // runtime already reaches 29-37 GB/s: those copies stay with it.)
 //
 // Memory that the device can write itself (pinned by the caller, managed, or

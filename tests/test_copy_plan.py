@@ -34,6 +34,6 @@ def test_pinned_memory_is_in_proportion(plan, mb):
     chunk, own, helpers, pinned = plan(size)
     assert chunk % 8 == 0 and chunk * 2 <= size  # whole values, something to overlap
     assert own >= 2 and pinned == chunk * (own + 2 * helpers)
-    assert pinned <= 0.45 * size  # 370 us per MB of it, 70 to 100 us per MB of a plain copy, several copies
+    assert pinned <= 0.5 * size  # 370 us per MB of it, 70 to 100 us per MB of a plain copy, several copies
     assert pinned <= (1 << 20) or helpers > 0
     assert pinned <= 18 << 20
