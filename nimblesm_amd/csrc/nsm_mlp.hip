@@ -385,7 +385,8 @@ __global__ __launch_bounds__(256) void k_adam(Adam o, const float* __restrict__ 
 // few loads: at batch 512 the products of the 4-256-256-256-64 network are
 // 0.46 GFLOP, under a microsecond of the matrix cores, and took 69 us.  But
 // the rows of a batch are independent until the weight gradients: a
-// workgroup takes 16 rows through every layer forward, the loss and the
+// workgroup takes a few rows (training: 4, 8 or 16, train_group; prediction:
+// 4, 16 or 32, forward_rows) through every layer forward, the loss and the
 // input gradients back (k_rows), activations in LDS, one wave per 16 columns
 // of a layer's output and the next layer's weights on their way to registers
 // while a layer computes.  It leaves H_l and D_l transposed, so that the
@@ -406,7 +407,7 @@ __global__ __launch_bounds__(256) void k_adam(Adam o, const float* __restrict__ 
 //
 // Training iteration of the 4-256-256-256-64 network, layer by layer and
 // here: batch 64 54 -> 19 us, 512 66 -> 23 us, 1024 100 -> 29 us, 2048 185 ->
-// 37 us, 4096 243 -> 56 us, 16384 693 -> 205 us.  At 512: k_rows 15 us, of
+// 37 us, 4096 243 -> 56 us, 16384 693 -> 205 us.  At 512 (128 workgroups of 4 rows): k_rows 15 us, of
 // which about 4 are weight loads (one CU reads the 0.6 MB of both copies from
 // L2) and 3 the stores of H, D and G, the rest the chain of seven dependent
 // products; k_weights 8 us, one round of loads per 16 K steps and Adam.
@@ -997,8 +998,11 @@ int backward(nsm_mlp* net, int64_t B, double* partial)
 }
 
 // ---- small networks: k_rows and k_weights
-// Training batches up to kRowBatch rows, the largest measured (205 us per
-// iteration against 693); longer ones, and other networks, run layer by layer.
+// Training batches up to kRowBatch rows; longer ones, and other networks, run
+// layer by layer.  The line is where the measurements it was drawn from ended,
+// no crossover: us per iteration layer by layer / in two
+// launches, 4-256-256-256-64 16,384 rows 693 / 205, 32,768 1348 / 445, 131,072
+// 6896 / 2156; 3-16-1 16,385 rows 251 / 123, 131,072 1786 / 780.
 constexpr int64_t kRowBatch = 16384;
 // A prediction of more rows goes layer by layer where no width passes 32: then
 // 2 of k_rows' 16 waves have columns, and with every CU busy that costs more

@@ -1237,10 +1237,14 @@ int model_create(int64_t num_nodes, const double* reference_coordinates, int num
 // Whether an FP64 model of E elements reads its reference inverse Jacobians
 // from a table formed once (80 doubles per element) instead of forming them
 // in every element launch: NSM_FP64_REF_TABLE=0/1 when set, else when the
-// table takes at most kRefTableBytes.  Reading the table saves 13% of the
-// element kernel's instructions, but it is a further 640 bytes per element
-// and launch: it pays while the table stays in the device's caches between
-// launches, and costs time once it streams from HBM.
+// table takes at most kRefTableBytes.  Reading the table saves 280 of the
+// element kernel's 1,717 instructions per lane, but it is a further 640 bytes
+// per element, of device memory and of each launch's traffic.  us per step
+// without / with it: 36^3 42.1 / 40.5, 40^3 54.2 / 50.3, 48^3 81.2 / 75.7, 54^3
+// (96 MB) 110.0 / 110.9, 64^3 170.5 / 171.3, 80^3 312 / 303, 96^3 524 / 497,
+// 128^3 1198 / 1135.  So it pays while it stays in the device's caches between
+// launches and is even just past them; the 3 to 5% of the largest models are
+// left for their memory (1.34 GB at 128^3).
 constexpr int64_t kRefTableBytes = 96ll << 20;
 bool use_reference_table(int64_t E)
 {

@@ -14,7 +14,7 @@
 namespace nsm {
 
 struct TileArgs {
-  int             tile_elems;       // 256 or 128: threads per workgroup, nodes per tile <= 2*tile_elems
+  int             tile_elems;       // 64, 128, 256 or 512: threads per workgroup, nodes per tile <= 2*tile_elems
   int             resident_groups;  // element-kernel workgroups resident on the device at once
   int             num_tiles;
   int             num_bnd;
@@ -69,7 +69,7 @@ struct EnsTileWork {
   EnsFold          fold;
 };
 
-// Small models, a whole step in one launch (one workgroup per tile): while
+// Models of few tiles (setup_tiles' rule), a whole step in one launch (one workgroup per tile): while
 // staging its nodes a tile first finishes the previous step of the shared
 // ones from the partials of the launch before, in every tile that holds the
 // node, the first of them storing the result; the shared nodes' u and v and

@@ -13,11 +13,13 @@
 // reaction partial per workgroup.
 //
 // The loads a tile needs are issued before its element arithmetic (one tile
-// ahead for X, u and element data, two for node ids; at the tile's start for
-// the flags, mass and v of its interior nodes) and the kinematic-condition
-// table sits in LDS: the F and sigma stores issued during the arithmetic
-// count in the same in-order vector-memory counter as loads, so a load
-// issued after them would wait until all of them had completed.
+// ahead for X, u and element data, two for node ids, where workgroups walk
+// several tiles; at the tile's start for the flags, mass and v of its interior
+// nodes) and the kinematic-condition table sits in LDS: the F and sigma stores
+// issued during the arithmetic count in the same in-order vector-memory
+// counter as loads, so a load issued after them would wait until all of them
+// had completed.  Lean tiles (kLeanTiles) store none and load their nodes'
+// state after the arithmetic, which frees the registers it would hold.
 #include "nsm_mixed_math.h"
 #include "nsm_node_step.h"
 #include "nsm_tiled.h"
