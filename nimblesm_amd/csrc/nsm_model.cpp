@@ -2067,12 +2067,21 @@ int nsm_model_set_uq_samples(nsm_model* md, int num_exact, const double* bulk_mo
       (void)hipGetLastError();
       return NSM_OK;
     }
+    // steps run on the tables as soon as uq_traj is set: only when they are filled
+    hipError_t e = hipMemcpyAsync(md->uq_moduli, moduli.data(), moduli.size() * sizeof(float), hipMemcpyHostToDevice,
+                                  md->stream);
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(d_traj, traj.data(), T * sizeof(nsm::UqTrajectory), hipMemcpyHostToDevice, md->stream);
+    const hipError_t done = hipStreamSynchronize(md->stream);
+    if (e == hipSuccess) e = done;
+    if (e != hipSuccess) {
+      free_dev(md->uq_moduli);
+      free_dev(md->uq_partials);
+      free_dev(d_traj);
+      return fail(NSM_ERR_HIP, "tables of the joint launches: %s", hipGetErrorString(e));
+    }
     md->device_bytes += T * (sizeof(nsm::UqTrajectory) + (2 * nb + np) * sizeof(float));
     md->uq_traj = d_traj;
-    NSM_HIP(hipMemcpyAsync(md->uq_moduli, moduli.data(), moduli.size() * sizeof(float), hipMemcpyHostToDevice,
-                           md->stream));
-    NSM_HIP(hipMemcpyAsync(d_traj, traj.data(), T * sizeof(nsm::UqTrajectory), hipMemcpyHostToDevice, md->stream));
-    NSM_HIP(hipStreamSynchronize(md->stream));
   }
   return NSM_OK;
 }
