@@ -500,13 +500,18 @@ int rebuild_bcs(nsm_model* md)
                         hipMemcpyHostToDevice));
   }
   std::vector<int> tiles;
-  md->num_bnd_reaction_groups = 0;
-  const bool       have_rx = md->reaction_mask.size() == code.size();
-  for (size_t i = 0; i < code.size(); i++)  // device node order
-    if (have_rx && md->reaction_mask[(size_t)mesh_node(md, (int64_t)i)]) {
-      code[i] |= nsm::kReactionFlag;
+  size_t           element_tiles = 0;  // entries before the boundary groups'
+  const bool       have_rx       = md->reaction_mask.size() == code.size();
+  // the arrays by pointer: the loop's byte stores may alias the model's members
+  const uint8_t* const mask = md->reaction_mask.data();
+  const int32_t* const old  = md->tiled ? md->tiles.node_old.data() : nullptr;
+  uint8_t* const       byte = code.data();
+  const size_t         N    = have_rx ? code.size() : 0;
+  for (size_t i = 0; i < N; i++)  // device node order
+    if (mask[old ? (size_t)old[i] : i]) {
+      byte[i] |= nsm::kReactionFlag;
       const int t = (int)(i / 256);  // node tile of the node kernel
-      if (!md->tiled && (tiles.empty() || tiles.back() != t)) tiles.push_back(t);
+      if (!old && (tiles.empty() || tiles.back() != t)) tiles.push_back(t);
     }
   if (md->tiled && have_rx) {
     // element tiles whose interior nodes hold reaction nodes, then the
@@ -514,17 +519,18 @@ int rebuild_bcs(nsm_model* md)
     const nsm::TileSet& ts = md->tiles;
     for (int t = 0; t < ts.num_tiles; t++)
       for (int s = ts.node_off[(size_t)t]; s < ts.node_off[(size_t)t + 1]; s++)
-        if ((ts.node_info[(size_t)s] & nsm::kInteriorNode) &&
-            md->reaction_mask[(size_t)mesh_node(md, ts.nodes[(size_t)s])]) {
+        if ((ts.node_info[(size_t)s] & nsm::kInteriorNode) && mask[(size_t)old[ts.nodes[(size_t)s]]]) {
           tiles.push_back(t);
           break;
         }
+    element_tiles = tiles.size();
     for (size_t b = 0; b < ts.bnd_nodes.size(); b++)
-      if (md->reaction_mask[(size_t)mesh_node(md, ts.bnd_nodes[b])]) {
+      if (mask[(size_t)old[ts.bnd_nodes[b]]]) {
         const int g = ts.num_tiles + (int)(b / nsm::kBoundaryNodesPerGroup);
-        if (tiles.empty() || tiles.back() != g) tiles.push_back(g), md->num_bnd_reaction_groups++;
+        if (tiles.empty() || tiles.back() != g) tiles.push_back(g);
       }
   }
+  md->num_bnd_reaction_groups = md->tiled ? (int)(tiles.size() - element_tiles) : 0;
   NSM_HIP(hipMemcpy(md->flags, code.data(), code.size(), hipMemcpyHostToDevice));
   free_dev(md->reaction_tiles);
   md->num_reaction_tiles = 0;
