@@ -15,9 +15,9 @@
 // one: chunks are claimed one at a time, the caller carries whatever the
 // helpers do not, and a helper that starts late finds none left.
 // Into fresh memory, hipMemcpy / here: 2.8 MB 188 / 133 us, 6.6 MB 456 / 277,
-// 15 MB 1.04 / 0.62 ms, 21.9 MB 1.50 / 0.95, 30 MB 2.11 / 1.33, 45 MB 4.32 /
+// 15 MB 1.04 / 0.62 ms, 21.9 MB 1.49 / 0.86, 32 MB 2.20 / 1.24, 45 MB 4.32 /
 // 1.34, 51.5 MB 5.04 / 1.49; into memory the caller keeps, 2.8 MB 154 / 112
-// us, 21.9 MB 1.22 / 0.63 ms, 51.5 MB 2.95 / 1.30.  (Host to device the
+// us, 21.9 MB 1.19 / 0.56 ms, 51.5 MB 2.95 / 1.30.  (Host to device the
 // runtime already reaches 29-37 GB/s: those copies stay with it.)
 //
 // Memory that the device can write itself (pinned by the caller, managed, or

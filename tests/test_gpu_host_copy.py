@@ -58,9 +58,9 @@ def test_pinned_and_device_destinations(hip_device, num_nodes):
     m.close()
 
 
-@pytest.mark.parametrize("sizes", [(699050, 699051, 1747626), (1747627, 100000, 2500000)])
+@pytest.mark.parametrize("sizes", [(699050, 699051, 1398101), (1398102, 100000, 2500000)])
 def test_copies_of_every_cut_in_turn(hip_device, sizes):
-    """Fields on both sides of the sizes at which the cut changes (16 and 40
+    """Fields on both sides of the sizes at which the cut changes (16 and 32
     MB), read by three threads at once, each in its own order: every value
     arrives, whichever pinned slots a copy finds."""
     import threading
